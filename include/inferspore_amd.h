@@ -261,6 +261,26 @@ int isp_repeat_kv_cache_f16(const void* k_cache, const void* v_cache, void* k_ds
                             isp_stream_t stream);
 
 /*
+ * Causal attention of a prefill batch or a decode step, straight from the KV cache to packed rows:
+ *   out[first[b] + i, h, :] = softmax_j(scale * q[b, h, i, :] . k[j]) v[j]     for i < input_length[b]
+ * over the keys j < min(history_length[b] + i + 1, context_length[b], max_k_len) of
+ * cache[layer][b, h / (head_num / kv_head_num), j, :], first[b] = sum of the input lengths before b.
+ *   q [batch, head_num, max_q_len, head_size] (rows of padded queries are never read);
+ *   k_cache, v_cache [layers, batch, kv_head_num, max_seq_len, head_size] (base pointers; rows from
+ *   context_length[b] on are never used); out [token_num, head_num, head_size].
+ * head_size 128 or 64, 16-byte aligned pointers, else ISP_ERR_UNSUPPORTED.
+ * One kernel for the reference's launchRepeatKVCache, batched q x k^T, launchScaleMaskAndSoftmax,
+ * batched p x v and launchTransposeOutRemovePadding (src/kernels/repeat_kv.cu:10-100, linear.cu:67-109,
+ * attn_softmax_kernel.cu:50-125, build_casual_mask.cu:5-42; the history is visible here, see
+ * csrc/context_attention.hip).
+ */
+int isp_context_attention_f16(const void* q, const void* k_cache, const void* v_cache, void* out,
+                              const int32_t* history_length, const int32_t* input_length,
+                              const int32_t* context_length, int layer, int batch, int head_num,
+                              int kv_head_num, int head_size, int max_q_len, int max_k_len,
+                              int max_seq_len, int token_num, float scale, isp_stream_t stream);
+
+/*
  * Measurement aids (no reference counterpart).
  * isp_calibration_copy: a plain copy kernel of known traffic (`bytes` read + `bytes` written;
  *   16-byte aligned, multiple of 16) used to calibrate profiler byte counters and to measure the

@@ -9,17 +9,15 @@ order a model runs them:
     normed, residual                       (packed [tokens, H]; `normed` = RMSNorm(residual) by attn_norm)
     qkv      = normed @ Wqkv                                 library GEMM (out of this library's scope)
     q, cache += k, v = add_fused_qkv_bias_transpose_rope_and_append(qkv)    * this library
-    k_all, v_all = repeat(cache)                             * this library
-    ctx      = softmax(q k^T / sqrt(d) + mask) v             library attention (out of scope)
-    packed   = transpose_out_remove_padding(ctx)             * this library
+    packed   = context_attention(q, cache)                   * this library (float16 heads of 64 or 128 elements; others:
+                                                               repeat_kv_cache, torch's attention, transpose_out_remove_padding)
     attn_out = packed @ Wo                                   library GEMM
     residual, normed2 = fused_add_bias_residual_rmsnorm(residual, attn_out, ffn_norm)      * this library
     act      = SwiGLU(normed2 @ Wgate_up)                    library GEMM + * this library
     ffn_out  = act @ Wdown                                   library GEMM
     residual, normed_next = fused_add_bias_residual_rmsnorm(residual, ffn_out, next attn_norm)   * this library
 
-Dense contractions and attention are deliberately left to torch's library calls (hipBLASLt GEMMs,
-scaled_dot_product_attention); everything marked * goes through the C ABI.  All work is issued on
+Dense contractions are left to torch's library calls (hipBLASLt GEMMs); everything marked * goes through the C ABI.  All work is issued on
 torch's current stream.
 """
 import math
@@ -63,26 +61,37 @@ class BatchState:
         self.padding_offset = torch.zeros((self.batch, max_q_len), dtype=torch.int32, device=dev)
         self.cum_seqlens = torch.zeros(self.batch + 1, dtype=torch.int32, device=dev)
         ops.cal_padding_offset(self.padding_offset, self.cum_seqlens, self.lengths)
-        hidden = head_num * head_size
         z = lambda *s: torch.zeros(s, dtype=dtype, device=dev)
         self.q = z(self.batch, head_num, max_q_len, head_size)
         self.k_cache = z(layers, self.batch, kv_head_num, max_seq_len, head_size)
         self.v_cache = z(layers, self.batch, kv_head_num, max_seq_len, head_size)
-        self.k_all = z(self.batch, head_num, self.max_k_len, head_size)
-        self.v_all = z(self.batch, head_num, self.max_k_len, head_size)
         self.packed_ctx = z(self.tokens, head_num, head_size)
         self.act = z(self.tokens, inter)
-        # additive attention mask [batch, 1, max_q_len, max_k_len]: query s of sequence b sees keys
-        # 0 .. history[b] + s, and only when s is a valid position
-        s = torch.arange(max_q_len, device=dev)[None, :, None]
+
+    def __getattr__(self, name):
+        # Only the padded form of the attention (repeat, mask, transpose) uses these: they are built when it first asks
+        if name == "mask":
+            self.mask = self._build_mask()
+        elif name in ("k_all", "v_all"):
+            shape = (self.batch, self.head_num, self.max_k_len, self.head_size)
+            setattr(self, name, torch.zeros(shape, dtype=self.q.dtype, device=self.q.device))
+        else:
+            raise AttributeError(name)
+        return self.__dict__[name]
+
+    def _build_mask(self):
+        """Additive attention mask [batch, 1, max_q_len, max_k_len]: query s of sequence b sees keys
+        0 .. history[b] + s, and only when s is a valid position."""
+        dev = self.q.device
+        s = torch.arange(self.max_q_len, device=dev)[None, :, None]
         kpos = torch.arange(self.max_k_len, device=dev)[None, None, :]
         hist = self.history[:, None, None]
         visible = (kpos <= hist + s) & (s < self.lengths[:, None, None])
-        self.mask = torch.zeros((self.batch, 1, max_q_len, self.max_k_len), dtype=dtype, device=dev)
-        self.mask.masked_fill_(~visible[:, None], float("-inf"))
+        mask = torch.zeros((self.batch, 1, self.max_q_len, self.max_k_len), dtype=self.q.dtype, device=dev)
+        mask.masked_fill_(~visible[:, None], float("-inf"))
         # fully padded query rows would be all -inf: let them see key 0 (their output is discarded)
-        self.mask[:, :, :, 0].masked_fill_(~(s[:, :, 0] < self.lengths[:, None])[:, None], 0.0)
-        del hidden
+        mask[:, :, :, 0].masked_fill_(~(s[:, :, 0] < self.lengths[:, None])[:, None], 0.0)
+        return mask
 
 
 def context_decoder_layer(normed, residual, w, state, layer_id, next_norm_gamma, rotary_dim=128,
@@ -96,10 +105,14 @@ def context_decoder_layer(normed, residual, w, state, layer_id, next_norm_gamma,
     ops.add_fused_qkv_bias_transpose_rope_and_append(st.q, None, None, st.k_cache, st.v_cache, layer_id, qkv,
                                                      w.qkv_bias, st.padding_offset, st.history, st.lengths,
                                                      rotary_dim, rotary_base)
-    ops.repeat_kv_cache(st.k_cache, st.v_cache, st.context, layer_id, st.k_all, st.v_all)
-    ctx = torch.nn.functional.scaled_dot_product_attention(st.q, st.k_all, st.v_all, attn_mask=st.mask,
-                                                           scale=1.0 / math.sqrt(st.head_size))
-    ops.transpose_out_remove_padding(ctx.contiguous(), st.padding_offset, st.packed_ctx)
+    if ops.context_attention_supports(st.q.dtype, st.head_size):
+        ops.context_attention(st.q, st.k_cache, st.v_cache, layer_id, st.history, st.lengths, st.context, st.max_k_len,
+                              st.packed_ctx)
+    else:
+        ops.repeat_kv_cache(st.k_cache, st.v_cache, st.context, layer_id, st.k_all, st.v_all)
+        ctx = torch.nn.functional.scaled_dot_product_attention(st.q, st.k_all, st.v_all, attn_mask=st.mask,
+                                                               scale=1.0 / math.sqrt(st.head_size))
+        ops.transpose_out_remove_padding(ctx.contiguous(), st.padding_offset, st.packed_ctx)
     attn_out = st.packed_ctx.view(st.tokens, -1) @ w.o
     ops.fused_add_bias_residual_rmsnorm(residual, attn_out, None, w.ffn_norm, eps)   # attn_out := normed
     gate_up = (attn_out @ w.gate_up).view(st.tokens, 2, -1)

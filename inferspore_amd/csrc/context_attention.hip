@@ -1,4 +1,4 @@
-// Fused causal attention of the context-decoder layer for fp16 heads of 128 or 64 elements: one kernel in place of
+// Fused causal attention of a context-decoder layer for fp16 heads of 128 or 64 elements: one kernel in place of
 // KV broadcast, q x k^T, masked softmax, p x v and the transpose back to packed tokens.  It reads the padded
 // queries [batch, head_num, max_q_len, hs], the layer's slice of the KV cache [batch, kv_head_num,
 // max_seq_len, hs] (keys and values of the history and of this call's tokens) and writes the packed
@@ -22,17 +22,9 @@
 // long as both operands agree.  K tiles sit in LDS as stored ([key][d], padded rows), V tiles transposed
 // ([d][key], written two keys at a time, the keys of a row in the operand's order) so that the A operand of the
 // second product is one 16-byte read.
-#include <hip/hip_fp16.h>
-#include <hip/hip_runtime.h>
+#include "isp_common.h"
 
-#include <cmath>
-#include <cstdint>
-#include <string>
-
-#include "src/layers/decoder/context_decoder_layer.h"
-#include "src/utils/macro.h"
-
-namespace isp_layers {
+namespace isp {
 
 namespace {
 
@@ -56,12 +48,6 @@ __device__ __forceinline__ int vt_unit(int d, int unit) { return d * (kKeyTile /
 __device__ __forceinline__ int vt_pair(int d, int pair) {
     const int key = 2 * pair, step = key / 16, quad = (key % 16) / 4;  // quads 0..3 of a step: h = quad % 2, second half = quad / 2
     return vt_unit(d, 2 * step + quad % 2) + 2 * (quad / 2) + (key % 4) / 2;
-}
-
-__device__ __forceinline__ int uniform_int(const int* p, int i) {
-    // the lengths never change while the kernel runs: read them through the scalar cache
-    typedef const int __attribute__((address_space(4)))* constant_ints;
-    return reinterpret_cast<constant_ints>((unsigned long long)p)[i];
 }
 
 // Maximum / sum of a value with the one in the other half of the wavefront (lane ^ 32), without a trip through LDS:
@@ -94,12 +80,12 @@ __global__ __launch_bounds__(256, 2) void context_attention_f16(
     // (the kernel takes as long as its longest workgroup: pinning the query tiles of a (sequence, head) pair to one
     // XCD so that they share its L2 gives up that order and measured 50 instead of 41 us)
     const int head = blockIdx.x, b = blockIdx.y, q0 = (int)(gridDim.z - 1 - blockIdx.z) * kQueryTile;
-    const int len = min(uniform_int(input_length, b), max_q_len);
+    const int len = min(read_only_i32(input_length, b), max_q_len);
     if (q0 >= len) return;  // workgroup-uniform: only padded queries here
-    const int hist = uniform_int(history_length, b);
-    const int ctx = min(min(uniform_int(context_length, b), max_k_len), max_seq_len);
+    const int hist = read_only_i32(history_length, b);
+    const int ctx = min(min(read_only_i32(context_length, b), max_k_len), max_seq_len);
     int first_token = 0;
-    for (int i = 0; i < b; i++) first_token += uniform_int(input_length, i);
+    for (int i = 0; i < b; i++) first_token += read_only_i32(input_length, i);
     const int kv_head = head / (head_num / kv_head_num);
     const size_t kv_offset = ((size_t)b * kv_head_num + kv_head) * (size_t)max_seq_len * kHeadSize;
     const _Float16* keys = k_cache + kv_offset;
@@ -295,35 +281,47 @@ __global__ __launch_bounds__(256, 2) void context_attention_f16(
 
 }  // namespace
 
-bool fused_context_attention_supports(int head_size, int head_num, int kv_head_num) {
-    return (head_size == 128 || head_size == 64) && kv_head_num > 0 && head_num % kv_head_num == 0;
-}
-
-void launch_fused_context_attention(const half* q_buf, const half* k_cache, const half* v_cache, half* out,
-                                    const int* history_length, const int* input_length, const int* context_length,
-                                    int batch, int head_num, int kv_head_num, int head_size, int max_q_len,
-                                    int max_k_len, int max_seq_len, int tokens, float scale) {
-    LLM_CHECK_WITH_INFO(q_buf && k_cache && v_cache && out && history_length && input_length && context_length,
-                        "fused attention: null operand");
-    LLM_CHECK_WITH_INFO(head_size == 128 || head_size == 64, "fused attention: heads of 128 or 64 elements only");
-    LLM_CHECK_WITH_INFO(batch > 0 && batch <= 65535 && head_num > 0 && kv_head_num > 0 && head_num % kv_head_num == 0 &&
-                            max_q_len > 0 && (max_q_len + kQueryTile - 1) / kQueryTile <= 65535 && max_k_len > 0 && max_seq_len > 0 &&
-                            tokens >= 0 && scale > 0.0f,
-                        "fused attention: extents out of range");
-    const uintptr_t bits = reinterpret_cast<uintptr_t>(q_buf) | reinterpret_cast<uintptr_t>(k_cache) |
-                           reinterpret_cast<uintptr_t>(v_cache) | reinterpret_cast<uintptr_t>(out);
-    LLM_CHECK_WITH_INFO((bits & 15u) == 0, "fused attention: operands must be 16-byte aligned");
-    const dim3 grid((unsigned)head_num, (unsigned)batch, (unsigned)((max_q_len + kQueryTile - 1) / kQueryTile));
-#define ISP_LAUNCH_ATTENTION(HS)                                                                                  \
-    hipLaunchKernelGGL(context_attention_f16<HS>, grid, dim3(256), 0, nullptr,                                    \
-                       reinterpret_cast<const _Float16*>(q_buf), reinterpret_cast<const _Float16*>(k_cache),      \
-                       reinterpret_cast<const _Float16*>(v_cache), reinterpret_cast<_Float16*>(out), history_length, \
-                       input_length, context_length, head_num, kv_head_num, max_q_len, max_k_len, max_seq_len,   \
-                       tokens, scale * 1.4426950408889634f)
+static int context_attention(const _Float16* q, const _Float16* k_cache, const _Float16* v_cache, _Float16* out,
+                             const int32_t* history_length, const int32_t* input_length, const int32_t* context_length,
+                             int layer, int batch, int head_num, int kv_head_num, int head_size, int max_q_len,
+                             int max_k_len, int max_seq_len, int token_num, float scale, hipStream_t stream) {
+    if (layer < 0 || batch < 0 || head_num <= 0 || kv_head_num <= 0 || head_num % kv_head_num != 0 || max_q_len < 0 ||
+        max_k_len < 0 || max_seq_len < 0 || token_num < 0 || !(scale > 0.0f))
+        return ISP_ERR_BAD_SHAPE;
+    if (head_size != 128 && head_size != 64) return ISP_ERR_UNSUPPORTED;
+    if (batch == 0 || max_q_len == 0 || token_num == 0) return ISP_OK;
+    if (max_k_len == 0 || max_seq_len == 0) return ISP_ERR_BAD_SHAPE;
+    const int tiles = (max_q_len + kQueryTile - 1) / kQueryTile;
+    if (batch > 65535 || tiles > 65535) return ISP_ERR_UNSUPPORTED;
+    ISP_REQUIRE_PTR(q);
+    ISP_REQUIRE_PTR(k_cache);
+    ISP_REQUIRE_PTR(v_cache);
+    ISP_REQUIRE_PTR(out);
+    ISP_REQUIRE_PTR(history_length);
+    ISP_REQUIRE_PTR(input_length);
+    ISP_REQUIRE_PTR(context_length);
+    if (!aligned16(q) || !aligned16(k_cache) || !aligned16(v_cache) || !aligned16(out)) return ISP_ERR_UNSUPPORTED;
+    const size_t slice = (size_t)layer * batch * kv_head_num * max_seq_len * head_size;
+    const dim3 grid((unsigned)head_num, (unsigned)batch, (unsigned)tiles);
+#define ISP_LAUNCH_ATTENTION(HS)                                                                                    \
+    hipLaunchKernelGGL(context_attention_f16<HS>, grid, dim3(256), 0, stream, q, k_cache + slice, v_cache + slice, out, \
+                       history_length, input_length, context_length, head_num, kv_head_num, max_q_len, max_k_len,   \
+                       max_seq_len, token_num, scale * 1.4426950408889634f)
     if (head_size == 128) ISP_LAUNCH_ATTENTION(128);
     else ISP_LAUNCH_ATTENTION(64);
 #undef ISP_LAUNCH_ATTENTION
-    CHECK(hipGetLastError());
+    return note_launch(hipGetLastError());
 }
 
-}  // namespace isp_layers
+}  // namespace isp
+
+extern "C" int isp_context_attention_f16(const void* q, const void* k_cache, const void* v_cache, void* out,
+                                         const int32_t* history_length, const int32_t* input_length,
+                                         const int32_t* context_length, int layer, int batch, int head_num,
+                                         int kv_head_num, int head_size, int max_q_len, int max_k_len, int max_seq_len,
+                                         int token_num, float scale, isp_stream_t stream) {
+    return isp::context_attention(static_cast<const _Float16*>(q), static_cast<const _Float16*>(k_cache),
+                                  static_cast<const _Float16*>(v_cache), static_cast<_Float16*>(out), history_length,
+                                  input_length, context_length, layer, batch, head_num, kv_head_num, head_size, max_q_len,
+                                  max_k_len, max_seq_len, token_num, scale, static_cast<hipStream_t>(stream));
+}

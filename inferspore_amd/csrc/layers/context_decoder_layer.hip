@@ -19,6 +19,7 @@
 #include <vector>
 #include <algorithm>
 
+#include "inferspore_amd.h"
 #include "src/kernels/act_kernel.h"
 #include "src/kernels/fused_addresidual_norm.h"
 #include "src/kernels/fused_transpose_and_remv_pad.h"
@@ -446,6 +447,21 @@ void launch_masked_scaled_softmax(T* scores, const int* history_length, const in
 
 template void launch_masked_scaled_softmax<float>(float*, const int*, const int*, const int*, int, int, int, int, float);
 template void launch_masked_scaled_softmax<half>(half*, const int*, const int*, const int*, int, int, int, int, float);
+
+bool fused_context_attention_supports(int head_size, int head_num, int kv_head_num) {
+    return (head_size == 128 || head_size == 64) && kv_head_num > 0 && head_num % kv_head_num == 0;
+}
+
+void launch_fused_context_attention(const half* q_buf, const half* k_cache, const half* v_cache, half* out,
+                                    const int* history_length, const int* input_length, const int* context_length,
+                                    int batch, int head_num, int kv_head_num, int head_size, int max_q_len,
+                                    int max_k_len, int max_seq_len, int tokens, float scale) {
+    LLM_CHECK_WITH_INFO(batch > 0 && max_q_len > 0 && max_k_len > 0 && max_seq_len > 0, "fused attention: extents out of range");
+    const int status = isp_context_attention_f16(q_buf, k_cache, v_cache, out, history_length, input_length, context_length,
+                                                 0, batch, head_num, kv_head_num, head_size, max_q_len, max_k_len,
+                                                 max_seq_len, tokens, scale, nullptr);
+    LLM_CHECK_WITH_INFO(status == ISP_OK, std::string("fused attention: ") + isp_strerror(status));
+}
 
 }  // namespace isp_layers
 

@@ -266,6 +266,38 @@ def transpose_out_remove_padding(qkv_buf_w_pad, padding_offset, qkv_buf_wo_pad):
     return qkv_buf_wo_pad
 
 
+def context_attention_supports(dtype, head_size):
+    """Whether context_attention takes heads of this type and size."""
+    return dtype == torch.float16 and head_size in (64, 128)
+
+
+def context_attention(q_buf, k_cache, v_cache, layer_id, history_length, input_length, context_length, max_k_len, out,
+                      scale=None):
+    """Causal attention over the KV cache (history included), to packed rows: q_buf [batch, heads, max_q_len, hs], caches
+    [layers, batch, kv_heads, max_seq_len, hs], out [tokens, heads, hs].  scale defaults to hs ** -0.5."""
+    _same_dtype(q_buf, k_cache, v_cache, out)
+    _int32(history_length, input_length, context_length)
+    _expect(q_buf.dim() == 4 and k_cache.dim() == 5 and out.dim() == 3,
+            "attention takes q [batch, heads, max_q_len, head_size], caches [layers, batch, kv_heads, max_seq_len, head_size] "
+            "and out [tokens, heads, head_size]")
+    batch, head_num, max_q_len, head_size = q_buf.shape
+    kv_head_num, max_seq_len = k_cache.shape[2], k_cache.shape[3]
+    _expect(tuple(k_cache.shape) == tuple(v_cache.shape) and k_cache.shape[1] == batch and k_cache.shape[4] == head_size,
+            "caches must be [layers, batch, kv_head_num, max_seq_len, head_size]")
+    _expect(context_attention_supports(q_buf.dtype, head_size), "attention takes float16 heads of 64 or 128 elements")
+    _expect(kv_head_num > 0 and head_num % kv_head_num == 0, "head_num must be a multiple of kv_head_num")
+    _expect(tuple(out.shape[1:]) == (head_num, head_size), "out must be [tokens, heads, head_size]")
+    _expect(0 <= int(layer_id) < k_cache.shape[0], "layer_id outside the cache")
+    _expect(min(history_length.numel(), input_length.numel(), context_length.numel()) >= batch,
+            "length tensors are shorter than the batch")
+    _dev(q_buf, k_cache, v_cache, history_length, input_length, context_length, out)
+    capi.check(capi.lib().isp_context_attention_f16(
+        _p(q_buf), _p(k_cache), _p(v_cache), _p(out), _p(history_length), _p(input_length), _p(context_length),
+        int(layer_id), batch, head_num, kv_head_num, head_size, max_q_len, int(max_k_len), max_seq_len, out.shape[0],
+        float(head_size ** -0.5 if scale is None else scale), _stream()), "isp_context_attention")
+    return out
+
+
 def concat_kv_cache(k_src, v_src, layer_id, cur_query_length, history_length, k_dst, v_dst):
     """launchConcatKVCache; shapes as the reference derives them (concat_past_kv.cu:84-90)."""
     _same_dtype(k_src, v_src, k_dst, v_dst)

@@ -1,0 +1,61 @@
+"""ops.context_attention against a float64 attention on the CPU, at the extents where its kernels can go wrong: queries
+and keys that end inside, at and just past a tile, a single query over long and short histories, grouped heads, an
+empty sequence, padded extents larger than the longest query.  Rows that must not be read hold NaN.
+
+Bound: the probabilities are rounded to fp16 before the second product (relative 2^-11 each, averaging out over the
+keys) and the result once more; 2e-3 of the largest output is several times that."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+#        lens                 history              heads kv  max_q max_seq
+CASES = [([5], [0], 2, 2, 5, 8),
+         ([16, 5, 11], [0, 9, 30], 4, 2, 16, 48),
+         ([200, 133], [0, 70], 2, 2, 210, 300),
+         ([129], [0], 8, 1, 130, 130),
+         ([64, 64], [0, 64], 2, 1, 64, 128),
+         ([40, 0, 17], [0, 5, 9], 2, 2, 40, 64),
+         ([1, 1, 1], [1000, 63, 64], 4, 2, 1, 1100),
+         ([1, 1, 1, 1], [0, 31, 32, 33], 8, 2, 1, 64),
+         ([1, 1], [255, 700], 32, 1, 1, 1024),
+         ([1] * 9, [3, 700, 128, 127, 129, 511, 512, 513, 0], 16, 16, 1, 768),
+         ([2, 1, 3], [100, 257, 64], 6, 2, 3, 300)]
+
+
+def reference(q, k, v, lens, hist, out):
+    heads, hs, group = q.shape[1], q.shape[3], q.shape[1] // k.shape[1]
+    t = 0
+    for b, (n, h) in enumerate(zip(lens, hist)):
+        kk = k[b, :, :h + n].double().repeat_interleave(group, 0)
+        vv = v[b, :, :h + n].double().repeat_interleave(group, 0)
+        s = (q[b, :, :n].double()[:, :, None, :] * kk[:, None]).sum(-1) * hs ** -0.5
+        s.masked_fill_(torch.arange(h + n)[None, None] > h + torch.arange(n)[None, :, None], float("-inf"))
+        out[t:t + n] = (torch.softmax(s, -1)[..., None] * vv[:, None]).sum(2).transpose(0, 1)
+        t += n
+    return out
+
+
+@pytest.mark.parametrize("hs", [128, 64])
+@pytest.mark.parametrize("case", range(len(CASES)))
+def test_attention_matches_float64(isp, hs, case):
+    lens, hist, heads, kv, max_q, max_seq = CASES[case]
+    print("[case] attention %s hs %d" % (CASES[case], hs), flush=True)
+    g = torch.Generator().manual_seed(case)
+    batch, tokens = len(lens), sum(lens)
+    nan = float("nan")
+    q = torch.full((batch, heads, max_q, hs), nan, dtype=torch.float16)
+    k, v = (torch.full((2, batch, kv, max_seq, hs), nan, dtype=torch.float16) for _ in range(2))
+    for b in range(batch):
+        q[b, :, :lens[b]] = 2 * torch.randn(heads, lens[b], hs, generator=g)
+        n = lens[b] + hist[b]
+        k[1, b, :, :n] = 2 * torch.randn(kv, n, hs, generator=g)
+        v[1, b, :, :n] = torch.randn(kv, n, hs, generator=g)
+    expect = reference(q, k[1], v[1], lens, hist, torch.zeros(tokens, heads, hs, dtype=torch.float64))
+    ints = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")   # noqa: E731
+    out = torch.full((tokens, heads, hs), nan, dtype=torch.float16, device="cuda")
+    context = [a + b for a, b in zip(lens, hist)]
+    isp.context_attention(q.cuda(), k.cuda(), v.cuda(), 1, ints(hist), ints(lens), ints(context), max(context), out)
+    got = out.cpu().double()
+    assert torch.isfinite(got).all()
+    assert (got - expect).abs().max() <= 2e-3 * expect.abs().max()

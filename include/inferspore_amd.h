@@ -281,6 +281,16 @@ int isp_context_attention_f16(const void* q, const void* k_cache, const void* v_
                               int max_seq_len, int token_num, float scale, isp_stream_t stream);
 
 /*
+ * Product of a few rows with a weight matrix, fp32 accumulation: out[m, n] = a[m, k] x w[k, n], all row-major and
+ * contiguous (the reference's launchLinearGemm with trans_b = false, src/kernels/linear.cu:7-66).  For the rows of a
+ * decode step or a short prompt: m <= 64, n and k multiples of 8, 16-byte aligned pointers, else ISP_ERR_UNSUPPORTED.
+ * workspace: isp_linear_f16_workspace(m, n, k) bytes of device memory that no other work in flight uses; may be NULL
+ * where that is 0.
+ */
+size_t isp_linear_f16_workspace(int m, int n, int k);
+int isp_linear_f16(const void* a, const void* w, void* out, void* workspace, int m, int n, int k, isp_stream_t stream);
+
+/*
  * Measurement aids (no reference counterpart).
  * isp_calibration_copy: a plain copy kernel of known traffic (`bytes` read + `bytes` written;
  *   16-byte aligned, multiple of 16) used to calibrate profiler byte counters and to measure the

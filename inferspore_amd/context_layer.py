@@ -17,8 +17,8 @@ order a model runs them:
     ffn_out  = act @ Wdown                                   library GEMM
     residual, normed_next = fused_add_bias_residual_rmsnorm(residual, ffn_out, next attn_norm)   * this library
 
-Dense contractions are left to torch's library calls (hipBLASLt GEMMs); everything marked * goes through the C ABI.  All work is issued on
-torch's current stream.
+Dense contractions of more than 64 rows are left to torch's library calls (hipBLASLt GEMMs), those of fewer float16 rows go to
+ops.linear; everything marked * goes through the C ABI.  All work is issued on torch's current stream.
 """
 import math
 
@@ -94,12 +94,16 @@ class BatchState:
         return mask
 
 
+def _linear(x, w):
+    return ops.linear(x, w) if ops.linear_supports(x, w) else x @ w
+
+
 def context_decoder_layer(normed, residual, w, state, layer_id, next_norm_gamma, rotary_dim=128,
                           rotary_base=10000.0, eps=1e-5):
     """Runs one prefill layer.  `normed` and `residual` are packed [tokens, H]; `residual` is updated in
     place; returns the next layer's normalised input (a new tensor)."""
     st = state
-    qkv = normed @ w.qkv                                                       # [tokens, 3H]
+    qkv = _linear(normed, w.qkv)                                                 # [tokens, 3H]
     qkv = qkv.view(st.tokens, st.head_num + 2 * st.kv_head_num, st.head_size)
     # bias + RoPE + re-pad of q, with k and v written straight into the cache (one launch, no padded k / v)
     ops.add_fused_qkv_bias_transpose_rope_and_append(st.q, None, None, st.k_cache, st.v_cache, layer_id, qkv,
@@ -113,10 +117,10 @@ def context_decoder_layer(normed, residual, w, state, layer_id, next_norm_gamma,
         ctx = torch.nn.functional.scaled_dot_product_attention(st.q, st.k_all, st.v_all, attn_mask=st.mask,
                                                                scale=1.0 / math.sqrt(st.head_size))
         ops.transpose_out_remove_padding(ctx.contiguous(), st.padding_offset, st.packed_ctx)
-    attn_out = st.packed_ctx.view(st.tokens, -1) @ w.o
+    attn_out = _linear(st.packed_ctx.view(st.tokens, -1), w.o)
     ops.fused_add_bias_residual_rmsnorm(residual, attn_out, None, w.ffn_norm, eps)   # attn_out := normed
-    gate_up = (attn_out @ w.gate_up).view(st.tokens, 2, -1)
+    gate_up = _linear(attn_out, w.gate_up).view(st.tokens, 2, -1)
     ops.act(gate_up, st.act)
-    ffn_out = st.act @ w.down
+    ffn_out = _linear(st.act, w.down)
     ops.fused_add_bias_residual_rmsnorm(residual, ffn_out, None, next_norm_gamma, eps)
     return ffn_out

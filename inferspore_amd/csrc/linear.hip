@@ -1,0 +1,78 @@
+// isp_linear_f16: the product of a few activation rows with a weight matrix (see linear_rows.h for the kernel).
+// The reference calls cuBLAS for it (src/kernels/linear.cu:7-66); the library here, hipBLASLt, reads the weights of a
+// 16-row product at 1.4-3.8 TB/s and those of a 64-row product at 1.2-1.8 (4.9 for the widest), this kernel at 4.3-5.5
+// and 3.0-4.7.
+#include "linear_rows.h"
+
+namespace isp {
+
+void launch_skinny(const SkinnyPlan& plan, const __half* a, const __half* w, __half* out, float* partial, int m, int n, int k,
+                   hipStream_t stream) {
+    const dim3 grid((unsigned)plan.strips, (unsigned)plan.splits);
+#define ISP_SKINNY(MT)                                                                                                    \
+    if (out)                                                                                                              \
+        hipLaunchKernelGGL((linear_skinny_f16<MT, false>), grid, dim3(kBlock), 0, stream, a, w, out, partial, m, n, k,    \
+                           plan.steps_per_split);                                                                         \
+    else                                                                                                                  \
+        hipLaunchKernelGGL((linear_skinny_f16<MT, true>), grid, dim3(kBlock), 0, stream, a, w, out, partial, m, n, k,     \
+                           plan.steps_per_split)
+    if (m <= 16) ISP_SKINNY(1);
+    else if (m <= 32) ISP_SKINNY(2);
+    else if (m <= 48) ISP_SKINNY(3);
+    else ISP_SKINNY(4);
+#undef ISP_SKINNY
+}
+
+// out = fp16(sum over the splits, in their order); four columns per lane.
+__global__ __launch_bounds__(kBlock) void linear_add_splits(const float* __restrict__ partial, __half* __restrict__ out,
+                                                            unsigned quads, int splits) {
+    const unsigned i = blockIdx.x * kBlock + threadIdx.x;
+    if (i >= quads) return;
+    const float4v* p = reinterpret_cast<const float4v*>(partial) + i;
+    float4v sum = p[0];
+#pragma unroll 8
+    for (int s = 1; s < splits; s++) sum += p[(size_t)s * quads];
+    const __half2 lo = __floats2half2_rn(sum[0], sum[1]), hi = __floats2half2_rn(sum[2], sum[3]);
+    reinterpret_cast<uint2*>(out)[i] = make_uint2(*reinterpret_cast<const uint32_t*>(&lo), *reinterpret_cast<const uint32_t*>(&hi));
+}
+
+static int linear(const __half* a, const __half* w, __half* out, float* workspace, int m, int n, int k, hipStream_t stream) {
+    if (m < 0 || n < 0 || k < 0) return ISP_ERR_BAD_SHAPE;
+    if (m == 0 || n == 0) return ISP_OK;
+    if (k == 0 || m > kSkinnyMaxRows || n % 8 != 0 || k % 8 != 0) return ISP_ERR_UNSUPPORTED;
+    ISP_REQUIRE_PTR(a);
+    ISP_REQUIRE_PTR(w);
+    ISP_REQUIRE_PTR(out);
+    if (!aligned16(a) || !aligned16(w) || !aligned16(out)) return ISP_ERR_UNSUPPORTED;
+    const SkinnyPlan plan = skinny_plan(m, n, k);
+    if (plan.splits == 1) {
+        launch_skinny(plan, a, w, out, nullptr, m, n, k, stream);
+        return note_launch(hipGetLastError());
+    }
+    ISP_REQUIRE_PTR(workspace);
+    if (!aligned16(workspace)) return ISP_ERR_UNSUPPORTED;
+    launch_skinny(plan, a, w, nullptr, workspace, m, n, k, stream);
+    const int status = note_launch(hipGetLastError());
+    if (status != ISP_OK) return status;
+    const unsigned quads = (unsigned)((size_t)m * (size_t)n / 4);
+    hipLaunchKernelGGL(linear_add_splits, dim3((quads + kBlock - 1) / kBlock), dim3(kBlock), 0, stream, workspace, out, quads,
+                       plan.splits);
+    return note_launch(hipGetLastError());
+}
+
+}  // namespace isp
+
+extern "C" {
+
+size_t isp_linear_f16_workspace(int m, int n, int k) {
+    if (m <= 0 || n <= 0 || k <= 0) return 0;
+    const isp::SkinnyPlan plan = isp::skinny_plan(m, n, k);
+    return plan.splits == 1 ? 0 : plan.partial_floats(m, n) * sizeof(float);
+}
+
+int isp_linear_f16(const void* a, const void* w, void* out, void* workspace, int m, int n, int k, isp_stream_t stream) {
+    return isp::linear(static_cast<const __half*>(a), static_cast<const __half*>(w), static_cast<__half*>(out),
+                       static_cast<float*>(workspace), m, n, k, static_cast<hipStream_t>(stream));
+}
+
+}  // extern "C"

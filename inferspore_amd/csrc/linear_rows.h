@@ -1,0 +1,178 @@
+// Skinny product of a layer: C[m, n] = A[m, k] x W[k, n], fp16, row-major, fp32 accumulation, for the few rows of a
+// decode step or a short prompt.  The weights are read once and bound the time; everything below serves that one stream.
+//
+// A wavefront owns 128 columns and takes 32 rows of W per step: lane (j = lane % 16, g = lane / 16) loads the eight
+// columns 8 j ... 8 j + 7 of the eight rows 8 g ... 8 g + 7, so that every load instruction covers four whole 256-byte row
+// segments and nothing goes through LDS.  Matrix cores want, per lane, eight consecutive k of ONE column
+// (v_mfma_f32_16x16x32_f16): an 8 x 8 transpose inside the lane's own registers, one byte-permute per result dword.  Product c
+// (0 ... 7) then takes column 8 j + c of every lane, and a lane ends with eight neighbouring columns of its output rows.
+// The wavefronts of a workgroup take every WAVES-th step of the workgroup's k range and add up through LDS in a fixed
+// order; workgroups that share a strip of columns write fp32 partial sums [splits][m][n] that the consumer adds in order.
+#pragma once
+
+#include "isp_common.h"
+
+namespace isp {
+
+typedef _Float16 half8 __attribute__((ext_vector_type(8)));
+typedef float float4v __attribute__((ext_vector_type(4)));
+
+constexpr int kStripCols = 128;  // columns of a workgroup
+constexpr int kStepRows = 32;    // rows of W per step of a wavefront
+
+struct SkinnyStep {
+    vec16 w[8];
+};
+
+// Column c of the lane's 8 x 8 block as one operand: dword i holds rows 2 i and 2 i + 1.
+__device__ __forceinline__ half8 block_column(const SkinnyStep& t, int c) {
+    union { uint32_t u[4]; half8 h; } r;
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+        r.u[i] = __builtin_amdgcn_perm(t.w[2 * i + 1].w[c / 2], t.w[2 * i].w[c / 2], c % 2 ? 0x07060302u : 0x05040100u);
+    return r.h;
+}
+
+// MT: tiles of 16 rows of A.  SPLIT: fp32 partial sums to `partial`, else fp16 to `out`.
+template <int MT, bool SPLIT>
+__global__ __launch_bounds__(kBlock) void linear_skinny_f16(const __half* __restrict__ a, const __half* __restrict__ w,
+                                                                 __half* __restrict__ out, float* __restrict__ partial, int m,
+                                                                 int n, int k, int steps_per_split) {
+    constexpr int WAVES = kBlock / kWave;
+    const int tid = threadIdx.x, lane = tid % kWave, wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const int j = lane % 16, g = lane / 16;
+    const int strip0 = (int)blockIdx.x * kStripCols;
+    const int steps = (k + kStepRows - 1) / kStepRows;
+    const int first = (int)blockIdx.y * steps_per_split, last = min(steps, first + steps_per_split);
+    // lanes past the last column (row of A past m) read the last ones that exist; their results are not stored
+    const __half* w_lane = w + min(strip0 + 8 * j, n - 8);
+    const __half* a_lane[MT];
+#pragma unroll
+    for (int t = 0; t < MT; t++) a_lane[t] = a + (size_t)min(16 * t + j, m - 1) * (size_t)k;
+
+    float4v acc[MT][8];
+#pragma unroll
+    for (int t = 0; t < MT; t++)
+#pragma unroll
+        for (int c = 0; c < 8; c++) acc[t][c] = float4v{0.0f, 0.0f, 0.0f, 0.0f};
+
+    SkinnyStep buf[2];
+    half8 af[2][MT];
+    auto load = [&](int which, int s) {
+        // k is a multiple of 8, so a lane's eight rows exist together or not at all (last step only)
+        const int row = min(s * kStepRows + 8 * g, k - 8);
+        const __half* p = w_lane + (size_t)row * (size_t)n;
+#pragma unroll
+        for (int i = 0; i < 8; i++) buf[which].w[i] = load16_stream(p + (size_t)i * (size_t)n);
+#pragma unroll
+        for (int t = 0; t < MT; t++) af[which][t] = *reinterpret_cast<const half8*>(a_lane[t] + row);
+    };
+    auto compute = [&](int which, int s) {
+        if ((s + 1) * kStepRows > k) {  // wavefront-uniform: rows past k count as zero on both sides (0 x inf is NaN)
+            const uint32_t keep = s * kStepRows + 8 * g < k ? 0xffffffffu : 0u;
+#pragma unroll
+            for (int i = 0; i < 8; i++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) buf[which].w[i].w[e] &= keep;
+#pragma unroll
+            for (int t = 0; t < MT; t++)
+                if (!keep) af[which][t] = half8{0, 0, 0, 0, 0, 0, 0, 0};
+        }
+#pragma unroll
+        for (int c = 0; c < 8; c++) {
+            const half8 b = block_column(buf[which], c);
+#pragma unroll
+            for (int t = 0; t < MT; t++) acc[t][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[which][t], b, acc[t][c], 0, 0, 0);
+        }
+    };
+    // The next step's loads are in flight while a step is computed.  No load sits behind a branch that joins again (how many
+    // are outstanding would no longer be known, and every one would be waited for): each half of the loop has its own way
+    // out.  A third or fourth step in flight measured the same at 16 rows and spills registers from 48 rows on.
+    int s = first + wave;
+    if (s < last) {
+        load(0, s);
+        for (;;) {
+            if (s + WAVES >= last) {
+                compute(0, s);
+                break;
+            }
+            load(1, s + WAVES);
+            compute(0, s);
+            s += WAVES;
+            if (s + WAVES >= last) {
+                compute(1, s);
+                break;
+            }
+            load(0, s + WAVES);
+            compute(1, s);
+            s += WAVES;
+        }
+    }
+
+    // 16 rows at a time through LDS: lane (j, g) holds rows 4 g + r and columns 8 j + c
+    __shared__ __align__(16) float tile[WAVES][16][kStripCols];
+    constexpr int elems = 16 * kStripCols / kBlock;  // floats a thread adds up: 8
+    const int row = tid * elems / kStripCols, col = tid * elems % kStripCols;
+#pragma unroll
+    for (int t = 0; t < MT; t++) {
+        if (t > 0) __syncthreads();
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+#pragma unroll
+            for (int h = 0; h < 2; h++)
+                *reinterpret_cast<float4v*>(&tile[wave][4 * g + r][8 * j + 4 * h]) =
+                    float4v{acc[t][4 * h][r], acc[t][4 * h + 1][r], acc[t][4 * h + 2][r], acc[t][4 * h + 3][r]};
+        __syncthreads();
+        const int out_row = 16 * t + row, out_col = strip0 + col;
+        if (out_row < m && out_col < n) {  // n is a multiple of 8: a thread's columns exist together
+#pragma unroll
+            for (int e = 0; e < elems; e += 4) {
+                float4v sum = *reinterpret_cast<const float4v*>(&tile[0][row][col + e]);
+#pragma unroll
+                for (int v = 1; v < WAVES; v++) sum += *reinterpret_cast<const float4v*>(&tile[v][row][col + e]);
+                const size_t at = (size_t)out_row * (size_t)n + (size_t)(out_col + e);
+                if (SPLIT) {
+                    *reinterpret_cast<float4v*>(partial + (size_t)blockIdx.y * (size_t)m * (size_t)n + at) = sum;
+                } else {
+                    __half2 lo = __floats2half2_rn(sum[0], sum[1]), hi = __floats2half2_rn(sum[2], sum[3]);
+                    *reinterpret_cast<uint2*>(out + at) = make_uint2(*reinterpret_cast<uint32_t*>(&lo), *reinterpret_cast<uint32_t*>(&hi));
+                }
+            }
+        }
+    }
+}
+
+// How many workgroups share a strip of columns.  Two costs are weighed: the rounds of one workgroup per compute unit that
+// strips x splits make, over those that whole rounds would make (idle units at the end), and the partial sums, whose bytes
+// are 4 m splits / k of the weights' and count twice (they are written and read back by a dependent kernel).  Measured with 16
+// rows: 96 strips of 4096 rows (100.7 MB) 1, 2, 3, 4, 5, 8 splits 30.0, 19.4, 24.7, 20.5, 18.5, 19.0 us (taken: 5); 32
+// strips (33.6 MB) 4, 8, 16 splits 9.9, 7.8, 7.7 (8); 172 strips 1, 2, 4 splits 34.7, 37.9, 32.5 (4).  With 64 rows: 32
+// strips 4, 8, 16 splits 14.7, 11.3, 15.9 (8); 224 strips 1, 2 splits 49.7, 57.2 (1).  Every wavefront keeps a step.
+struct SkinnyPlan {
+    int strips, splits, steps_per_split;
+    size_t partial_floats(int m, int n) const { return (size_t)splits * (size_t)m * (size_t)n; }
+};
+constexpr int kSkinnyMaxRows = 64, kSkinnyMaxSplits = 16;
+inline SkinnyPlan skinny_plan(int m, int n, int k) {
+    SkinnyPlan p;
+    const int steps = (k + kStepRows - 1) / kStepRows, waves = kBlock / kWave, units = resident_waves() / 32;
+    p.strips = (n + kStripCols - 1) / kStripCols;
+    p.steps_per_split = steps;
+    double best = 0.0;
+    for (int s = 1; s <= kSkinnyMaxSplits && (s == 1 || s * waves <= steps); s++) {
+        const long long groups = (long long)p.strips * s, rounds = (groups + units - 1) / units;
+        const double cost = (double)(rounds * units) / (double)groups + 8.0 * (double)m * (double)s / (double)k;
+        if (s == 1 || cost < best) {
+            best = cost;
+            p.steps_per_split = (steps + s - 1) / s;
+        }
+    }
+    p.splits = (steps + p.steps_per_split - 1) / p.steps_per_split;
+    return p;
+}
+
+// Partial sums of the product to `partial`, or with `out` (one split only) the fp16 product itself.  Operands checked by the caller.
+void launch_skinny(const SkinnyPlan& plan, const __half* a, const __half* w, __half* out, float* partial, int m, int n, int k,
+                   hipStream_t stream);
+
+}  // namespace isp

@@ -266,6 +266,32 @@ def transpose_out_remove_padding(qkv_buf_w_pad, padding_offset, qkv_buf_wo_pad):
     return qkv_buf_wo_pad
 
 
+def linear_supports(x, w):
+    """Whether linear() takes this product: a few contiguous float16 rows outside autograd.  Above 32768 columns more
+    than one round of workgroups is needed, and from 17 rows on the library is faster there (5120 x 40928: 37 rows 88
+    against 112 us, 64 rows 85 against 124; 8 rows 80 against 85)."""
+    return (x.dtype == torch.float16 and w.dtype == torch.float16 and x.dim() == 2 and w.dim() == 2 and x.is_cuda and
+            0 < x.shape[0] <= 64 and (x.shape[0] <= 16 or w.shape[1] <= 32768) and x.shape[1] == w.shape[0] and w.device == x.device and
+            w.shape[0] % 8 == 0 and w.shape[1] % 8 == 0 and w.numel() > 0 and
+            x.is_contiguous() and w.is_contiguous() and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and
+            type(x) is torch.Tensor and type(w) in (torch.Tensor, torch.nn.Parameter) and
+            not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad)) and
+            not torch.is_autocast_enabled())
+
+
+def linear(x, w):
+    """x [rows, k] @ w [k, n] for up to 64 float16 rows, float32 accumulation."""
+    _expect(linear_supports(x, w), "linear takes up to 64 (above 32768 columns: 16) contiguous float16 rows and a contiguous weight [k, n], "
+            "extents in multiples of 8")
+    m, k = x.shape
+    n = w.shape[1]
+    out = torch.empty((m, n), dtype=x.dtype, device=x.device)
+    need = capi.lib().isp_linear_f16_workspace(m, n, k)
+    workspace = torch.empty(need, dtype=torch.uint8, device=x.device) if need else None
+    capi.check(capi.lib().isp_linear_f16(_p(x), _p(w), _p(out), _p(workspace), m, n, k, _stream()), "isp_linear")
+    return out
+
+
 def context_attention_supports(dtype, head_size):
     """Whether context_attention takes heads of this type and size."""
     return dtype == torch.float16 and head_size in (64, 128)

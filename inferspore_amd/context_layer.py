@@ -68,15 +68,20 @@ class BatchState:
         self.packed_ctx = z(self.tokens, head_num, head_size)
         self.act = z(self.tokens, inter)
 
+        if not ops.context_attention_supports(dtype, head_size):
+            self._padded_buffers()
+
+    def _padded_buffers(self):
+        """What the padded form of the attention (repeat, mask, transpose) works on."""
+        shape = (self.batch, self.head_num, self.max_k_len, self.head_size)
+        self.k_all, self.v_all = (torch.zeros(shape, dtype=self.q.dtype, device=self.q.device) for _ in range(2))
+        self.mask = self._build_mask()
+
     def __getattr__(self, name):
-        # Only the padded form of the attention (repeat, mask, transpose) uses these: they are built when it first asks
-        if name == "mask":
-            self.mask = self._build_mask()
-        elif name in ("k_all", "v_all"):
-            shape = (self.batch, self.head_num, self.max_k_len, self.head_size)
-            setattr(self, name, torch.zeros(shape, dtype=self.q.dtype, device=self.q.device))
-        else:
+        # the fused attention needs none of them: there they are built when a program first asks
+        if name not in ("mask", "k_all", "v_all") or "act" not in self.__dict__:
             raise AttributeError(name)
+        self._padded_buffers()
         return self.__dict__[name]
 
     def _build_mask(self):

@@ -279,12 +279,277 @@ __global__ __launch_bounds__(256, 2) void context_attention_f16(
     }
 }
 
+// ---- a few queries per key / value head (a decode step): the keys and values bound the time --------------------------
+//
+// A workgroup serves ONE key / value head of a sequence: the queries of all heads of its group (and of all, at most a few,
+// tokens) share v_mfma_f32_16x16x32_f16's 16 columns, so that a key is read once however many heads use it -- the kernel
+// above would read it once per head, through a tile of 128 queries of which one is real.  A wavefront takes every
+// fourth step of 32 keys, straight from memory into registers, the next step's loads in flight while it computes one:
+//   S^T[key, query] = K x Q^T   lane (j = lane % 16, g = lane / 16) loads 16 bytes of key j (d = 32 i + 8 g ...): the operand as is;
+//                               its results belong to query j and the keys 4 g ... 4 g + 3 of a block of 16;
+//   O^T[d, query] = V^T x P^T   the contraction index is matched to that: the lane loads the kChunk elements d = kChunk j ... of
+//                               its eight keys (whole rows per instruction) and transposes them in its registers, one
+//                               byte-permute per dword; product c yields the rows d = kChunk (4 g + r) + c.
+// The wavefronts' (maximum, sum, O) are combined through LDS; where sequences x key heads leave compute units idle, a
+// sequence's keys are split over workgroups as well and a second kernel combines those.
+// 16 sequences of 256-1023 keys, 32 heads (165 MB of keys and values): 41.3 us with the kernel above, 32.1 us here (5.1 TB/s); 64
+// sequences of 125-500 keys, 8 key heads for 32 (85 MB): 73.3 and 17.4 us.
+constexpr int kSlots = 16;     // queries (heads of the group x tokens) of a workgroup
+constexpr int kStepKeys = 32;
+
+// one workgroup's result for a query: unnormalised O, its maximum (of scale * log2 e * score) and its sum
+constexpr int partial_floats(int hs) { return hs + 4; }  // + maximum, sum; padded to whole 16-byte units
+
+typedef float float4w __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ float rows_max(float x) {  // over lane % 16 == const
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return halves_max(fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1])));
+}
+__device__ __forceinline__ float rows_sum(float x) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return halves_sum(__uint_as_float(r[0]) + __uint_as_float(r[1]));
+}
+
+template <int HS, bool SPLIT>
+__global__ __launch_bounds__(256, 2) void decode_attention_f16(
+    const _Float16* __restrict__ q_buf, const _Float16* __restrict__ k_cache, const _Float16* __restrict__ v_cache,
+    _Float16* __restrict__ out, float* __restrict__ partial, const int* history_length, const int* input_length,
+    const int* context_length, int head_num, int kv_head_num, int max_q_len, int max_k_len, int max_seq_len, int tokens,
+    float scale_log2e) {
+    constexpr int kChunk = HS / 16, kDSteps = HS / 32, kWords = kChunk / 2;  // kWords: dwords of a lane's piece of a value row
+    const int tid = threadIdx.x, lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64), j = lane % 16, g = lane / 16;
+    const int kv_head = blockIdx.x, b = blockIdx.y;
+    const int group = head_num / kv_head_num;
+    const int len = min(read_only_i32(input_length, b), max_q_len);
+    const int used = SPLIT ? group * max_q_len : group * len;  // slots with a result
+    if (len <= 0 && !SPLIT) return;
+    const int hist = read_only_i32(history_length, b);
+    const int ctx = min(min(read_only_i32(context_length, b), max_k_len), max_seq_len);
+    const int wg_visible = len > 0 ? max(0, min(hist + len, ctx)) : 0;
+    const int head_in_group = j % group, my_q = j / group;
+    const bool real = j < group * len;
+    const int my_visible = real ? min(hist + my_q + 1, ctx) : 0;
+    const size_t kv_offset = ((size_t)b * kv_head_num + kv_head) * (size_t)max_seq_len * HS;
+    const _Float16 *keys = k_cache + kv_offset, *values = v_cache + kv_offset;
+
+    half8 qf[kDSteps];
+    {
+        const _Float16* q_row =
+            q_buf + (((size_t)b * head_num + kv_head * group + (real ? head_in_group : 0)) * (size_t)max_q_len + (real ? my_q : 0)) * HS;
+#pragma unroll
+        for (int i = 0; i < kDSteps; i++) {
+            qf[i] = *reinterpret_cast<const half8*>(q_row + 32 * i + 8 * g);
+            if (!real) qf[i] = half8{0, 0, 0, 0, 0, 0, 0, 0};
+        }
+    }
+    const int all_steps = (wg_visible + kStepKeys - 1) / kStepKeys;
+    const int per_split = (all_steps + (int)gridDim.z - 1) / (int)gridDim.z;
+    const int first = (int)blockIdx.z * per_split, last = min(all_steps, first + per_split);
+
+    struct Step {
+        half8 k[2][kDSteps];
+        uint32_t v[8][kWords];
+    } buf[2];
+    auto load = [&](int which, int s) {  // a key past the visible ones re-reads the last visible row: masked below
+        Step& t = buf[which];
+#pragma unroll
+        for (int blk = 0; blk < 2; blk++) {
+            const _Float16* row = keys + (size_t)min(s * kStepKeys + 16 * blk + j, wg_visible - 1) * HS + 8 * g;
+#pragma unroll
+            for (int i = 0; i < kDSteps; i++) t.k[blk][i] = *reinterpret_cast<const half8*>(row + 32 * i);
+        }
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            const _Float16* row = values + (size_t)min(s * kStepKeys + 16 * (i / 4) + 4 * g + i % 4, wg_visible - 1) * HS + kChunk * j;
+            if constexpr (kWords == 4) {
+                const uint4 x = *reinterpret_cast<const uint4*>(row);
+                t.v[i][0] = x.x, t.v[i][1] = x.y, t.v[i][2] = x.z, t.v[i][3] = x.w;
+            } else {
+                const uint2 x = *reinterpret_cast<const uint2*>(row);
+                t.v[i][0] = x.x, t.v[i][1] = x.y;
+            }
+        }
+    };
+    float4w acc[kChunk];
+#pragma unroll
+    for (int c = 0; c < kChunk; c++) acc[c] = float4w{0.0f, 0.0f, 0.0f, 0.0f};
+    float run_max = -INFINITY, run_sum = 0.0f;  // run_sum: this lane's keys only
+    auto compute = [&](int which, int s) {
+        const Step& t = buf[which];
+        float4w sc[2];
+#pragma unroll
+        for (int blk = 0; blk < 2; blk++) {
+            sc[blk] = float4w{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int i = 0; i < kDSteps; i++) sc[blk] = __builtin_amdgcn_mfma_f32_16x16x32_f16(t.k[blk][i], qf[i], sc[blk], 0, 0, 0);
+        }
+        float m = -INFINITY;
+#pragma unroll
+        for (int blk = 0; blk < 2; blk++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const int key = s * kStepKeys + 16 * blk + 4 * g + r;
+                sc[blk][r] = key < my_visible ? sc[blk][r] * scale_log2e : -INFINITY;
+                m = fmaxf(m, sc[blk][r]);
+            }
+        const float new_max = fmaxf(run_max, rows_max(m));
+        const float safe_max = new_max == -INFINITY ? 0.0f : new_max;  // no visible key yet
+        const float rescale = __builtin_amdgcn_exp2f(run_max - safe_max);
+        run_max = new_max;
+        run_sum *= rescale;
+        half8 p;
+#pragma unroll
+        for (int blk = 0; blk < 2; blk++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const float e = __builtin_amdgcn_exp2f(sc[blk][r] - safe_max);
+                run_sum += e;
+                p[4 * blk + r] = (_Float16)e;
+            }
+        if (__any(rescale != 1.0f)) {
+#pragma unroll
+            for (int c = 0; c < kChunk; c++) acc[c] *= rescale;
+        }
+#pragma unroll
+        for (int c = 0; c < kChunk; c++) {
+            union { uint32_t u[4]; half8 h; } vt;
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+                vt.u[i] = __builtin_amdgcn_perm(t.v[2 * i + 1][c / 2], t.v[2 * i][c / 2], c % 2 ? 0x07060302u : 0x05040100u);
+            acc[c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vt.h, p, acc[c], 0, 0, 0);
+        }
+    };
+    int s = first + wave;
+    if (s < last) {
+        load(0, s);
+        for (;;) {
+            if (s + kWaves >= last) {
+                compute(0, s);
+                break;
+            }
+            load(1, s + kWaves);
+            compute(0, s);
+            s += kWaves;
+            if (s + kWaves >= last) {
+                compute(1, s);
+                break;
+            }
+            load(0, s + kWaves);
+            compute(1, s);
+            s += kWaves;
+        }
+    }
+
+    __shared__ __align__(16) float o_lds[kWaves][kSlots][HS];
+    __shared__ float m_lds[kWaves][kSlots], l_lds[kWaves][kSlots];
+    run_sum = rows_sum(run_sum);
+    if (g == 0) {
+        m_lds[wave][j] = run_max;
+        l_lds[wave][j] = run_sum;
+    }
+    if (j < used) {
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+#pragma unroll
+            for (int c = 0; c < kChunk; c += 4)
+                *reinterpret_cast<float4w*>(&o_lds[wave][j][kChunk * (4 * g + r) + c]) =
+                    float4w{acc[c][r], acc[c + 1][r], acc[c + 2][r], acc[c + 3][r]};
+    }
+    int first_token = 0;
+    if (!SPLIT) {
+        int n = 0;
+        for (int i = lane; i < b; i += 64) n += read_only_i32(input_length, i);
+        for (int off = 32; off > 0; off >>= 1) n += __shfl_xor(n, off, 64);
+        first_token = n;
+    }
+    __syncthreads();
+    for (int at = tid; at < used * (HS / 4); at += 256) {
+        const int slot = at / (HS / 4), d = 4 * (at % (HS / 4));
+        float m = m_lds[0][slot];
+#pragma unroll
+        for (int w = 1; w < kWaves; w++) m = fmaxf(m, m_lds[w][slot]);
+        const float safe = m == -INFINITY ? 0.0f : m;
+        float4w o = {0.0f, 0.0f, 0.0f, 0.0f};
+        float l = 0.0f;
+#pragma unroll
+        for (int w = 0; w < kWaves; w++) {
+            const float e = __builtin_amdgcn_exp2f(m_lds[w][slot] - safe);
+            l += e * l_lds[w][slot];
+            o += e * *reinterpret_cast<const float4w*>(&o_lds[w][slot][d]);
+        }
+        const int head = kv_head * group + slot % group, q = slot / group;
+        if (SPLIT) {
+            float* p = partial + ((((size_t)b * head_num + head) * max_q_len + q) * gridDim.z + blockIdx.z) * partial_floats(HS);
+            *reinterpret_cast<float4w*>(p + d) = o;
+            if (d == 0) p[HS] = m, p[HS + 1] = l;
+        } else {
+            const long long token = (long long)first_token + q;
+            if (token < tokens) {
+                const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+                half4 h;
+#pragma unroll
+                for (int e = 0; e < 4; e++) h[e] = (_Float16)(o[e] * inv);
+                *reinterpret_cast<half4*>(out + ((size_t)token * head_num + head) * HS + d) = h;
+            }
+        }
+    }
+}
+
+// The splits of a query together: a wavefront per (head, sequence and token), HS / 64 elements per lane.
+template <int HS>
+__global__ __launch_bounds__(64) void combine_splits_f16(const float* __restrict__ partial, _Float16* __restrict__ out,
+                                                         const int* input_length, int head_num, int max_q_len, int splits,
+                                                         int tokens) {
+    const int lane = threadIdx.x, head = blockIdx.x, b = (int)blockIdx.y / max_q_len, q = (int)blockIdx.y % max_q_len;
+    int n = 0;
+    for (int i = lane; i < b; i += 64) n += read_only_i32(input_length, i);
+    const float* p = partial + (((size_t)b * head_num + head) * max_q_len + q) * (size_t)splits * partial_floats(HS);
+    float m = -INFINITY, l = 0.0f;
+    for (int z = lane; z < splits; z += 64) m = fmaxf(m, p[z * partial_floats(HS) + HS]);
+    for (int off = 32; off > 0; off >>= 1) {
+        m = fmaxf(m, __shfl_xor(m, off, 64));
+        n += __shfl_xor(n, off, 64);
+    }
+    const float safe = m == -INFINITY ? 0.0f : m;
+    float o[HS / 64] = {};
+    for (int z = 0; z < splits; z++) {
+        const float* pz = p + z * partial_floats(HS);
+        const float e = __builtin_amdgcn_exp2f(pz[HS] - safe);
+        l += e * pz[HS + 1];
+#pragma unroll
+        for (int i = 0; i < HS / 64; i++) o[i] += e * pz[HS / 64 * lane + i];
+    }
+    const long long token = (long long)n + q;
+    if (q >= read_only_i32(input_length, b) || token >= tokens) return;
+    const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+#pragma unroll
+    for (int i = 0; i < HS / 64; i++) out[((size_t)token * head_num + head) * HS + HS / 64 * lane + i] = (_Float16)(o[i] * inv);
+}
+
 }  // namespace
 
-static int context_attention(const _Float16* q, const _Float16* k_cache, const _Float16* v_cache, _Float16* out,
-                             const int32_t* history_length, const int32_t* input_length, const int32_t* context_length,
-                             int layer, int batch, int head_num, int kv_head_num, int head_size, int max_q_len,
-                             int max_k_len, int max_seq_len, int token_num, float scale, hipStream_t stream) {
+// Workgroups that share a (sequence, key head): enough for two on every compute unit, each with at least 128 keys (four
+// steps, one per wavefront).
+int attention_splits(int batch, int head_num, int kv_head_num, int max_q_len, int max_k_len) {
+    if (batch <= 0 || kv_head_num <= 0 || head_num / kv_head_num * (long long)max_q_len > kSlots) return 1;
+    const long long groups = (long long)batch * kv_head_num, units = resident_waves() / 32;
+    long long splits = (2 * units) / groups;
+    const long long most = (max_k_len + 4 * kStepKeys - 1) / (4 * kStepKeys);
+    if (splits > most) splits = most;
+    return splits < 1 ? 1 : (int)splits;
+}
+
+size_t attention_workspace(int batch, int head_num, int kv_head_num, int head_size, int max_q_len, int max_k_len) {
+    const int splits = attention_splits(batch, head_num, kv_head_num, max_q_len, max_k_len);
+    return splits == 1 ? 0 : (size_t)splits * batch * head_num * max_q_len * partial_floats(head_size) * sizeof(float);
+}
+
+// `workspace` NULL: a sequence's keys are not split.
+int context_attention(const _Float16* q, const _Float16* k_cache, const _Float16* v_cache, _Float16* out,
+                      const int32_t* history_length, const int32_t* input_length, const int32_t* context_length,
+                      int layer, int batch, int head_num, int kv_head_num, int head_size, int max_q_len,
+                      int max_k_len, int max_seq_len, int token_num, float scale, float* workspace, hipStream_t stream) {
     if (layer < 0 || batch < 0 || head_num <= 0 || kv_head_num <= 0 || head_num % kv_head_num != 0 || max_q_len < 0 ||
         max_k_len < 0 || max_seq_len < 0 || token_num < 0 || !(scale > 0.0f))
         return ISP_ERR_BAD_SHAPE;
@@ -302,11 +567,39 @@ static int context_attention(const _Float16* q, const _Float16* k_cache, const _
     ISP_REQUIRE_PTR(context_length);
     if (!aligned16(q) || !aligned16(k_cache) || !aligned16(v_cache) || !aligned16(out)) return ISP_ERR_UNSUPPORTED;
     const size_t slice = (size_t)layer * batch * kv_head_num * max_seq_len * head_size;
+    const float scale_log2e = scale * 1.4426950408889634f;
+    if ((long long)(head_num / kv_head_num) * max_q_len <= kSlots) {
+        if (!aligned16(workspace) || (long long)batch * max_q_len > 65535) return ISP_ERR_UNSUPPORTED;
+        const int splits = workspace ? attention_splits(batch, head_num, kv_head_num, max_q_len, max_k_len) : 1;
+        const dim3 grid((unsigned)kv_head_num, (unsigned)batch, (unsigned)splits);
+#define ISP_LAUNCH_DECODE(HS, SPLIT)                                                                                          \
+    hipLaunchKernelGGL((decode_attention_f16<HS, SPLIT>), grid, dim3(256), 0, stream, q, k_cache + slice, v_cache + slice, out, \
+                       workspace, history_length, input_length, context_length, head_num, kv_head_num, max_q_len, max_k_len,  \
+                       max_seq_len, token_num, scale_log2e)
+        if (splits == 1) {
+            if (head_size == 128) ISP_LAUNCH_DECODE(128, false);
+            else ISP_LAUNCH_DECODE(64, false);
+            return note_launch(hipGetLastError());
+        }
+        if (head_size == 128) ISP_LAUNCH_DECODE(128, true);
+        else ISP_LAUNCH_DECODE(64, true);
+#undef ISP_LAUNCH_DECODE
+        const int status = note_launch(hipGetLastError());
+        if (status != ISP_OK) return status;
+        const dim3 queries((unsigned)head_num, (unsigned)(batch * max_q_len));
+        if (head_size == 128)
+            hipLaunchKernelGGL(combine_splits_f16<128>, queries, dim3(64), 0, stream, workspace, out, input_length, head_num,
+                               max_q_len, splits, token_num);
+        else
+            hipLaunchKernelGGL(combine_splits_f16<64>, queries, dim3(64), 0, stream, workspace, out, input_length, head_num,
+                               max_q_len, splits, token_num);
+        return note_launch(hipGetLastError());
+    }
     const dim3 grid((unsigned)head_num, (unsigned)batch, (unsigned)tiles);
 #define ISP_LAUNCH_ATTENTION(HS)                                                                                    \
     hipLaunchKernelGGL(context_attention_f16<HS>, grid, dim3(256), 0, stream, q, k_cache + slice, v_cache + slice, out, \
                        history_length, input_length, context_length, head_num, kv_head_num, max_q_len, max_k_len,   \
-                       max_seq_len, token_num, scale * 1.4426950408889634f)
+                       max_seq_len, token_num, scale_log2e)
     if (head_size == 128) ISP_LAUNCH_ATTENTION(128);
     else ISP_LAUNCH_ATTENTION(64);
 #undef ISP_LAUNCH_ATTENTION
@@ -315,13 +608,32 @@ static int context_attention(const _Float16* q, const _Float16* k_cache, const _
 
 }  // namespace isp
 
-extern "C" int isp_context_attention_f16(const void* q, const void* k_cache, const void* v_cache, void* out,
-                                         const int32_t* history_length, const int32_t* input_length,
-                                         const int32_t* context_length, int layer, int batch, int head_num,
-                                         int kv_head_num, int head_size, int max_q_len, int max_k_len, int max_seq_len,
-                                         int token_num, float scale, isp_stream_t stream) {
+extern "C" {
+
+size_t isp_context_attention_f16_workspace(int batch, int head_num, int kv_head_num, int head_size, int max_q_len,
+                                           int max_k_len) {
+    return isp::attention_workspace(batch, head_num, kv_head_num, head_size, max_q_len, max_k_len);
+}
+
+int isp_context_attention_split_f16(const void* q, const void* k_cache, const void* v_cache, void* out,
+                                    const int32_t* history_length, const int32_t* input_length,
+                                    const int32_t* context_length, int layer, int batch, int head_num, int kv_head_num,
+                                    int head_size, int max_q_len, int max_k_len, int max_seq_len, int token_num, float scale,
+                                    void* workspace, isp_stream_t stream) {
     return isp::context_attention(static_cast<const _Float16*>(q), static_cast<const _Float16*>(k_cache),
                                   static_cast<const _Float16*>(v_cache), static_cast<_Float16*>(out), history_length,
                                   input_length, context_length, layer, batch, head_num, kv_head_num, head_size, max_q_len,
-                                  max_k_len, max_seq_len, token_num, scale, static_cast<hipStream_t>(stream));
+                                  max_k_len, max_seq_len, token_num, scale, static_cast<float*>(workspace),
+                                  static_cast<hipStream_t>(stream));
 }
+
+int isp_context_attention_f16(const void* q, const void* k_cache, const void* v_cache, void* out,
+                              const int32_t* history_length, const int32_t* input_length, const int32_t* context_length,
+                              int layer, int batch, int head_num, int kv_head_num, int head_size, int max_q_len,
+                              int max_k_len, int max_seq_len, int token_num, float scale, isp_stream_t stream) {
+    return isp_context_attention_split_f16(q, k_cache, v_cache, out, history_length, input_length, context_length, layer,
+                                           batch, head_num, kv_head_num, head_size, max_q_len, max_k_len, max_seq_len,
+                                           token_num, scale, nullptr, stream);
+}
+
+}  // extern "C"

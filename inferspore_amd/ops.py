@@ -317,10 +317,12 @@ def context_attention(q_buf, k_cache, v_cache, layer_id, history_length, input_l
     _expect(min(history_length.numel(), input_length.numel(), context_length.numel()) >= batch,
             "length tensors are shorter than the batch")
     _dev(q_buf, k_cache, v_cache, history_length, input_length, context_length, out)
-    capi.check(capi.lib().isp_context_attention_f16(
+    need = capi.lib().isp_context_attention_f16_workspace(batch, head_num, kv_head_num, head_size, max_q_len, int(max_k_len))
+    workspace = torch.empty(need, dtype=torch.uint8, device=q_buf.device) if need else None
+    capi.check(capi.lib().isp_context_attention_split_f16(
         _p(q_buf), _p(k_cache), _p(v_cache), _p(out), _p(history_length), _p(input_length), _p(context_length),
         int(layer_id), batch, head_num, kv_head_num, head_size, max_q_len, int(max_k_len), max_seq_len, out.shape[0],
-        float(head_size ** -0.5 if scale is None else scale), _stream()), "isp_context_attention")
+        float(head_size ** -0.5 if scale is None else scale), _p(workspace), _stream()), "isp_context_attention")
     return out
 
 

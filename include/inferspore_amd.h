@@ -301,6 +301,29 @@ size_t isp_linear_f16_workspace(int m, int n, int k);
 int isp_linear_f16(const void* a, const void* w, void* out, void* workspace, int m, int n, int k, isp_stream_t stream);
 
 /*
+ * A whole context-decoder layer for up to 64 packed fp16 rows (a decode step, a short prompt) in one call: QKV product,
+ * bias + RoPE + KV append, attention, output projection, residual + RMSNorm by ffn_norm, gate / up product, SwiGLU, down
+ * projection, residual + RMSNorm by next_norm.  What the reference's kernels do one by one (src/kernels/linear.cu,
+ * qkv_bias_and_RoPE.cu, concat_past_kv.cu, fused_addresidual_norm.cu, act_kernel.cu).
+ *   normed, out [token_num, hidden]; residual likewise, updated in place; qkv_weight [hidden, (head_num + 2 kv_head_num) *
+ *   head_size], qkv_bias its columns or NULL; o_weight [head_num * head_size, hidden]; gate_up_weight [hidden, 2 inter];
+ *   down_weight [inter, hidden]; q, k_cache, v_cache, padding_offset and the lengths as for the entry points above;
+ *   context [token_num, head_num * head_size] and act [token_num, inter] are written on the way;
+ *   workspace: isp_context_layer_f16_workspace() bytes that no other work in flight uses (0: the shape is unsupported).
+ * ISP_ERR_UNSUPPORTED: more rows, head_size other than 64 / 128, hidden or inter not a multiple of 8, hidden > 8192, more
+ * than 32768 columns in a product of more than 16 rows, pointers that are not 16-byte aligned.
+ */
+size_t isp_context_layer_f16_workspace(int batch, int token_num, int hidden, int head_num, int kv_head_num, int head_size,
+                                       int max_q_len, int max_k_len, int max_seq_len, int inter);
+int isp_context_layer_f16(const void* normed, void* residual, void* out, const void* qkv_weight, const void* qkv_bias,
+                          const void* o_weight, const void* gate_up_weight, const void* down_weight, const void* ffn_norm,
+                          const void* next_norm, void* q, void* k_cache, void* v_cache, void* context, void* act,
+                          const int32_t* padding_offset, const int32_t* history_length, const int32_t* input_length,
+                          const int32_t* context_length, void* workspace, int layer, int batch, int token_num, int hidden,
+                          int head_num, int kv_head_num, int head_size, int max_q_len, int max_k_len, int max_seq_len, int inter,
+                          int rotary_dim, float rotary_base, float eps, isp_stream_t stream);
+
+/*
  * Measurement aids (no reference counterpart).
  * isp_calibration_copy: a plain copy kernel of known traffic (`bytes` read + `bytes` written;
  *   16-byte aligned, multiple of 16) used to calibrate profiler byte counters and to measure the

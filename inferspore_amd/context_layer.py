@@ -18,13 +18,15 @@ order a model runs them:
     residual, normed_next = fused_add_bias_residual_rmsnorm(residual, ffn_out, next attn_norm)   * this library
 
 Dense contractions of more than 64 rows are left to torch's library calls (hipBLASLt GEMMs), those of fewer float16 rows go to
-ops.linear; everything marked * goes through the C ABI.  All work is issued on torch's current stream.
+ops.linear, and a layer of such rows is one call of the C ABI (isp_context_layer_f16); everything marked * goes through the C ABI.  All work is issued on torch's current stream.
 """
 import math
 
 import torch
 
-from . import ops
+from . import capi, ops
+
+_PLAIN = (torch.Tensor, torch.nn.Parameter)
 
 
 class LayerWeights:
@@ -99,6 +101,50 @@ class BatchState:
         return mask
 
 
+def _layer_in_one_call(normed, residual, w, st, layer_id, gamma, rotary_dim, rotary_base, eps):
+    """The whole layer as one call of the C ABI, or None where it is not the plain case of a few float16 rows: everything
+    that the steps below accept or refuse otherwise stays with them."""
+    if normed.dtype != torch.float16 or normed.dim() != 2 or not 0 < normed.shape[0] <= 64:
+        return None
+    (tokens, hidden), batch, heads, kv, hs = normed.shape, st.batch, st.head_num, st.kv_head_num, st.head_size
+    inter, width, max_seq = st.act.shape[-1], (heads + 2 * kv) * hs, st.k_cache.shape[3]
+    halves = ((normed, (tokens, hidden)), (residual, (tokens, hidden)), (w.qkv, (hidden, width)), (w.qkv_bias, (width,)),
+              (w.o, (heads * hs, hidden)), (w.gate_up, (hidden, 2 * inter)), (w.down, (inter, hidden)), (w.ffn_norm, (hidden,)),
+              (gamma, (hidden,)), (st.q, (batch, heads, st.max_q_len, hs)),
+              (st.k_cache, (st.k_cache.shape[0], batch, kv, max_seq, hs)), (st.v_cache, tuple(st.k_cache.shape)),
+              (st.packed_ctx, (tokens, heads, hs)), (st.act, (tokens, inter)))
+    grad, device = torch.is_grad_enabled(), normed.device
+    if not normed.is_cuda or torch.is_autocast_enabled():
+        return None
+    for t, shape in halves:
+        if t is None and shape == (width,):
+            continue
+        if (type(t) not in _PLAIN or t.dtype != torch.float16 or t.shape != shape or not t.is_contiguous() or
+                t.device != device or t.data_ptr() % 16 or (grad and t.requires_grad)):
+            return None
+    for t, most in ((st.padding_offset, tokens), (st.history, batch), (st.lengths, batch), (st.context, batch)):
+        if (type(t) not in _PLAIN or t.dtype != torch.int32 or t.numel() < most or not t.is_contiguous() or
+                t.device != device):
+            return None
+    if not (st.tokens == tokens and 0 <= int(layer_id) < st.k_cache.shape[0] and
+            0 <= int(rotary_dim) <= hs and int(rotary_dim) % 2 == 0) or normed.data_ptr() == residual.data_ptr():
+        return None
+    lib = capi.lib()
+    need = lib.isp_context_layer_f16_workspace(batch, tokens, hidden, heads, kv, hs, st.max_q_len, st.max_k_len, max_seq, inter)
+    if need == 0:
+        return None
+    workspace = torch.empty(need, dtype=torch.uint8, device=device)
+    out = torch.empty_like(normed)
+    p = torch.Tensor.data_ptr
+    capi.check(lib.isp_context_layer_f16(
+        p(normed), p(residual), p(out), p(w.qkv), None if w.qkv_bias is None else p(w.qkv_bias), p(w.o), p(w.gate_up),
+        p(w.down), p(w.ffn_norm), p(gamma), p(st.q), p(st.k_cache), p(st.v_cache), p(st.packed_ctx), p(st.act),
+        p(st.padding_offset), p(st.history), p(st.lengths), p(st.context), p(workspace), int(layer_id), batch, tokens, hidden,
+        heads, kv, hs, st.max_q_len, st.max_k_len, max_seq, inter, int(rotary_dim), float(rotary_base), float(eps),
+        torch.cuda.current_stream().cuda_stream), "isp_context_layer")
+    return out
+
+
 def _linear(x, w):
     return ops.linear(x, w) if ops.linear_supports(x, w) else x @ w
 
@@ -108,6 +154,9 @@ def context_decoder_layer(normed, residual, w, state, layer_id, next_norm_gamma,
     """Runs one prefill layer.  `normed` and `residual` are packed [tokens, H]; `residual` is updated in
     place; returns the next layer's normalised input (a new tensor)."""
     st = state
+    out = _layer_in_one_call(normed, residual, w, st, layer_id, next_norm_gamma, rotary_dim, rotary_base, eps)
+    if out is not None:
+        return out
     qkv = _linear(normed, w.qkv)                                                 # [tokens, 3H]
     qkv = qkv.view(st.tokens, st.head_num + 2 * st.kv_head_num, st.head_size)
     # bias + RoPE + re-pad of q, with k and v written straight into the cache (one launch, no padded k / v)

@@ -134,8 +134,8 @@ __global__ __launch_bounds__(kBlock) void linear_skinny_f16(const __half* __rest
                 if (SPLIT) {
                     *reinterpret_cast<float4v*>(partial + (size_t)blockIdx.y * (size_t)m * (size_t)n + at) = sum;
                 } else {
-                    __half2 lo = __floats2half2_rn(sum[0], sum[1]), hi = __floats2half2_rn(sum[2], sum[3]);
-                    *reinterpret_cast<uint2*>(out + at) = make_uint2(*reinterpret_cast<uint32_t*>(&lo), *reinterpret_cast<uint32_t*>(&hi));
+                    const __half2 lo = __floats2half2_rn(sum[0], sum[1]), hi = __floats2half2_rn(sum[2], sum[3]);
+                    *reinterpret_cast<uint2*>(out + at) = make_uint2(*reinterpret_cast<const uint32_t*>(&lo), *reinterpret_cast<const uint32_t*>(&hi));
                 }
             }
         }
@@ -174,5 +174,36 @@ inline SkinnyPlan skinny_plan(int m, int n, int k) {
 // Partial sums of the product to `partial`, or with `out` (one split only) the fp16 product itself.  Operands checked by the caller.
 void launch_skinny(const SkinnyPlan& plan, const __half* a, const __half* w, __half* out, float* partial, int m, int n, int k,
                    hipStream_t stream);
+
+// Eight neighbouring columns of a product left as partial sums: the splits added in their order and rounded to fp16 once, the
+// value linear_add_splits would have stored.  `stride`: floats between two splits.
+__device__ __forceinline__ vec16 add_splits8(const float* p, size_t stride, int splits) {
+    float4v a = *reinterpret_cast<const float4v*>(p), b = *reinterpret_cast<const float4v*>(p + 4);
+#pragma unroll 4
+    for (int s = 1; s < splits; s++) {
+        a += *reinterpret_cast<const float4v*>(p + s * stride);
+        b += *reinterpret_cast<const float4v*>(p + s * stride + 4);
+    }
+    const float f[8] = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
+    return Elem<__half>::pack(f);
+}
+
+// Consumers of partial sums: what the entry points of the same step do with a stored fp16 product (same bits), with that
+// product's addition of splits, its store and its read back taken out.  Operands checked by the caller.
+void launch_qkv_sums(const float* partial, int splits, const __half* bias, __half* q, __half* k_cache, __half* v_cache,
+                     const int32_t* padding_offset, const int32_t* history_length, const int32_t* input_length, int batch,
+                     int seq_len, int tokens, int head_num, int kv_head_num, int head_size, int max_seq_len, int rot, float base,
+                     hipStream_t stream);
+void launch_norm_sums(const float* partial, int splits, __half* residual, __half* out, const __half* gamma, float eps,
+                      int tokens, int hidden, hipStream_t stream);
+constexpr int kNormSumsMaxHidden = 8192;
+void launch_swiglu_sums(const float* partial, int splits, __half* out, int tokens, int inter, hipStream_t stream);
+
+// csrc/context_attention.hip
+size_t attention_workspace(int batch, int head_num, int kv_head_num, int head_size, int max_q_len, int max_k_len);
+int context_attention(const _Float16* q, const _Float16* k_cache, const _Float16* v_cache, _Float16* out,
+                      const int32_t* history_length, const int32_t* input_length, const int32_t* context_length,
+                      int layer, int batch, int head_num, int kv_head_num, int head_size, int max_q_len,
+                      int max_k_len, int max_seq_len, int token_num, float scale, float* workspace, hipStream_t stream);
 
 }  // namespace isp

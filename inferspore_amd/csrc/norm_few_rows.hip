@@ -6,6 +6,7 @@
 // that is nothing but a chain of round trips (64 x 4096 fp32: 2.40 against 2.64 us per launch; 256 rows 3.2
 // against 3.4).  The general kernel (norm.hip) is built without it: the benchmark configuration, 2048 x 4096
 // fp16 with residual and bias in one round of waves, measured 1 % slower with it.
+#include "linear_rows.h"
 #include "norm_rows.h"
 
 namespace isp {
@@ -52,5 +53,46 @@ NormFewKernel<T> norm_few_variant(int wpr, int nv, int st, int ops) {
 
 template NormFewKernel<float> norm_few_variant<float>(int, int, int, int);
 template NormFewKernel<__half> norm_few_variant<__half>(int, int, int, int);
+
+// Residual + RMSNorm of a product left as partial sums [splits][tokens][hidden]: a row per workgroup, one vector per lane;
+// the operations and their order are norm_rows_body's (absent waves add exact zeros), so the bits are too.
+__global__ __launch_bounds__(1024) void fused_norm_sums_f16(const float* __restrict__ partial, int splits, __half* __restrict__ residual,
+                                                            __half* __restrict__ out, const __half* __restrict__ gamma, float eps,
+                                                            int tokens, int hidden) {
+    __shared__ float sums[16];
+    const int tid = threadIdx.x, waves = blockDim.x / kWave;
+    const bool ok = tid * 8 < hidden;
+    const size_t at = (size_t)blockIdx.x * (size_t)hidden + (size_t)(ok ? tid : 0) * 8u;
+    const vec16 vr = load16(residual + at), vg = load16(gamma + (ok ? tid : 0) * 8);
+    const vec16 vo = add_splits8(partial + at, (size_t)tokens * (size_t)hidden, splits);
+    float x[8];
+    Elem<__half>::sum(vo, vr, x);
+#pragma unroll
+    for (int e = 0; e < 8; e++) x[e] = Elem<__half>::pinned(x[e]);
+    float p = x[0] * x[0];
+#pragma unroll
+    for (int e = 1; e < 8; e++) p = __fmaf_rn(x[e], x[e], p);
+    p = wave_sum(ok ? p : 0.0f);
+    if (tid % kWave == 0) sums[tid / kWave] = p;
+    __syncthreads();
+    float part[16];
+#pragma unroll
+    for (int w = 0; w < 16; w++) part[w] = w < waves ? sums[w] : 0.0f;
+    const float inv = rsqrtf(tree_sum<16>(part) / (float)hidden + eps);
+    if (!ok) return;
+    store16(residual + at, Elem<__half>::pack_pinned(x));
+    float y[8];
+    Elem<__half>::scale(vg, x, y);
+#pragma unroll
+    for (int e = 0; e < 8; e++) y[e] *= inv;
+    store16(out + at, Elem<__half>::pack(y));
+}
+
+void launch_norm_sums(const float* partial, int splits, __half* residual, __half* out, const __half* gamma, float eps,
+                      int tokens, int hidden, hipStream_t stream) {
+    const unsigned threads = (unsigned)((hidden / 8 + kWave - 1) / kWave * kWave);
+    hipLaunchKernelGGL(fused_norm_sums_f16, dim3((unsigned)tokens), dim3(threads), 0, stream, partial, splits, residual, out,
+                       gamma, eps, tokens, hidden);
+}
 
 }  // namespace isp

@@ -30,7 +30,7 @@
 
 #include <type_traits>
 
-#include "isp_common.h"
+#include "linear_rows.h"
 
 namespace isp {
 
@@ -1246,6 +1246,90 @@ static int qkv_rope(void* q_, void* k_, void* v_, const void* qkv_, const void* 
         e = hipGetLastError();
     }
     return note_launch(e);
+}
+
+// The fused QKV step (bias, rotation, re-padded queries, keys and values into the cache) of a product left as partial sums
+// [splits][tokens][heads * head_size], for the few rows of a decode step: a lane owns eight elements of a half head row and
+// their rotation partners, the first lanes of every workgroup evaluate the token's (cos, sin) pairs beside its loads.
+// Same operations per element as the kernels above: same bits.  grid = (tokens, units of 256 lanes).
+__global__ __launch_bounds__(kBlock) void qkv_rope_sums_f16(RopeDivisors tab, const float* __restrict__ partial, int splits,
+                                                            const __half* __restrict__ bias, __half* __restrict__ q,
+                                                            const int32_t* __restrict__ padding_offset,
+                                                            const int32_t* __restrict__ history_length, unsigned positions,
+                                                            FastDiv seq, FastDiv half_units, int tokens, int head_num,
+                                                            int kv_head_num, int half_rot, KvAppend<__half> ap) {
+    __shared__ float2 cs[kMaxHalfRot];
+    const int token = (int)blockIdx.x, half = (int)half_units.d * 8, hs = 2 * half, heads = head_num + 2 * kv_head_num;
+    const unsigned unit = blockIdx.y * kBlock + threadIdx.x, units = (unsigned)heads * half_units.d;
+    const bool live = unit < units;
+    unsigned h, g;
+    half_units.divmod(live ? unit : 0u, h, g);
+    const size_t col = (size_t)h * hs + (size_t)g * 8u, width = (size_t)heads * hs;
+    const float* src = partial + (size_t)token * width + col;
+    const vec16 lo = add_splits8(src, (size_t)tokens * width, splits);
+    const vec16 hi = add_splits8(src + half, (size_t)tokens * width, splits);
+    vec16 blo, bhi;
+    if (bias) {
+        blo = load16(bias + col);
+        bhi = load16(bias + col + half);
+    }
+    const long long p = (long long)token + (long long)read_only_i32(padding_offset, token);
+    if (p < 0 || p >= (long long)positions) return;  // workgroup-uniform
+    unsigned b, s;
+    seq.divmod((unsigned)p, b, s);
+    if ((int)threadIdx.x < half_rot)
+        cs[threadIdx.x] = rope_coefficients(read_only_i32(history_length, (int)b) + (int)s, tab.div[threadIdx.x]);
+    __syncthreads();
+    if (!live) return;
+    float x0[8], x1[8];
+    Elem<__half>::unpack(lo, x0);
+    Elem<__half>::unpack(hi, x1);
+    if (bias) {
+        float b0[8], b1[8];
+        Elem<__half>::unpack(blo, b0);
+        Elem<__half>::unpack(bhi, b1);
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+            x0[e] += b0[e];
+            x1[e] += b1[e];
+        }
+    }
+    const bool rotates = (int)h < head_num + kv_head_num;
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+        const int d = (int)g * 8 + e;
+        if (rotates && d < half_rot) {
+            const float2 c = cs[d];
+            float y0, y1;
+            rotate_pair(c.x, c.y, x0[e], x1[e], y0, y1);
+            x0[e] = y0;
+            x1[e] = y1;
+        }
+    }
+    __half* dst;
+    if ((int)h < head_num) {
+        dst = q + (((size_t)b * head_num + h) * seq.d + s) * hs;
+    } else {
+        const long long row = append_row(ap, history_length, (int)b, (int)s);
+        if (row < 0) return;
+        const unsigned kvh = rotates ? h - (unsigned)head_num : h - (unsigned)(head_num + kv_head_num);
+        dst = (rotates ? ap.k_cache : ap.v_cache) + (((size_t)b * kv_head_num + kvh) * (size_t)ap.max_seq_len + (size_t)row) * hs;
+    }
+    store16(dst + g * 8u, Elem<__half>::pack(x0));
+    store16(dst + half + g * 8u, Elem<__half>::pack(x1));
+}
+
+void launch_qkv_sums(const float* partial, int splits, const __half* bias, __half* q, __half* k_cache, __half* v_cache,
+                     const int32_t* padding_offset, const int32_t* history_length, const int32_t* input_length, int batch,
+                     int seq_len, int tokens, int head_num, int kv_head_num, int head_size, int max_seq_len, int rot, float base,
+                     hipStream_t stream) {
+    RopeDivisors tab;
+    fill_divisors(tab, rot, base);
+    const unsigned half_units = (unsigned)head_size / 16u, units = (unsigned)(head_num + 2 * kv_head_num) * half_units;
+    hipLaunchKernelGGL(qkv_rope_sums_f16, dim3((unsigned)tokens, (units + kBlock - 1) / kBlock), dim3(kBlock), 0, stream, tab,
+                       partial, splits, bias, q, padding_offset, history_length, (unsigned)batch * (unsigned)seq_len,
+                       make_fastdiv((unsigned)seq_len), make_fastdiv(half_units), tokens, head_num, kv_head_num, rot / 2,
+                       KvAppend<__half>{k_cache, v_cache, input_length, max_seq_len});
 }
 
 }  // namespace isp

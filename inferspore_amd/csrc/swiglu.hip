@@ -5,7 +5,7 @@
 // Design: the output is treated as one flat array of 16-byte vectors, so every lane of every wave
 // is busy whatever the row length (the reference's one-block-per-token loop leaves decode batches
 // with 256 half2-wide blocks); each lane keeps UNROLL gate/up vector pairs in flight.
-#include "isp_common.h"
+#include "linear_rows.h"
 
 namespace isp {
 
@@ -116,6 +116,27 @@ static int swiglu(const void* in_, void* out_, int tokens, int inter, hipStream_
         e = hipGetLastError();
     }
     return note_launch(e);
+}
+
+// SwiGLU of a gate / up product left as partial sums [splits][tokens][2 inter] (inter a multiple of 8).
+__global__ __launch_bounds__(kWave) void swiglu_sums_f16(const float* __restrict__ partial, int splits, __half* __restrict__ out,
+                                                         int tokens, int inter) {
+    const int unit = (int)(blockIdx.x * kWave + threadIdx.x), token = (int)blockIdx.y;
+    if (unit * 8 >= inter) return;
+    const size_t stride = (size_t)tokens * 2u * (size_t)inter;
+    const float* gate = partial + (size_t)token * 2u * (size_t)inter + (size_t)unit * 8u;
+    const vec16 g = add_splits8(gate, stride, splits), u = add_splits8(gate + inter, stride, splits);
+    float a[8], b[8], y[8];
+    Elem<__half>::unpack(g, a);
+    Elem<__half>::unpack(u, b);
+#pragma unroll
+    for (int e = 0; e < 8; e++) y[e] = silu_for<__half>(a[e]) * b[e];
+    store16(out + (size_t)token * (size_t)inter + (size_t)unit * 8u, Elem<__half>::pack(y));
+}
+
+void launch_swiglu_sums(const float* partial, int splits, __half* out, int tokens, int inter, hipStream_t stream) {
+    const dim3 grid((unsigned)((inter / 8 + kWave - 1) / kWave), (unsigned)tokens);
+    hipLaunchKernelGGL(swiglu_sums_f16, grid, dim3(kWave), 0, stream, partial, splits, out, tokens, inter);
 }
 
 }  // namespace isp

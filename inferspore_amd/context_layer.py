@@ -141,7 +141,7 @@ def _layer_in_one_call(normed, residual, w, st, layer_id, gamma, rotary_dim, rot
         p(w.down), p(w.ffn_norm), p(gamma), p(st.q), p(st.k_cache), p(st.v_cache), p(st.packed_ctx), p(st.act),
         p(st.padding_offset), p(st.history), p(st.lengths), p(st.context), p(workspace), int(layer_id), batch, tokens, hidden,
         heads, kv, hs, st.max_q_len, st.max_k_len, max_seq, inter, int(rotary_dim), float(rotary_base), float(eps),
-        torch.cuda.current_stream().cuda_stream), "isp_context_layer")
+        ops._stream()), "isp_context_layer")
     return out
 
 

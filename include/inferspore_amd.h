@@ -279,7 +279,13 @@ int isp_context_attention_f16(const void* q, const void* k_cache, const void* v_
                               const int32_t* context_length, int layer, int batch, int head_num,
                               int kv_head_num, int head_size, int max_q_len, int max_k_len,
                               int max_seq_len, int token_num, float scale, isp_stream_t stream);
-/* The same with a workspace of isp_context_attention_f16_workspace() bytes (16-byte aligned device memory that no other
+/* The same in fp32 throughout, for heads of 128, 96 or 64 elements. */
+int isp_context_attention_f32(const void* q, const void* k_cache, const void* v_cache, void* out,
+                              const int32_t* history_length, const int32_t* input_length,
+                              const int32_t* context_length, int layer, int batch, int head_num,
+                              int kv_head_num, int head_size, int max_q_len, int max_k_len,
+                              int max_seq_len, int token_num, float scale, isp_stream_t stream);
+/* The fp16 form with a workspace of isp_context_attention_f16_workspace() bytes (16-byte aligned device memory that no other
  * work in flight uses; NULL is accepted): where sequences x key heads would leave compute units idle and the heads of a
  * group have at most 16 queries together, several workgroups share a sequence's keys. */
 size_t isp_context_attention_f16_workspace(int batch, int head_num, int kv_head_num, int head_size, int max_q_len,

@@ -48,6 +48,7 @@ SIGNATURES = {
     "isp_repeat_kv_cache_f32": (_i, [_vp, _vp, _vp, _vp, _i, _vp, _i, _i, _i, _i, _i, _i, _vp]),
     "isp_repeat_kv_cache_f16": (_i, [_vp, _vp, _vp, _vp, _i, _vp, _i, _i, _i, _i, _i, _i, _vp]),
     "isp_context_attention_f16": (_i, [_vp] * 7 + [_i] * 9 + [_f, _vp]),
+    "isp_context_attention_f32": (_i, [_vp] * 7 + [_i] * 9 + [_f, _vp]),
     "isp_context_attention_f16_workspace": (C.c_size_t, [_i] * 6),
     "isp_context_attention_split_f16": (_i, [_vp] * 7 + [_i] * 9 + [_f, _vp, _vp]),
     "isp_linear_f16_workspace": (C.c_size_t, [_i, _i, _i]),

@@ -296,7 +296,7 @@ def linear(x, w):
 
 def context_attention_supports(dtype, head_size):
     """Whether context_attention takes heads of this type and size."""
-    return dtype == torch.float16 and head_size in (64, 128)
+    return head_size in ((64, 128) if dtype == torch.float16 else (64, 96, 128) if dtype == torch.float32 else ())
 
 
 def context_attention(q_buf, k_cache, v_cache, layer_id, history_length, input_length, context_length, max_k_len, out,
@@ -312,13 +312,19 @@ def context_attention(q_buf, k_cache, v_cache, layer_id, history_length, input_l
     kv_head_num, max_seq_len = k_cache.shape[2], k_cache.shape[3]
     _expect(k_cache.shape == v_cache.shape and k_cache.shape[1] == batch and k_cache.shape[4] == head_size,
             "caches must be [layers, batch, kv_head_num, max_seq_len, head_size]")
-    _expect(context_attention_supports(q_buf.dtype, head_size), "attention takes float16 heads of 64 or 128 elements")
+    _expect(context_attention_supports(q_buf.dtype, head_size), "attention takes float16 heads of 64 or 128 elements, float32 heads of 64, 96 or 128")
     _expect(kv_head_num > 0 and head_num % kv_head_num == 0, "head_num must be a multiple of kv_head_num")
     _expect(out.shape[1:] == (head_num, head_size), "out must be [tokens, heads, head_size]")
     _expect(0 <= int(layer_id) < k_cache.shape[0], "layer_id outside the cache")
     _expect(min(history_length.numel(), input_length.numel(), context_length.numel()) >= batch,
             "length tensors are shorter than the batch")
     _dev(q_buf, k_cache, v_cache, history_length, input_length, context_length, out)
+    if q_buf.dtype == torch.float32:
+        capi.check(capi.lib().isp_context_attention_f32(
+            _p(q_buf), _p(k_cache), _p(v_cache), _p(out), _p(history_length), _p(input_length), _p(context_length),
+            int(layer_id), batch, head_num, kv_head_num, head_size, max_q_len, int(max_k_len), max_seq_len, out.shape[0],
+            float(head_size ** -0.5 if scale is None else scale), _stream()), "isp_context_attention")
+        return out
     need = capi.lib().isp_context_attention_f16_workspace(batch, head_num, kv_head_num, head_size, max_q_len, int(max_k_len))
     workspace = torch.empty(need, dtype=torch.uint8, device=q_buf.device) if need else None
     capi.check(capi.lib().isp_context_attention_split_f16(

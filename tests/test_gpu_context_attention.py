@@ -2,8 +2,10 @@
 and keys that end inside, at and just past a tile, a single query over long and short histories, grouped heads, an
 empty sequence, padded extents larger than the longest query.  Rows that must not be read hold NaN.
 
-Bound: the probabilities are rounded to fp16 before the second product (relative 2^-11 each, averaging out over the
-keys) and the result once more; 2e-3 of the largest output is several times that."""
+Bound in float16: the probabilities are rounded to fp16 before the second product (relative 2^-11 each, averaging out over the
+keys) and the result once more; 2e-3 of the largest output is several times that.
+In float32: a score of size S has an error of about S 2^-23 (S up to 100 here: sums of 128 products of 2 x 2 standard deviations,
+times log2 e / sqrt(128)), which is the relative error of its probability: 100 x 2^-23 = 1.2e-5, and 2e-5 is the bound."""
 import pytest
 import torch
 
@@ -36,16 +38,17 @@ def reference(q, k, v, lens, hist, out):
     return out
 
 
-@pytest.mark.parametrize("hs", [128, 64])
+@pytest.mark.parametrize("dtype,hs", [(torch.float16, 128), (torch.float16, 64), (torch.float32, 128), (torch.float32, 96),
+                                      (torch.float32, 64)])
 @pytest.mark.parametrize("case", range(len(CASES)))
-def test_attention_matches_float64(isp, hs, case):
+def test_attention_matches_float64(isp, dtype, hs, case):
     lens, hist, heads, kv, max_q, max_seq = CASES[case]
-    print("[case] attention %s hs %d" % (CASES[case], hs), flush=True)
+    print("[case] attention %s %s hs %d" % (CASES[case], dtype, hs), flush=True)
     g = torch.Generator().manual_seed(case)
     batch, tokens = len(lens), sum(lens)
     nan = float("nan")
-    q = torch.full((batch, heads, max_q, hs), nan, dtype=torch.float16)
-    k, v = (torch.full((2, batch, kv, max_seq, hs), nan, dtype=torch.float16) for _ in range(2))
+    q = torch.full((batch, heads, max_q, hs), nan, dtype=dtype)
+    k, v = (torch.full((2, batch, kv, max_seq, hs), nan, dtype=dtype) for _ in range(2))
     for b in range(batch):
         q[b, :, :lens[b]] = 2 * torch.randn(heads, lens[b], hs, generator=g)
         n = lens[b] + hist[b]
@@ -53,9 +56,9 @@ def test_attention_matches_float64(isp, hs, case):
         v[1, b, :, :n] = torch.randn(kv, n, hs, generator=g)
     expect = reference(q, k[1], v[1], lens, hist, torch.zeros(tokens, heads, hs, dtype=torch.float64))
     ints = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")   # noqa: E731
-    out = torch.full((tokens, heads, hs), nan, dtype=torch.float16, device="cuda")
+    out = torch.full((tokens, heads, hs), nan, dtype=dtype, device="cuda")
     context = [a + b for a, b in zip(lens, hist)]
     isp.context_attention(q.cuda(), k.cuda(), v.cuda(), 1, ints(hist), ints(lens), ints(context), max(context), out)
     got = out.cpu().double()
     assert torch.isfinite(got).all()
-    assert (got - expect).abs().max() <= 2e-3 * expect.abs().max()
+    assert (got - expect).abs().max() <= (2e-3 if dtype == torch.float16 else 2e-5) * expect.abs().max()

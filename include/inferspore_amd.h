@@ -268,7 +268,7 @@ int isp_repeat_kv_cache_f16(const void* k_cache, const void* v_cache, void* k_ds
  *   q [batch, head_num, max_q_len, head_size] (rows of padded queries are never read);
  *   k_cache, v_cache [layers, batch, kv_head_num, max_seq_len, head_size] (base pointers; rows from
  *   context_length[b] on are never used); out [token_num, head_num, head_size].
- * head_size 128 or 64, 16-byte aligned pointers, else ISP_ERR_UNSUPPORTED.
+ * head_size 128, 96 or 64, 16-byte aligned pointers, else ISP_ERR_UNSUPPORTED.
  * One kernel for the reference's launchRepeatKVCache, batched q x k^T, launchScaleMaskAndSoftmax,
  * batched p x v and launchTransposeOutRemovePadding (src/kernels/repeat_kv.cu:10-100, linear.cu:67-109,
  * attn_softmax_kernel.cu:50-125, build_casual_mask.cu:5-42; the history is visible here, see
@@ -316,7 +316,7 @@ int isp_linear_f16(const void* a, const void* w, void* out, void* workspace, int
  *   down_weight [inter, hidden]; q, k_cache, v_cache, padding_offset and the lengths as for the entry points above;
  *   context [token_num, head_num * head_size] and act [token_num, inter] are written on the way;
  *   workspace: isp_context_layer_f16_workspace() bytes that no other work in flight uses (0: the shape is unsupported).
- * ISP_ERR_UNSUPPORTED: more rows, head_size other than 64 / 128, hidden or inter not a multiple of 8, hidden > 8192, more
+ * ISP_ERR_UNSUPPORTED: more rows, head_size other than 64 / 96 / 128, hidden or inter not a multiple of 8, hidden > 8192, more
  * than 32768 columns in a product of more than 16 rows, pointers that are not 16-byte aligned.
  */
 size_t isp_context_layer_f16_workspace(int batch, int token_num, int hidden, int head_num, int kv_head_num, int head_size,

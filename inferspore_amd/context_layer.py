@@ -9,7 +9,7 @@ order a model runs them:
     normed, residual                       (packed [tokens, H]; `normed` = RMSNorm(residual) by attn_norm)
     qkv      = normed @ Wqkv                                 library GEMM (out of this library's scope)
     q, cache += k, v = add_fused_qkv_bias_transpose_rope_and_append(qkv)    * this library
-    packed   = context_attention(q, cache)                   * this library (heads of 64, 128 and, in float32, 96 elements; others:
+    packed   = context_attention(q, cache)                   * this library (heads of 64, 96 or 128 elements; others:
                                                                repeat_kv_cache, torch's attention, transpose_out_remove_padding)
     attn_out = packed @ Wo                                   library GEMM
     residual, normed2 = fused_add_bias_residual_rmsnorm(residual, attn_out, ffn_norm)      * this library

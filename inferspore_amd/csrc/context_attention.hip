@@ -531,8 +531,8 @@ __global__ __launch_bounds__(64) void combine_splits_f16(const float* __restrict
 
 // Workgroups that share a (sequence, key head): enough for two on every compute unit, each with at least 128 keys (four
 // steps, one per wavefront).
-int attention_splits(int batch, int head_num, int kv_head_num, int max_q_len, int max_k_len) {
-    if (batch <= 0 || kv_head_num <= 0 || head_num / kv_head_num * (long long)max_q_len > kSlots) return 1;
+static int attention_splits(int batch, int head_num, int kv_head_num, int head_size, int max_q_len, int max_k_len) {
+    if (batch <= 0 || kv_head_num <= 0 || head_size == 96 || head_num / kv_head_num * (long long)max_q_len > kSlots) return 1;
     const long long groups = (long long)batch * kv_head_num, units = resident_waves() / 32;
     long long splits = (2 * units) / groups;
     const long long most = (max_k_len + 4 * kStepKeys - 1) / (4 * kStepKeys);
@@ -541,9 +541,15 @@ int attention_splits(int batch, int head_num, int kv_head_num, int max_q_len, in
 }
 
 size_t attention_workspace(int batch, int head_num, int kv_head_num, int head_size, int max_q_len, int max_k_len) {
-    const int splits = attention_splits(batch, head_num, kv_head_num, max_q_len, max_k_len);
+    const int splits = attention_splits(batch, head_num, kv_head_num, head_size, max_q_len, max_k_len);
     return splits == 1 ? 0 : (size_t)splits * batch * head_num * max_q_len * partial_floats(head_size) * sizeof(float);
 }
+
+// csrc/context_attention_f32.hip: fp16 heads of 96 elements, computed in fp32
+int context_attention_f16_96(const __half* q, const __half* k_cache, const __half* v_cache, __half* out,
+                             const int32_t* history_length, const int32_t* input_length, const int32_t* context_length, int layer,
+                             int batch, int head_num, int kv_head_num, int max_q_len, int max_k_len, int max_seq_len,
+                             int token_num, float scale, hipStream_t stream);
 
 // `workspace` NULL: a sequence's keys are not split.
 int context_attention(const _Float16* q, const _Float16* k_cache, const _Float16* v_cache, _Float16* out,
@@ -553,6 +559,11 @@ int context_attention(const _Float16* q, const _Float16* k_cache, const _Float16
     if (layer < 0 || batch < 0 || head_num <= 0 || kv_head_num <= 0 || head_num % kv_head_num != 0 || max_q_len < 0 ||
         max_k_len < 0 || max_seq_len < 0 || token_num < 0 || !(scale > 0.0f))
         return ISP_ERR_BAD_SHAPE;
+    if (head_size == 96)
+        return context_attention_f16_96(reinterpret_cast<const __half*>(q), reinterpret_cast<const __half*>(k_cache),
+                                        reinterpret_cast<const __half*>(v_cache), reinterpret_cast<__half*>(out), history_length,
+                                        input_length, context_length, layer, batch, head_num, kv_head_num, max_q_len, max_k_len,
+                                        max_seq_len, token_num, scale, stream);
     if (head_size != 128 && head_size != 64) return ISP_ERR_UNSUPPORTED;
     if (batch == 0 || max_q_len == 0 || token_num == 0) return ISP_OK;
     if (max_k_len == 0 || max_seq_len == 0) return ISP_ERR_BAD_SHAPE;
@@ -570,7 +581,7 @@ int context_attention(const _Float16* q, const _Float16* k_cache, const _Float16
     const float scale_log2e = scale * 1.4426950408889634f;
     if ((long long)(head_num / kv_head_num) * max_q_len <= kSlots) {
         if (!aligned16(workspace) || (long long)batch * max_q_len > 65535) return ISP_ERR_UNSUPPORTED;
-        const int splits = workspace ? attention_splits(batch, head_num, kv_head_num, max_q_len, max_k_len) : 1;
+        const int splits = workspace ? attention_splits(batch, head_num, kv_head_num, head_size, max_q_len, max_k_len) : 1;
         const dim3 grid((unsigned)kv_head_num, (unsigned)batch, (unsigned)splits);
 #define ISP_LAUNCH_DECODE(HS, SPLIT)                                                                                          \
     hipLaunchKernelGGL((decode_attention_f16<HS, SPLIT>), grid, dim3(256), 0, stream, q, k_cache + slice, v_cache + slice, out, \

@@ -1,4 +1,5 @@
-// Fused causal attention for fp32 heads of 64, 96 or 128 elements: what context_attention.hip does for fp16, in fp32 throughout
+// Fused causal attention for fp32 heads of 64, 96 or 128 elements, and for fp16 heads of 96 (the tiles of the fp16 kernels want
+// multiples of 64), which are converted when they are loaded: what context_attention.hip does for fp16, in fp32 throughout
 // (v_mfma_f32_16x16x4_f32 multiplies and adds fp32; probabilities and sums stay fp32).  In place of KV broadcast, a mask tensor,
 // torch's attention, two layout copies and the transpose to packed rows.
 //
@@ -12,7 +13,9 @@
 // Bound by the fp32 matrix rate (157 TFLOP/s) for long prompts and by the chain of dependent blocks for short ones.
 // Against those five launches, us: 4 prompts of 100 tokens, 16 heads of 128: 11.0, 46.7; 1000 and 700 tokens, 32 heads over 8 key
 // heads: 225, 887; 8 x 300 tokens on a history of 700, 32 heads: 650, 860; decode, 16 sequences of 1000 keys, 32 heads: 117, 449;
-// 64 of 400, 32 heads of 96 over 8: 34, 343.  Error against 64 bits 1.5e-7 ... 3.7e-7 (2-norm), there 2.1e-7 ... 6.9e-7.
+// 64 of 400, 32 heads of 96 over 8: 34, 343.  fp16 heads of 96: decode, 16 x 1000 keys, 32 heads 47, 140; 64 x 400, 32 over 8
+// 26, 234; 8 prompts of 100 tokens 19, 51; 4 of 1000 291, 352; 4 of 2000 1086, 1164; 12 x 200 on a history of 800, 40 heads 415, 401
+// (16 queries per tile: the keys come from the caches once per tile), the one measured extent where it is not ahead.  Error against 64 bits 1.5e-7 ... 3.7e-7 (2-norm), there 2.1e-7 ... 6.9e-7.
 #include "isp_common.h"
 
 namespace isp {
@@ -36,12 +39,45 @@ __device__ __forceinline__ float rows_sum(float x) {
     return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
+// N elements from a 16-byte aligned address / two at a time, as fp32
+template <int N>
+__device__ __forceinline__ void load_row(const float* p, float* f) {
+#pragma unroll
+    for (int i = 0; i < N; i += 4) Elem<float>::unpack(load16(p + i), f + i);
+}
+template <int N>
+__device__ __forceinline__ void load_row(const __half* p, float* f) {
+#pragma unroll
+    for (int i = 0; i < N; i += 8) Elem<__half>::unpack(load16(p + i), f + i);
+}
+template <int N>
+__device__ __forceinline__ void load_pairs(const float* p, float* f) {
+#pragma unroll
+    for (int i = 0; i < N; i += 2) {
+        const float2 x = *reinterpret_cast<const float2*>(p + i);
+        f[i] = x.x, f[i + 1] = x.y;
+    }
+}
+template <int N>
+__device__ __forceinline__ void load_pairs(const __half* p, float* f) {
+#pragma unroll
+    for (int i = 0; i < N; i += 2) {
+        const float2 x = __half22float2(*reinterpret_cast<const __half2*>(p + i));
+        f[i] = x.x, f[i + 1] = x.y;
+    }
+}
+__device__ __forceinline__ void store4(float* p, float4w x) { *reinterpret_cast<float4w*>(p) = x; }
+__device__ __forceinline__ void store4(__half* p, float4w x) {
+    reinterpret_cast<__half2*>(p)[0] = __floats2half2_rn(x[0], x[1]);
+    reinterpret_cast<__half2*>(p)[1] = __floats2half2_rn(x[2], x[3]);
+}
+
 // GROUPED: the 16 queries are those of a group's heads (grid x = key head), else of 16 tokens of a head (x = head); grid y =
 // sequence, z = tile of queries, the last (longest) first.
-template <int HS, bool GROUPED>
+template <typename T, int HS, bool GROUPED>
 __global__ __launch_bounds__(256) void context_attention_f32(
-    const float* __restrict__ q_buf, const float* __restrict__ k_cache, const float* __restrict__ v_cache,
-    float* __restrict__ out, const int* history_length, const int* input_length, const int* context_length, int head_num,
+    const T* __restrict__ q_buf, const T* __restrict__ k_cache, const T* __restrict__ v_cache, T* __restrict__ out,
+    const int* history_length, const int* input_length, const int* context_length, int head_num,
     int kv_head_num, int max_q_len, int max_k_len, int max_seq_len, int tokens, float scale_log2e) {
     constexpr int kQuarter = HS / 4, kChunk = HS / 16;
     const int tid = threadIdx.x, lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64), j = lane % 16, g = lane / 16;
@@ -60,17 +96,14 @@ __global__ __launch_bounds__(256) void context_attention_f32(
     const int my_head = GROUPED ? kv_head * group + (real ? j % group : 0) : (int)blockIdx.x;
     const int my_visible = real ? min(hist + my_q + 1, ctx) : 0;
     const size_t kv_offset = ((size_t)b * kv_head_num + kv_head) * (size_t)max_seq_len * HS;
-    const float *keys = k_cache + kv_offset, *values = v_cache + kv_offset;
+    const T *keys = k_cache + kv_offset, *values = v_cache + kv_offset;
 
     float qf[kQuarter];
     {
-        const float* q_row = q_buf + (((size_t)b * head_num + my_head) * (size_t)max_q_len + my_q) * HS + kQuarter * g;
+        const T* q_row = q_buf + (((size_t)b * head_num + my_head) * (size_t)max_q_len + my_q) * HS + kQuarter * g;
+        load_row<kQuarter>(q_row, qf);
 #pragma unroll
-        for (int i = 0; i < kQuarter; i += 4) {
-            const float4w x = *reinterpret_cast<const float4w*>(q_row + i);
-#pragma unroll
-            for (int e = 0; e < 4; e++) qf[i + e] = real ? x[e] : 0.0f;
-        }
+        for (int i = 0; i < kQuarter; i++) qf[i] = real ? qf[i] : 0.0f;
     }
     float4w acc[kChunk];
 #pragma unroll
@@ -81,21 +114,12 @@ __global__ __launch_bounds__(256) void context_attention_f32(
     for (int s = wave; s < blocks; s += kWaves) {
         // a key past the visible ones re-reads the last visible row and is masked below
         float kf[kQuarter], vf[4][kChunk];
-        const float* k_row = keys + (size_t)min(s * kBlockKeys + j, wg_visible - 1) * HS + kQuarter * g;
-#pragma unroll
-        for (int i = 0; i < kQuarter; i += 4) {
-            const float4w x = *reinterpret_cast<const float4w*>(k_row + i);
-#pragma unroll
-            for (int e = 0; e < 4; e++) kf[i + e] = x[e];
-        }
+        const T* k_row = keys + (size_t)min(s * kBlockKeys + j, wg_visible - 1) * HS + kQuarter * g;
+        load_row<kQuarter>(k_row, kf);
 #pragma unroll
         for (int r = 0; r < 4; r++) {
-            const float* v_row = values + (size_t)min(s * kBlockKeys + 4 * g + r, wg_visible - 1) * HS + kChunk * j;
-#pragma unroll
-            for (int c = 0; c < kChunk; c += 2) {
-                const float2 x = *reinterpret_cast<const float2*>(v_row + c);
-                vf[r][c] = x.x, vf[r][c + 1] = x.y;
-            }
+            const T* v_row = values + (size_t)min(s * kBlockKeys + 4 * g + r, wg_visible - 1) * HS + kChunk * j;
+            load_pairs<kChunk>(v_row, vf[r]);
         }
         // two chains of products, so that one does not wait for the other's result
         float4w even = {0.0f, 0.0f, 0.0f, 0.0f}, odd = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -166,20 +190,21 @@ __global__ __launch_bounds__(256) void context_attention_f32(
         const int head = GROUPED ? kv_head * group + slot % group : (int)blockIdx.x;
         const long long token = (long long)first_token + (GROUPED ? slot / group : q0 + slot);
         if (token < tokens)
-            *reinterpret_cast<float4w*>(out + ((size_t)token * head_num + head) * HS + d) = o * (l > 0.0f ? 1.0f / l : 0.0f);
+            store4(out + ((size_t)token * head_num + head) * HS + d, o * (l > 0.0f ? 1.0f / l : 0.0f));
     }
 }
 
 }  // namespace
 
-static int attention_f32(const float* q, const float* k_cache, const float* v_cache, float* out, const int32_t* history_length,
+template <typename T>
+static int attention_f32(const T* q, const T* k_cache, const T* v_cache, T* out, const int32_t* history_length,
                          const int32_t* input_length, const int32_t* context_length, int layer, int batch, int head_num,
                          int kv_head_num, int head_size, int max_q_len, int max_k_len, int max_seq_len, int token_num, float scale,
                          hipStream_t stream) {
     if (layer < 0 || batch < 0 || head_num <= 0 || kv_head_num <= 0 || head_num % kv_head_num != 0 || max_q_len < 0 ||
         max_k_len < 0 || max_seq_len < 0 || token_num < 0 || !(scale > 0.0f))
         return ISP_ERR_BAD_SHAPE;
-    if (head_size != 128 && head_size != 96 && head_size != 64) return ISP_ERR_UNSUPPORTED;
+    if (head_size != 96 && (sizeof(T) == 2 || (head_size != 128 && head_size != 64))) return ISP_ERR_UNSUPPORTED;
     if (batch == 0 || max_q_len == 0 || token_num == 0) return ISP_OK;
     if (max_k_len == 0 || max_seq_len == 0) return ISP_ERR_BAD_SHAPE;
     const bool grouped = (long long)(head_num / kv_head_num) * max_q_len <= kSlots;
@@ -196,7 +221,7 @@ static int attention_f32(const float* q, const float* k_cache, const float* v_ca
     const size_t slice = (size_t)layer * batch * kv_head_num * max_seq_len * head_size;
     const dim3 grid((unsigned)(grouped ? kv_head_num : head_num), (unsigned)batch, (unsigned)tiles);
 #define ISP_LAUNCH_F32(HS, GROUPED)                                                                                          \
-    hipLaunchKernelGGL((context_attention_f32<HS, GROUPED>), grid, dim3(256), 0, stream, q, k_cache + slice, v_cache + slice, out, \
+    hipLaunchKernelGGL((context_attention_f32<T, HS, GROUPED>), grid, dim3(256), 0, stream, q, k_cache + slice, v_cache + slice, out, \
                        history_length, input_length, context_length, head_num, kv_head_num, max_q_len, max_k_len,            \
                        max_seq_len, token_num, scale * 1.4426950408889634f)
 #define ISP_LAUNCH_F32_HS(HS)               \
@@ -204,12 +229,24 @@ static int attention_f32(const float* q, const float* k_cache, const float* v_ca
         if (grouped) ISP_LAUNCH_F32(HS, true); \
         else ISP_LAUNCH_F32(HS, false);     \
     } while (0)
-    if (head_size == 128) ISP_LAUNCH_F32_HS(128);
-    else if (head_size == 96) ISP_LAUNCH_F32_HS(96);
-    else ISP_LAUNCH_F32_HS(64);
+    if constexpr (sizeof(T) == 2) {
+        ISP_LAUNCH_F32_HS(96);
+    } else {
+        if (head_size == 128) ISP_LAUNCH_F32_HS(128);
+        else if (head_size == 96) ISP_LAUNCH_F32_HS(96);
+        else ISP_LAUNCH_F32_HS(64);
+    }
 #undef ISP_LAUNCH_F32_HS
 #undef ISP_LAUNCH_F32
     return note_launch(hipGetLastError());
+}
+
+int context_attention_f16_96(const __half* q, const __half* k_cache, const __half* v_cache, __half* out,
+                             const int32_t* history_length, const int32_t* input_length, const int32_t* context_length, int layer,
+                             int batch, int head_num, int kv_head_num, int max_q_len, int max_k_len, int max_seq_len,
+                             int token_num, float scale, hipStream_t stream) {
+    return attention_f32<__half>(q, k_cache, v_cache, out, history_length, input_length, context_length, layer, batch, head_num,
+                                 kv_head_num, 96, max_q_len, max_k_len, max_seq_len, token_num, scale, stream);
 }
 
 }  // namespace isp
@@ -219,7 +256,7 @@ extern "C" int isp_context_attention_f32(const void* q, const void* k_cache, con
                                          const int32_t* context_length, int layer, int batch, int head_num,
                                          int kv_head_num, int head_size, int max_q_len, int max_k_len, int max_seq_len,
                                          int token_num, float scale, isp_stream_t stream) {
-    return isp::attention_f32(static_cast<const float*>(q), static_cast<const float*>(k_cache),
+    return isp::attention_f32<float>(static_cast<const float*>(q), static_cast<const float*>(k_cache),
                               static_cast<const float*>(v_cache), static_cast<float*>(out), history_length, input_length,
                               context_length, layer, batch, head_num, kv_head_num, head_size, max_q_len, max_k_len,
                               max_seq_len, token_num, scale, static_cast<hipStream_t>(stream));

@@ -38,7 +38,7 @@ static int layer_shape(int layer, int batch, int tokens, int hidden, int head_nu
         max_q_len <= 0 || max_k_len <= 0 || max_seq_len <= 0 || inter <= 0 || rotary_dim < 0 || head_num % kv_head_num != 0 ||
         rotary_dim % 2 != 0 || rotary_dim > head_size)
         return ISP_ERR_BAD_SHAPE;
-    if (tokens > kSkinnyMaxRows || (head_size != 64 && head_size != 128) || hidden % 8 != 0 || hidden > kNormSumsMaxHidden ||
+    if (tokens > kSkinnyMaxRows || (head_size != 64 && head_size != 96 && head_size != 128) || hidden % 8 != 0 || hidden > kNormSumsMaxHidden ||
         inter % 8 != 0 || batch > 65535 || (long long)batch * max_q_len > 0x7fffffffll ||
         ((long long)head_num + 2ll * kv_head_num) * head_size > (1 << 24) || inter > (1 << 24))
         return ISP_ERR_UNSUPPORTED;

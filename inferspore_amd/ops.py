@@ -296,7 +296,7 @@ def linear(x, w):
 
 def context_attention_supports(dtype, head_size):
     """Whether context_attention takes heads of this type and size."""
-    return head_size in ((64, 128) if dtype == torch.float16 else (64, 96, 128) if dtype == torch.float32 else ())
+    return head_size in (64, 96, 128) and dtype in (torch.float16, torch.float32)
 
 
 def context_attention(q_buf, k_cache, v_cache, layer_id, history_length, input_length, context_length, max_k_len, out,
@@ -312,7 +312,7 @@ def context_attention(q_buf, k_cache, v_cache, layer_id, history_length, input_l
     kv_head_num, max_seq_len = k_cache.shape[2], k_cache.shape[3]
     _expect(k_cache.shape == v_cache.shape and k_cache.shape[1] == batch and k_cache.shape[4] == head_size,
             "caches must be [layers, batch, kv_head_num, max_seq_len, head_size]")
-    _expect(context_attention_supports(q_buf.dtype, head_size), "attention takes float16 heads of 64 or 128 elements, float32 heads of 64, 96 or 128")
+    _expect(context_attention_supports(q_buf.dtype, head_size), "attention takes float16 or float32 heads of 64, 96 or 128 elements")
     _expect(kv_head_num > 0 and head_num % kv_head_num == 0, "head_num must be a multiple of kv_head_num")
     _expect(out.shape[1:] == (head_num, head_size), "out must be [tokens, heads, head_size]")
     _expect(0 <= int(layer_id) < k_cache.shape[0], "layer_id outside the cache")

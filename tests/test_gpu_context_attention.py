@@ -38,7 +38,7 @@ def reference(q, k, v, lens, hist, out):
     return out
 
 
-@pytest.mark.parametrize("dtype,hs", [(torch.float16, 128), (torch.float16, 64), (torch.float32, 128), (torch.float32, 96),
+@pytest.mark.parametrize("dtype,hs", [(torch.float16, 128), (torch.float16, 96), (torch.float16, 64), (torch.float32, 128), (torch.float32, 96),
                                       (torch.float32, 64)])
 @pytest.mark.parametrize("case", range(len(CASES)))
 def test_attention_matches_float64(isp, dtype, hs, case):

@@ -13,6 +13,7 @@ CASES = [([1], [0], 2, 2, 64, 264, 1, 8, 64, False, 128),
          ([5, 3], [0, 0], 2, 1, 128, 520, 5, 16, 128, True, 256),
          ([1] * 16, list(range(0, 160, 10)), 8, 2, 128, 1040, 1, 256, 96, False, 1024),
          ([7, 0, 20], [3, 9, 0], 4, 4, 64, 1000, 24, 32, 64, True, 264),
+         ([1, 4], [50, 0], 6, 3, 96, 392, 4, 64, 96, True, 576),
          ([64], [0], 12, 3, 128, 88, 64, 64, 128, False, 1536),
          ([1, 1, 1], [30, 31, 40], 16, 16, 64, 2816, 1, 32, 0, True, 1024),   # the last two sequences' rows are past the cache
          ([2, 2], [100, 7], 64, 8, 128, 4096, 2, 128, 128, False, 8192)]

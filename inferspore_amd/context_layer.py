@@ -18,7 +18,8 @@ order a model runs them:
     residual, normed_next = fused_add_bias_residual_rmsnorm(residual, ffn_out, next attn_norm)   * this library
 
 Dense contractions of more than 64 rows are left to torch's library calls (hipBLASLt GEMMs), those of fewer float16 rows go to
-ops.linear, and a layer of such rows is one call of the C ABI (isp_context_layer_f16); everything marked * goes through the C ABI.  All work is issued on torch's current stream.
+ops.linear, and a layer of such rows is one call of the C ABI (isp_context_layer_f16); everything marked * goes through the
+C ABI.  All work is issued on torch's current stream.
 """
 import math
 

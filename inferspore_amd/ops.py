@@ -283,8 +283,8 @@ def linear_supports(x, w):
 
 def linear(x, w):
     """x [rows, k] @ w [k, n] for up to 64 float16 rows, float32 accumulation."""
-    _expect(linear_supports(x, w), "linear takes up to 64 (above 32768 columns: 16) contiguous float16 rows and a contiguous weight [k, n], "
-            "extents in multiples of 8")
+    _expect(linear_supports(x, w), "linear takes up to 64 (above 32768 columns: 16) contiguous float16 rows and a contiguous "
+            "weight [k, n], extents in multiples of 8")
     m, k = x.shape
     n = w.shape[1]
     out = torch.empty((m, n), dtype=x.dtype, device=x.device)

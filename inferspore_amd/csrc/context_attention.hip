@@ -351,7 +351,7 @@ __global__ __launch_bounds__(256, 2) void decode_attention_f16(
         half8 k[2][kDSteps];
         uint32_t v[8][kWords];
     } buf[2];
-    auto load = [&](int which, int s) {  // a key past the visible ones re-reads the last visible row: masked below
+    auto load = [&](int which, int s) {  // a key past the visible ones re-reads the last visible row: masked (blanked) below
         Step& t = buf[which];
 #pragma unroll
         for (int blk = 0; blk < 2; blk++) {
@@ -420,11 +420,23 @@ __global__ __launch_bounds__(256, 2) void decode_attention_f16(
             acc[c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vt.h, p, acc[c], 0, 0, 0);
         }
     };
+    // the only step with keys past the visible ones is the last of all, which its wavefront takes last: their value rows count as
+    // zero (0 x inf is NaN)
+    auto blank = [&](int which, int s) {
+        if ((s + 1) * kStepKeys <= wg_visible) return;  // wavefront-uniform
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            const uint32_t keep = s * kStepKeys + 16 * (i / 4) + 4 * g + i % 4 < wg_visible ? 0xffffffffu : 0u;
+#pragma unroll
+            for (int w = 0; w < kWords; w++) buf[which].v[i][w] &= keep;
+        }
+    };
     int s = first + wave;
     if (s < last) {
         load(0, s);
         for (;;) {
             if (s + kWaves >= last) {
+                blank(0, s);
                 compute(0, s);
                 break;
             }
@@ -432,6 +444,7 @@ __global__ __launch_bounds__(256, 2) void decode_attention_f16(
             compute(0, s);
             s += kWaves;
             if (s + kWaves >= last) {
+                blank(1, s);
                 compute(1, s);
                 break;
             }

@@ -16,6 +16,8 @@
 // 64 of 400, 32 heads of 96 over 8: 34, 343.  fp16 heads of 96: decode, 16 x 1000 keys, 32 heads 47, 140; 64 x 400, 32 over 8
 // 26, 234; 8 prompts of 100 tokens 19, 51; 4 of 1000 291, 352; 4 of 2000 1086, 1164; 12 x 200 on a history of 800, 40 heads 415, 401
 // (16 queries per tile: the keys come from the caches once per tile), the one measured extent where it is not ahead.  Error against 64 bits 1.5e-7 ... 3.7e-7 (2-norm), there 2.1e-7 ... 6.9e-7.
+#include <type_traits>
+
 #include "isp_common.h"
 
 namespace isp {
@@ -110,9 +112,8 @@ __global__ __launch_bounds__(256) void context_attention_f32(
     for (int c = 0; c < kChunk; c++) acc[c] = float4w{0.0f, 0.0f, 0.0f, 0.0f};
     float run_max = -INFINITY, run_sum = 0.0f;  // run_sum: this lane's keys only
 
-    const int blocks = (wg_visible + kBlockKeys - 1) / kBlockKeys;
-    for (int s = wave; s < blocks; s += kWaves) {
-        // a key past the visible ones re-reads the last visible row and is masked below
+    const auto block = [&](int s, auto tail) {
+        // a key past the visible ones (in a tail only) re-reads the last visible row: its score is masked, its value counts as zero
         float kf[kQuarter], vf[4][kChunk];
         const T* k_row = keys + (size_t)min(s * kBlockKeys + j, wg_visible - 1) * HS + kQuarter * g;
         load_row<kQuarter>(k_row, kf);
@@ -149,10 +150,17 @@ __global__ __launch_bounds__(256) void context_attention_f32(
             for (int c = 0; c < kChunk; c++) acc[c] *= rescale;
         }
 #pragma unroll
-        for (int r = 0; r < 4; r++)
+        for (int r = 0; r < 4; r++) {
+            const bool exists = !decltype(tail)::value || s * kBlockKeys + 4 * g + r < wg_visible;  // 0 x inf is NaN
 #pragma unroll
-            for (int c = 0; c < kChunk; c++) acc[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[r][c], p[r], acc[c], 0, 0, 0);
-    }
+            for (int c = 0; c < kChunk; c++)
+                acc[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(exists ? vf[r][c] : 0.0f, p[r], acc[c], 0, 0, 0);
+        }
+    };
+    const int whole = wg_visible / kBlockKeys, blocks = (wg_visible + kBlockKeys - 1) / kBlockKeys;
+    int s = wave;
+    for (; s < whole; s += kWaves) block(s, std::false_type{});
+    if (s < blocks) block(s, std::true_type{});
 
     // O^T row 4 g + r of product c is d = kChunk (4 g + r) + c
     __shared__ __align__(16) float o_lds[kWaves][kSlots][HS];

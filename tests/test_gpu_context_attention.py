@@ -62,3 +62,28 @@ def test_attention_matches_float64(isp, dtype, hs, case):
     got = out.cpu().double()
     assert torch.isfinite(got).all()
     assert (got - expect).abs().max() <= (2e-3 if dtype == torch.float16 else 2e-5) * expect.abs().max()
+
+
+@pytest.mark.parametrize("dtype,hs", [(torch.float16, 128), (torch.float16, 96), (torch.float16, 64), (torch.float32, 128),
+                                      (torch.float32, 96), (torch.float32, 64)])
+@pytest.mark.parametrize("lens,hist", [([1, 1, 1], [40, 100, 2]), ([20, 5], [0, 13])])
+def test_an_infinite_value_reaches_only_its_own_sum(isp, dtype, hs, lens, hist):
+    """An infinite element of a sequence's last visible value row, where no block of keys ends: the queries that see it get
+    infinity in that element (not NaN: the rest of the block counts as nothing), and no other element is touched."""
+    print("[case] infinite value %s hs %d %s" % (dtype, hs, lens), flush=True)
+    g = torch.Generator().manual_seed(hs)
+    batch, heads, max_seq = len(lens), 4, 128
+    q = torch.randn(batch, heads, max(lens), hs, generator=g).to(dtype)
+    k, v = (torch.randn(1, batch, 2, max_seq, hs, generator=g).to(dtype) for _ in range(2))
+    context = [a + b for a, b in zip(lens, hist)]
+    expect = reference(q, k[0], v[0], lens, hist, torch.zeros(sum(lens), heads, hs, dtype=torch.float64))
+    for b in range(batch):
+        v[0, b, :, context[b] - 1, 5] = float("inf")
+    ints = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")   # noqa: E731
+    out = torch.zeros(sum(lens), heads, hs, dtype=dtype, device="cuda")
+    isp.context_attention(q.cuda(), k.cuda(), v.cuda(), 0, ints(hist), ints(lens), ints(context), max(context), out)
+    got = out.cpu().double()
+    last = torch.tensor(lens).cumsum(0) - 1
+    assert (got[last, :, 5] == float("inf")).all()
+    others = torch.arange(hs) != 5
+    assert (got - expect)[:, :, others].abs().max() <= (2e-3 if dtype == torch.float16 else 2e-5) * expect.abs().max()

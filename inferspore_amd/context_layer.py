@@ -28,6 +28,7 @@ import torch
 from . import capi, ops
 
 _PLAIN = (torch.Tensor, torch.nn.Parameter)
+_PADDED = frozenset(("mask", "k_all", "v_all"))
 
 
 class LayerWeights:
@@ -71,18 +72,26 @@ class BatchState:
         self.packed_ctx = z(self.tokens, head_num, head_size)
         self.act = z(self.tokens, inter)
 
+        self._attended = None   # the layer whose attention ran last without the buffers below
         if not ops.context_attention_supports(dtype, head_size):
             self._padded_buffers()
 
     def _padded_buffers(self):
-        """What the padded form of the attention (repeat, mask, transpose) works on."""
+        """What the padded form of the attention (repeat, mask, transpose) works on; what a program has set itself stays."""
         shape = (self.batch, self.head_num, self.max_k_len, self.head_size)
-        self.k_all, self.v_all = (torch.zeros(shape, dtype=self.q.dtype, device=self.q.device) for _ in range(2))
-        self.mask = self._build_mask()
+        missing = [name for name in ("k_all", "v_all") if name not in self.__dict__]
+        for name in missing:
+            self.__dict__[name] = torch.zeros(shape, dtype=self.q.dtype, device=self.q.device)
+        if missing and self._attended is not None:
+            ops.repeat_kv_cache(self.k_cache, self.v_cache, self.context, self._attended, self.k_all, self.v_all)
+        if "mask" not in self.__dict__:
+            self.mask = self._build_mask()
 
     def __getattr__(self, name):
-        # the fused attention needs none of them: there they are built when a program first asks
-        if name not in ("mask", "k_all", "v_all") or "act" not in self.__dict__:
+        # The fused attention needs none of them: they are built when a program first asks, k_all and v_all with the broadcast of
+        # the layer that ran last.  From then on (or from when a program sets one) the layers take the padded form, so that an
+        # edited mask counts and k_all, v_all hold what a layer attended to.
+        if name not in _PADDED or "act" not in self.__dict__:
             raise AttributeError(name)
         self._padded_buffers()
         return self.__dict__[name]
@@ -100,6 +109,13 @@ class BatchState:
         # fully padded query rows would be all -inf: let them see key 0 (their output is discarded)
         mask[:, :, :, 0].masked_fill_(~(s[:, :, 0] < self.lengths[:, None])[:, None], 0.0)
         return mask
+
+
+def _fused_attention(st):
+    """Whether a layer's attention is the fused kernel's: not where a program has set or asked for the padded form's mask or buffers."""
+    if not ops.context_attention_supports(st.q.dtype, st.head_size) or hasattr(type(st), "mask"):
+        return False
+    return _PADDED.isdisjoint(st.__dict__) if isinstance(st, BatchState) else not hasattr(st, "mask")
 
 
 def _layer_in_one_call(normed, residual, w, st, layer_id, gamma, rotary_dim, rotary_base, eps):
@@ -130,6 +146,8 @@ def _layer_in_one_call(normed, residual, w, st, layer_id, gamma, rotary_dim, rot
     if not (st.tokens == tokens and 0 <= int(layer_id) < st.k_cache.shape[0] and
             0 <= int(rotary_dim) <= hs and int(rotary_dim) % 2 == 0) or normed.data_ptr() == residual.data_ptr():
         return None
+    if not _fused_attention(st):
+        return None
     lib = capi.lib()
     need = lib.isp_context_layer_f16_workspace(batch, tokens, hidden, heads, kv, hs, st.max_q_len, st.max_k_len, max_seq, inter)
     if need == 0:
@@ -143,6 +161,8 @@ def _layer_in_one_call(normed, residual, w, st, layer_id, gamma, rotary_dim, rot
         p(st.padding_offset), p(st.history), p(st.lengths), p(st.context), p(workspace), int(layer_id), batch, tokens, hidden,
         heads, kv, hs, st.max_q_len, st.max_k_len, max_seq, inter, int(rotary_dim), float(rotary_base), float(eps),
         ops._stream()), "isp_context_layer")
+    if isinstance(st, BatchState):
+        st._attended = int(layer_id)
     return out
 
 
@@ -164,9 +184,11 @@ def context_decoder_layer(normed, residual, w, state, layer_id, next_norm_gamma,
     ops.add_fused_qkv_bias_transpose_rope_and_append(st.q, None, None, st.k_cache, st.v_cache, layer_id, qkv,
                                                      w.qkv_bias, st.padding_offset, st.history, st.lengths,
                                                      rotary_dim, rotary_base)
-    if ops.context_attention_supports(st.q.dtype, st.head_size):
+    if _fused_attention(st):
         ops.context_attention(st.q, st.k_cache, st.v_cache, layer_id, st.history, st.lengths, st.context, st.max_k_len,
                               st.packed_ctx)
+        if isinstance(st, BatchState):
+            st._attended = int(layer_id)
     else:
         ops.repeat_kv_cache(st.k_cache, st.v_cache, st.context, layer_id, st.k_all, st.v_all)
         ctx = torch.nn.functional.scaled_dot_product_attention(st.q, st.k_all, st.v_all, attn_mask=st.mask,

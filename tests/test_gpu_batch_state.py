@@ -1,0 +1,87 @@
+"""What a program does to a BatchState is what its layers see: an edited or replaced mask counts, and k_all / v_all hold the
+broadcast of the layer that ran last, whichever form of the attention the layer would take by itself.
+
+Bound of the attention: as in test_gpu_context_attention (float16 2e-3, float32 2e-5 of the largest output)."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+HEADS, KV, HS, INTER, HIDDEN = 4, 2, 64, 128, 256
+LENS = {"few": [7, 4], "many": [50, 33]}   # up to 64 rows: a layer of float16 rows is one call
+
+
+def layers(edit, dtype, rows, count=1):
+    from inferspore_amd import context_layer as cl
+    lens = LENS[rows]
+    g = torch.Generator(device="cuda").manual_seed(4)
+    st = cl.BatchState(lens, max(lens), HEADS, KV, HS, INTER, 64, 2, dtype)
+    x = torch.randn(sum(lens), HIDDEN, device="cuda", generator=g).to(dtype)
+    edit(st)
+    for layer in range(count):
+        w = cl.LayerWeights(HIDDEN, INTER, dtype, generator=g)
+        w.qkv = w.qkv[:, :(HEADS + 2 * KV) * HS].contiguous()
+        cl.context_decoder_layer(x, x.clone(), w, st, layer, w.attn_norm, rotary_dim=HS)
+    return st, lens
+
+
+def attention64(st, lens, hidden_key):
+    """Packed attention of layer 0 from the state's queries and caches; queries past 0 do not see `hidden_key` (None: see all)."""
+    rows = []
+    for b, n in enumerate(lens):
+        k, v = (c[0, b, :, :n].double().repeat_interleave(HEADS // KV, 0) for c in (st.k_cache, st.v_cache))
+        s = (st.q[b, :, :n].double()[:, :, None] * k[:, None]).sum(-1) * HS ** -0.5
+        i = torch.arange(n, device="cuda")
+        s.masked_fill_(i[None] > i[:, None], float("-inf"))
+        if hidden_key is not None:
+            s[:, 1:, hidden_key] = float("-inf")
+        rows.append((torch.softmax(s, -1)[..., None] * v[:, None]).sum(2).transpose(0, 1))
+    return torch.cat(rows)
+
+
+@pytest.mark.parametrize("rows", ["few", "many"])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("how", ["edited", "replaced"])
+def test_the_states_mask_counts(isp, dtype, rows, how):
+    def edit(st):
+        mask = st.mask if how == "edited" else st._build_mask()
+        mask[:, :, 1:, 0] = float("-inf")
+        for b, n in enumerate(LENS[rows]):
+            mask[b, :, n:, 0] = 0.0   # padded queries see something; their output is dropped
+        if how == "replaced":
+            st.mask = mask
+
+    st, lens = layers(edit, dtype, rows)
+    expect = attention64(st, lens, 0)
+    bound = (2e-3 if dtype == torch.float16 else 2e-5) * expect.abs().max()
+    assert (st.packed_ctx.double() - expect).abs().max() <= bound
+    assert (attention64(st, lens, None) - expect).abs().max() > 10 * bound   # the mask makes a difference
+
+
+@pytest.mark.parametrize("rows", ["few", "many"])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("asked", ["before", "after"])
+def test_k_all_holds_what_the_last_layer_attended_to(isp, dtype, rows, asked):
+    st, lens = layers(lambda st: st.k_all if asked == "before" else None, dtype, rows, count=2)
+    for got, cache in ((st.k_all, st.k_cache), (st.v_all, st.v_cache)):
+        for b, n in enumerate(lens):
+            assert torch.equal(got[b, :, :n], cache[1, b, :, :n].repeat_interleave(HEADS // KV, 0))
+            assert not got[b, :, n:].any()
+    assert (st.packed_ctx.double() - attention_of_layer_1(st, lens)).abs().max() <= 2e-3 * st.packed_ctx.abs().max()
+
+
+def attention_of_layer_1(st, lens):
+    from types import SimpleNamespace
+    return attention64(SimpleNamespace(q=st.q, k_cache=st.k_cache[1:], v_cache=st.v_cache[1:]), lens, None)
+
+
+def test_a_state_that_keeps_its_own_buffers_is_not_rebuilt(isp):
+    """A copy keeps what was set, and an attribute that never existed is still an error."""
+    import copy
+    from inferspore_amd import context_layer as cl
+    st = cl.BatchState([3], 3, HEADS, KV, HS, INTER, 8, 1, torch.float16)
+    own = torch.full((1, 1, 3, 3), -1.0, dtype=torch.float16, device="cuda")
+    st.mask = own
+    assert st.k_all.shape == (1, HEADS, 3, HS) and st.mask is own and copy.copy(st).mask is own
+    with pytest.raises(AttributeError):
+        st.masks

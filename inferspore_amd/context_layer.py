@@ -112,8 +112,9 @@ class BatchState:
 
 
 def _fused_attention(st):
-    """Whether a layer's attention is the fused kernel's: not where a program has set or asked for the padded form's mask or buffers."""
-    if not ops.context_attention_supports(st.q.dtype, st.head_size) or hasattr(type(st), "mask"):
+    """Whether a layer's attention is the fused kernel's: not where that does not take the state's buffers (an unaligned view in a
+    program's own cache, say), nor where a program has set or asked for the padded form's mask or buffers."""
+    if not ops.context_attention_takes(st.q, st.k_cache, st.v_cache, st.packed_ctx) or hasattr(type(st), "mask"):
         return False
     return _PADDED.isdisjoint(st.__dict__) if isinstance(st, BatchState) else not hasattr(st, "mask")
 

@@ -299,6 +299,17 @@ def context_attention_supports(dtype, head_size):
     return head_size in (64, 96, 128) and dtype in (torch.float16, torch.float32)
 
 
+def context_attention_takes(q_buf, k_cache, v_cache, out):
+    """Whether context_attention takes these operands: heads that it supports, extents that its grids hold, 16-byte aligned buffers,
+    and an output that does not lie in the queries' memory (workgroups still read queries while others write)."""
+    if not context_attention_supports(q_buf.dtype, q_buf.shape[-1]) or q_buf.shape[0] > 65535 or q_buf.shape[2] > 65535 * 16:
+        return False
+    q, o = q_buf.data_ptr(), out.data_ptr()
+    if (q | o | k_cache.data_ptr() | v_cache.data_ptr()) % 16:
+        return False
+    return o >= q + q_buf.numel() * q_buf.element_size() or q >= o + out.numel() * out.element_size()
+
+
 def context_attention(q_buf, k_cache, v_cache, layer_id, history_length, input_length, context_length, max_k_len, out,
                       scale=None):
     """Causal attention over the KV cache (history included), to packed rows: q_buf [batch, heads, max_q_len, hs], caches

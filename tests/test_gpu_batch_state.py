@@ -85,3 +85,38 @@ def test_a_state_that_keeps_its_own_buffers_is_not_rebuilt(isp):
     assert st.k_all.shape == (1, HEADS, 3, HS) and st.mask is own and copy.copy(st).mask is own
     with pytest.raises(AttributeError):
         st.masks
+
+
+def shifted(t):
+    """The same extents one element past an aligned address."""
+    flat = torch.zeros(t.numel() + 8, dtype=t.dtype, device="cuda")
+    return flat[1:1 + t.numel()].view(t.shape)
+
+
+@pytest.mark.parametrize("rows", ["few", "many"])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("name", ["q", "k_cache", "v_cache", "packed_ctx", "packed_ctx in q"])
+def test_a_programs_own_unaligned_buffers(isp, dtype, rows, name):
+    def edit(st):
+        if name == "packed_ctx in q":
+            st.packed_ctx = st.q.view(-1)[:st.packed_ctx.numel()].view(st.packed_ctx.shape)
+        else:
+            setattr(st, name, shifted(getattr(st, name)))
+
+    st, lens = layers(edit, dtype, rows)
+    if name == "packed_ctx in q":   # the queries are gone: against the run with buffers of their own
+        expect = layers(lambda st: st.mask, dtype, rows)[0].packed_ctx.double()
+    else:
+        expect = attention64(st, lens, None)
+    assert (st.packed_ctx.double() - expect).abs().max() <= (2e-3 if dtype == torch.float16 else 2e-5) * expect.abs().max()
+
+
+def test_more_sequences_than_a_grid_holds(isp):
+    """65536 sequences of one token: the padded form, as ever."""
+    from inferspore_amd import context_layer as cl
+    n = 65536
+    st = cl.BatchState([1] * n, 1, 1, 1, 64, 16, 1, 1, torch.float16)
+    w = cl.LayerWeights(64, 16, torch.float16)
+    x = torch.randn(n, 64, device="cuda").half()
+    cl.context_decoder_layer(x, x.clone(), w, st, 0, w.attn_norm, rotary_dim=64)
+    assert torch.equal(st.packed_ctx[:, 0], st.v_cache[0, :, 0, 0])   # one key: its value

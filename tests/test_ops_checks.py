@@ -113,3 +113,24 @@ def test_mover_checks():
         ops.rope_decode_and_append(t(2, 8, 8), None, t(1, 2, 3, 16, 8), t(1, 2, 3, 16, 8), 0, lens, 5, 4, 8, 10000.0)
     with pytest.raises(RuntimeError, match="GPU"):
         ops.rope_decode_and_append(t(2, 8, 8), None, t(1, 2, 2, 16, 8), t(1, 2, 2, 16, 8), 0, lens, 5, 4, 8, 10000.0)
+
+
+def test_attention_takes_what_its_kernels_can():
+    """A layer asks before it leaves the padded form: types, sizes, grid limits, alignment, an output inside the queries."""
+    def takes(batch=2, q_len=3, hs=64, dtype=H, shift=None, out=None):
+        def buf(name, *shape):
+            n = 1
+            for d in shape:
+                n *= d
+            flat = torch.empty(n + 8, dtype=dtype)
+            at = int(name == shift)
+            return flat[at:at + n].view(shape)
+        q = buf("q", batch, 2, q_len, hs)
+        return ops.context_attention_takes(q, buf("k", 1, batch, 1, 4, hs), buf("v", 1, batch, 1, 4, hs),
+                                           buf("out", 2, 2, hs) if out is None else out(q))
+    assert takes() and takes(hs=96) and takes(hs=128, dtype=torch.float32)
+    assert not takes(hs=80) and not takes(dtype=torch.bfloat16)
+    assert takes(batch=65535, q_len=1) and not takes(batch=65536, q_len=1)
+    assert takes(batch=1, q_len=65535 * 16) and not takes(batch=1, q_len=65535 * 16 + 1)
+    assert not any(takes(shift=s) for s in ("q", "k", "v", "out"))
+    assert not takes(out=lambda q: q.view(-1)[:256].view(2, 2, 64)) and not takes(out=lambda q: q.view(-1)[512:768].view(2, 2, 64))

@@ -543,9 +543,11 @@ __global__ __launch_bounds__(64) void combine_splits_f16(const float* __restrict
 }  // namespace
 
 // Workgroups that share a (sequence, key head): enough for two on every compute unit, each with at least 128 keys (four
-// steps, one per wavefront).
+// steps, one per wavefront).  One where the second kernel's grid, with a row per sequence and query, would not hold them.
 static int attention_splits(int batch, int head_num, int kv_head_num, int head_size, int max_q_len, int max_k_len) {
-    if (batch <= 0 || kv_head_num <= 0 || head_size == 96 || head_num / kv_head_num * (long long)max_q_len > kSlots) return 1;
+    if (batch <= 0 || kv_head_num <= 0 || head_size == 96 || head_num / kv_head_num * (long long)max_q_len > kSlots ||
+        (long long)batch * max_q_len > 65535)
+        return 1;
     const long long groups = (long long)batch * kv_head_num, units = resident_waves() / 32;
     long long splits = (2 * units) / groups;
     const long long most = (max_k_len + 4 * kStepKeys - 1) / (4 * kStepKeys);
@@ -593,7 +595,7 @@ int context_attention(const _Float16* q, const _Float16* k_cache, const _Float16
     const size_t slice = (size_t)layer * batch * kv_head_num * max_seq_len * head_size;
     const float scale_log2e = scale * 1.4426950408889634f;
     if ((long long)(head_num / kv_head_num) * max_q_len <= kSlots) {
-        if (!aligned16(workspace) || (long long)batch * max_q_len > 65535) return ISP_ERR_UNSUPPORTED;
+        if (!aligned16(workspace)) return ISP_ERR_UNSUPPORTED;
         const int splits = workspace ? attention_splits(batch, head_num, kv_head_num, head_size, max_q_len, max_k_len) : 1;
         const dim3 grid((unsigned)kv_head_num, (unsigned)batch, (unsigned)splits);
 #define ISP_LAUNCH_DECODE(HS, SPLIT)                                                                                          \

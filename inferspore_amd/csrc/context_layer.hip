@@ -39,7 +39,7 @@ static int layer_shape(int layer, int batch, int tokens, int hidden, int head_nu
         rotary_dim % 2 != 0 || rotary_dim > head_size)
         return ISP_ERR_BAD_SHAPE;
     if (tokens > kSkinnyMaxRows || (head_size != 64 && head_size != 96 && head_size != 128) || hidden % 8 != 0 || hidden > kNormSumsMaxHidden ||
-        inter % 8 != 0 || batch > 65535 || (long long)batch * max_q_len > 0x7fffffffll ||
+        inter % 8 != 0 || batch > 65535 || max_q_len > 65535 * 16 || (long long)batch * max_q_len > 0x7fffffffll ||
         ((long long)head_num + 2ll * kv_head_num) * head_size > (1 << 24) || inter > (1 << 24))
         return ISP_ERR_UNSUPPORTED;
     // wide products of many rows are the library's (5120 x 40928, 64 rows: 85 us there, 124 here)

@@ -165,3 +165,16 @@ def test_build_flags_for_the_kernel_files():
     few = open(os.path.join(build.CSRC, "norm_few_rows.hip")).read()
     assert "__global__" in few and "void fused_norm_few_rows(" in few
     assert "void fused_norm_few_rows(" not in open(os.path.join(build.CSRC, "norm.hip")).read()
+
+
+def test_layer_workspace_says_what_the_whole_layer_supports(lib):
+    """0 where any step of the layer would refuse: nothing may have been launched by then."""
+    need = lambda batch, q: lib.isp_context_layer_f16_workspace(batch, 5, 64, 1, 1, 64, q, 16, 16, 64)   # noqa: E731
+    assert need(1, 16) > 0 and need(65535, 16) > 0 and need(1, 65535 * 16) > 0
+    assert need(65536, 1) == 0 and need(1, 65535 * 16 + 1) == 0
+
+
+def test_no_split_keys_past_the_second_kernels_grid(lib):
+    """Up to 16 queries per group need no workspace where sequences x queries exceed a grid's 65535 rows."""
+    need = lambda batch, q: lib.isp_context_attention_f16_workspace(batch, 1, 1, 64, q, 4096)   # noqa: E731
+    assert need(1, 16) > 0 and need(4096, 16) == 0

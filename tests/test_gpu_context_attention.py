@@ -87,3 +87,21 @@ def test_an_infinite_value_reaches_only_its_own_sum(isp, dtype, hs, lens, hist):
     assert (got[last, :, 5] == float("inf")).all()
     others = torch.arange(hs) != 5
     assert (got - expect)[:, :, others].abs().max() <= (2e-3 if dtype == torch.float16 else 2e-5) * expect.abs().max()
+
+
+@pytest.mark.parametrize("hs", [128, 64])
+def test_more_short_prompts_than_a_grid_row(isp, hs):
+    """4200 sequences of up to 16 tokens: more than 65535 query rows, and few enough queries per group for the decode kernel."""
+    g = torch.Generator().manual_seed(1)
+    lens = [[16, 1, 5, 0][b % 4] for b in range(4200)]
+    q = torch.randn(len(lens), 1, 16, hs, generator=g).half()
+    k, v = (torch.randn(1, len(lens), 1, 16, hs, generator=g).half() for _ in range(2))
+    ints = torch.tensor(lens, dtype=torch.int32, device="cuda")
+    out = torch.zeros(sum(lens), 1, hs, dtype=torch.float16, device="cuda")
+    isp.context_attention(q.cuda(), k.cuda(), v.cuda(), 0, torch.zeros_like(ints), ints, ints, 16, out)
+    some = [b for b in range(len(lens)) if b % 4 != 3][-300:]
+    first = torch.tensor([0] + lens).cumsum(0)
+    expect = reference(q[some], k[0][some], v[0][some], [lens[b] for b in some], [0] * len(some),
+                       torch.zeros(sum(lens[b] for b in some), 1, hs, dtype=torch.float64))
+    got = torch.cat([out[first[b]:first[b + 1]] for b in some]).cpu().double()
+    assert (got - expect).abs().max() <= 2e-3 * expect.abs().max()

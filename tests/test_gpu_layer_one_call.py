@@ -65,3 +65,14 @@ def test_what_is_not_plain_goes_step_by_step(isp):
     out = cl.context_decoder_layer(x, x.clone(), w, st, 0, w.attn_norm)
     w.down = w.down.contiguous()
     assert (out.float() - call(x).float()).abs().max() <= 2.0 ** -9 * out.float().abs().max()
+
+
+def test_a_few_tokens_among_thousands_of_empty_sequences(isp):
+    """More than 65535 query rows: the layer still runs in one call."""
+    from inferspore_amd import context_layer as cl
+    w = cl.LayerWeights(64, 64, torch.float16)
+    st = cl.BatchState([5] + [0] * 4198 + [2], 16, 1, 1, 64, 64, 16, 1, torch.float16)
+    x = torch.randn(7, 64, device="cuda").half()
+    out = cl._layer_in_one_call(x, x.clone(), w, st, 0, w.attn_norm, 64, 1e4, 1e-5)
+    assert out is not None and torch.isfinite(out).all()
+    assert torch.equal(st.packed_ctx[[0, 5], 0], st.v_cache[0, [0, 4199], 0, 0])   # a first token attends to itself

@@ -144,7 +144,7 @@ def _layer_in_one_call(normed, residual, w, st, layer_id, gamma, rotary_dim, rot
         if (type(t) not in _PLAIN or t.dtype != torch.int32 or t.numel() < most or not t.is_contiguous() or
                 t.device != device):
             return None
-    if not (st.tokens == tokens and 0 <= int(layer_id) < st.k_cache.shape[0] and
+    if not (st.tokens == tokens and st.context.shape[0] == batch and 0 <= int(layer_id) < st.k_cache.shape[0] and
             0 <= int(rotary_dim) <= hs and int(rotary_dim) % 2 == 0) or normed.data_ptr() == residual.data_ptr():
         return None
     if not _fused_attention(st):
@@ -186,6 +186,7 @@ def context_decoder_layer(normed, residual, w, state, layer_id, next_norm_gamma,
                                                      w.qkv_bias, st.padding_offset, st.history, st.lengths,
                                                      rotary_dim, rotary_base)
     if _fused_attention(st):
+        ops._expect(st.context.shape[0] == st.k_cache.shape[1], "batch extents differ")
         ops.context_attention(st.q, st.k_cache, st.v_cache, layer_id, st.history, st.lengths, st.context, st.max_k_len,
                               st.packed_ctx)
         if isinstance(st, BatchState):

@@ -120,3 +120,13 @@ def test_more_sequences_than_a_grid_holds(isp):
     x = torch.randn(n, 64, device="cuda").half()
     cl.context_decoder_layer(x, x.clone(), w, st, 0, w.attn_norm, rotary_dim=64)
     assert torch.equal(st.packed_ctx[:, 0], st.v_cache[0, :, 0, 0])   # one key: its value
+
+
+@pytest.mark.parametrize("rows", ["few", "many"])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+def test_context_lengths_of_another_batch_are_refused(isp, dtype, rows):
+    def edit(st):
+        st.context = torch.cat([st.context, st.context])
+
+    with pytest.raises(RuntimeError, match="batch extents"):
+        layers(edit, dtype, rows)

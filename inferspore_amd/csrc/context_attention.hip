@@ -323,10 +323,10 @@ __global__ __launch_bounds__(256, 2) void decode_attention_f16(
     const int group = head_num / kv_head_num;
     const int len = min(read_only_i32(input_length, b), max_q_len);
     const int used = SPLIT ? group * max_q_len : group * len;  // slots with a result
-    if (len <= 0 && !SPLIT) return;
+    if (len <= 0) return;  // workgroup-uniform: no query row to read here, and combine_splits_f16 asks for none
     const int hist = read_only_i32(history_length, b);
     const int ctx = min(min(read_only_i32(context_length, b), max_k_len), max_seq_len);
-    const int wg_visible = len > 0 ? max(0, min(hist + len, ctx)) : 0;
+    const int wg_visible = max(0, min(hist + len, ctx));
     const int head_in_group = j % group, my_q = j / group;
     const bool real = j < group * len;
     const int my_visible = real ? min(hist + my_q + 1, ctx) : 0;
@@ -515,6 +515,7 @@ __global__ __launch_bounds__(64) void combine_splits_f16(const float* __restrict
                                                          const int* input_length, int head_num, int max_q_len, int splits,
                                                          int tokens) {
     const int lane = threadIdx.x, head = blockIdx.x, b = (int)blockIdx.y / max_q_len, q = (int)blockIdx.y % max_q_len;
+    if (q >= read_only_i32(input_length, b)) return;  // workgroup-uniform: no such query
     int n = 0;
     for (int i = lane; i < b; i += 64) n += read_only_i32(input_length, i);
     const float* p = partial + (((size_t)b * head_num + head) * max_q_len + q) * (size_t)splits * partial_floats(HS);
@@ -534,7 +535,7 @@ __global__ __launch_bounds__(64) void combine_splits_f16(const float* __restrict
         for (int i = 0; i < HS / 64; i++) o[i] += e * pz[HS / 64 * lane + i];
     }
     const long long token = (long long)n + q;
-    if (q >= read_only_i32(input_length, b) || token >= tokens) return;
+    if (token >= tokens) return;
     const float inv = l > 0.0f ? 1.0f / l : 0.0f;
 #pragma unroll
     for (int i = 0; i < HS / 64; i++) out[((size_t)token * head_num + head) * HS + HS / 64 * lane + i] = (_Float16)(o[i] * inv);

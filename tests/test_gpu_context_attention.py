@@ -22,7 +22,9 @@ CASES = [([5], [0], 2, 2, 5, 8),
          ([1, 1, 1, 1], [0, 31, 32, 33], 8, 2, 1, 64),
          ([1, 1], [255, 700], 32, 1, 1, 1024),
          ([1] * 9, [3, 700, 128, 127, 129, 511, 512, 513, 0], 16, 16, 1, 768),
-         ([2, 1, 3], [100, 257, 64], 6, 2, 3, 300)]
+         ([2, 1, 3], [100, 257, 64], 6, 2, 3, 300),
+         ([1, 0, 1], [300, 200, 700], 8, 2, 1, 1024),   # an empty sequence among split keys (fp16)
+         ([0, 1, 0], [3, 20, 0], 4, 4, 2, 32)]          # and among whole ones
 
 
 def reference(q, k, v, lens, hist, out):

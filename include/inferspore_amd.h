@@ -299,7 +299,8 @@ int isp_context_attention_split_f16(const void* q, const void* k_cache, const vo
 /*
  * Product of a few rows with a weight matrix, fp32 accumulation: out[m, n] = a[m, k] x w[k, n], all row-major and
  * contiguous (the reference's launchLinearGemm with trans_b = false, src/kernels/linear.cu:7-66).  For the rows of a
- * decode step or a short prompt: m <= 64, n and k multiples of 8, 16-byte aligned pointers, else ISP_ERR_UNSUPPORTED.
+ * decode step or a short prompt: m <= 64, n and k multiples of 8 up to 2^24, 16-byte aligned pointers, else
+ * ISP_ERR_UNSUPPORTED.
  * workspace: isp_linear_f16_workspace(m, n, k) bytes of device memory that no other work in flight uses; may be NULL
  * where that is 0.
  */

@@ -39,7 +39,8 @@ __global__ __launch_bounds__(kBlock) void linear_add_splits(const float* __restr
 static int linear(const __half* a, const __half* w, __half* out, float* workspace, int m, int n, int k, hipStream_t stream) {
     if (m < 0 || n < 0 || k < 0) return ISP_ERR_BAD_SHAPE;
     if (m == 0 || n == 0) return ISP_OK;
-    if (k == 0 || m > kSkinnyMaxRows || n % 8 != 0 || k % 8 != 0) return ISP_ERR_UNSUPPORTED;
+    if (k == 0 || m > kSkinnyMaxRows || n % 8 != 0 || k % 8 != 0 || n > kSkinnyMaxExtent || k > kSkinnyMaxExtent)
+        return ISP_ERR_UNSUPPORTED;
     ISP_REQUIRE_PTR(a);
     ISP_REQUIRE_PTR(w);
     ISP_REQUIRE_PTR(out);
@@ -65,7 +66,7 @@ static int linear(const __half* a, const __half* w, __half* out, float* workspac
 extern "C" {
 
 size_t isp_linear_f16_workspace(int m, int n, int k) {
-    if (m <= 0 || n <= 0 || k <= 0) return 0;
+    if (m <= 0 || n <= 0 || k <= 0 || m > isp::kSkinnyMaxRows || n > isp::kSkinnyMaxExtent || k > isp::kSkinnyMaxExtent) return 0;
     const isp::SkinnyPlan plan = isp::skinny_plan(m, n, k);
     return plan.splits == 1 ? 0 : plan.partial_floats(m, n) * sizeof(float);
 }

@@ -153,6 +153,7 @@ struct SkinnyPlan {
     size_t partial_floats(int m, int n) const { return (size_t)splits * (size_t)m * (size_t)n; }
 };
 constexpr int kSkinnyMaxRows = 64, kSkinnyMaxSplits = 16;
+constexpr int kSkinnyMaxExtent = 1 << 24;  // of n and k: the kernel counts columns, rows and results in 32 bits
 inline SkinnyPlan skinny_plan(int m, int n, int k) {
     SkinnyPlan p;
     const int steps = (k + kStepRows - 1) / kStepRows, waves = kBlock / kWave, units = resident_waves() / 32;

@@ -274,7 +274,7 @@ def linear_supports(x, w):
     against 112 us, 64 rows 85 against 124; 8 rows 80 against 85)."""
     return (x.dtype == torch.float16 and w.dtype == torch.float16 and x.dim() == 2 and w.dim() == 2 and x.is_cuda and
             0 < x.shape[0] <= 64 and (x.shape[0] <= 16 or w.shape[1] <= 32768) and x.shape[1] == w.shape[0] and w.device == x.device and
-            w.shape[0] % 8 == 0 and w.shape[1] % 8 == 0 and w.numel() > 0 and
+            w.shape[0] % 8 == 0 and w.shape[1] % 8 == 0 and w.numel() > 0 and max(w.shape) <= 1 << 24 and
             x.is_contiguous() and w.is_contiguous() and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and
             type(x) is torch.Tensor and type(w) in (torch.Tensor, torch.nn.Parameter) and
             not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad)) and

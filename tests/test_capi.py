@@ -178,3 +178,13 @@ def test_no_split_keys_past_the_second_kernels_grid(lib):
     """Up to 16 queries per group need no workspace where sequences x queries exceed a grid's 65535 rows."""
     need = lambda batch, q: lib.isp_context_attention_f16_workspace(batch, 1, 1, 64, q, 4096)   # noqa: E731
     assert need(1, 16) > 0 and need(4096, 16) == 0
+
+
+@pytest.mark.parametrize("n,k", [(2 ** 31 - 8, 8), (8, 2 ** 31 - 8), (2 ** 24 + 8, 64), (64, 2 ** 24 + 8)])
+def test_linear_refuses_extents_that_its_kernel_cannot_count(lib, n, k):
+    """n + 127 and k + 31 are formed in 32 bits: near 2^31 the strips or the steps came out negative, and a product of
+    zeros, or none, was reported as done."""
+    from inferspore_amd import capi
+    assert lib.isp_linear_f16(None, None, None, None, 1, n, k, None) == capi.ERR_UNSUPPORTED
+    assert lib.isp_linear_f16_workspace(1, n, k) == 0
+    assert lib.isp_linear_f16(None, None, None, None, 1, 2 ** 24, 2 ** 24, None) == capi.ERR_NULL_POINTER

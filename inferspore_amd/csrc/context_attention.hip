@@ -84,8 +84,6 @@ __global__ __launch_bounds__(256, 2) void context_attention_f16(
     if (q0 >= len) return;  // workgroup-uniform: only padded queries here
     const int hist = read_only_i32(history_length, b);
     const int ctx = min(min(read_only_i32(context_length, b), max_k_len), max_seq_len);
-    int first_token = 0;
-    for (int i = 0; i < b; i++) first_token += read_only_i32(input_length, i);
     const int kv_head = head / (head_num / kv_head_num);
     const size_t kv_offset = ((size_t)b * kv_head_num + kv_head) * (size_t)max_seq_len * kHeadSize;
     const _Float16* keys = k_cache + kv_offset;
@@ -101,8 +99,11 @@ __global__ __launch_bounds__(256, 2) void context_attention_f16(
     const bool real = my_q < len;
     const int my_visible = real ? min(hist + my_q + 1, ctx) : 0;
 
-    const long long token = (long long)first_token + my_q;
+    __shared__ int length_shares[kWaves];
+    sum_lengths_share(input_length, b, length_shares);
     if (wg_visible <= 0) {  // workgroup-uniform: a context of no keys (inconsistent lengths); nothing to attend to
+        __syncthreads();
+        const long long token = (long long)sum_lengths_total(length_shares) + my_q;
         if (real && token < tokens) {
             _Float16* o_row = out + ((size_t)token * head_num + head) * kHeadSize;
             for (int d = 8 * half_id; d < kHeadSize; d += 16) *reinterpret_cast<uint4*>(o_row + d) = make_uint4(0u, 0u, 0u, 0u);
@@ -263,6 +264,7 @@ __global__ __launch_bounds__(256, 2) void context_attention_f16(
         __syncthreads();
     }
 
+    const long long token = (long long)sum_lengths_total(length_shares) + my_q;
     // ---- O^T / sum -> the packed token row; accumulator i of block db is d = 32 db + 8 (i / 4) + 4 half_id + i % 4
     if (real && token < tokens) {
         const float inv = run_sum > 0.0f ? 1.0f / run_sum : 0.0f;
@@ -469,14 +471,10 @@ __global__ __launch_bounds__(256, 2) void decode_attention_f16(
                 *reinterpret_cast<float4w*>(&o_lds[wave][j][kChunk * (4 * g + r) + c]) =
                     float4w{acc[c][r], acc[c + 1][r], acc[c + 2][r], acc[c + 3][r]};
     }
-    int first_token = 0;
-    if (!SPLIT) {
-        int n = 0;
-        for (int i = lane; i < b; i += 64) n += read_only_i32(input_length, i);
-        for (int off = 32; off > 0; off >>= 1) n += __shfl_xor(n, off, 64);
-        first_token = n;
-    }
+    __shared__ int length_shares[kWaves];
+    if (!SPLIT) sum_lengths_share(input_length, b, length_shares);
     __syncthreads();
+    const int first_token = SPLIT ? 0 : sum_lengths_total(length_shares);
     for (int at = tid; at < used * (HS / 4); at += 256) {
         const int slot = at / (HS / 4), d = 4 * (at % (HS / 4));
         float m = m_lds[0][slot];

@@ -177,10 +177,10 @@ __global__ __launch_bounds__(256) void context_attention_f32(
             for (int c = 0; c < kChunk; c += 2)
                 *reinterpret_cast<float2*>(&o_lds[wave][j][kChunk * (4 * g + r) + c]) = make_float2(acc[c][r], acc[c + 1][r]);
     }
-    int first_token = 0;
-    for (int i = lane; i < b; i += 64) first_token += read_only_i32(input_length, i);
-    for (int off = 32; off > 0; off >>= 1) first_token += __shfl_xor(first_token, off, 64);
+    __shared__ int length_shares[kWaves];
+    sum_lengths_share(input_length, b, length_shares);
     __syncthreads();
+    const int first_token = sum_lengths_total(length_shares);
     for (int at = tid; at < used * (HS / 4); at += 256) {
         const int slot = at / (HS / 4), d = 4 * (at % (HS / 4));
         float m = m_lds[0][slot];

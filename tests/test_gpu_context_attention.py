@@ -24,7 +24,9 @@ CASES = [([5], [0], 2, 2, 5, 8),
          ([1] * 9, [3, 700, 128, 127, 129, 511, 512, 513, 0], 16, 16, 1, 768),
          ([2, 1, 3], [100, 257, 64], 6, 2, 3, 300),
          ([1, 0, 1], [300, 200, 700], 8, 2, 1, 1024),   # an empty sequence among split keys (fp16)
-         ([0, 1, 0], [3, 20, 0], 4, 4, 2, 32)]          # and among whole ones
+         ([0, 1, 0], [3, 20, 0], 4, 4, 2, 32),          # and among whole ones
+         ([1] * 50 + [0] + [1] * 250, [b % 37 for b in range(301)], 4, 4, 1, 40),   # more sequences than a workgroup has threads,
+         ([20, 3, 0, 17] * 75, [b % 5 for b in range(300)], 2, 1, 20, 25)]          # which add up the lengths before a sequence's
 
 
 def reference(q, k, v, lens, hist, out):

@@ -221,7 +221,8 @@ __global__ __launch_bounds__(256, 2) void context_attention_f16(
             tile_max = halves_max(tile_max);
             const float new_max = fmaxf(run_max, tile_max);
             const float safe_max = new_max == -INFINITY ? 0.0f : new_max;  // a query with no visible key yet
-            const float rescale = __builtin_amdgcn_exp2f((run_max - safe_max) * scale_log2e);
+            // 1 also for a column that sees no key (padded queries): its sum and accumulators are zero
+            const float rescale = new_max == run_max ? 1.0f : __builtin_amdgcn_exp2f((run_max - safe_max) * scale_log2e);
             const float mc = safe_max * scale_log2e;
             float tile_sum = 0.0f;
 #pragma unroll
@@ -397,7 +398,8 @@ __global__ __launch_bounds__(256, 2) void decode_attention_f16(
             }
         const float new_max = fmaxf(run_max, rows_max(m));
         const float safe_max = new_max == -INFINITY ? 0.0f : new_max;  // no visible key yet
-        const float rescale = __builtin_amdgcn_exp2f(run_max - safe_max);
+        // 1 also for a column without a query: its sum and accumulators are zero
+        const float rescale = new_max == run_max ? 1.0f : __builtin_amdgcn_exp2f(run_max - safe_max);
         run_max = new_max;
         run_sum *= rescale;
         half8 p;

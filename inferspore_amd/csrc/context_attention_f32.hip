@@ -137,7 +137,8 @@ __global__ __launch_bounds__(256) void context_attention_f32(
         }
         const float new_max = fmaxf(run_max, rows_max(m));
         const float safe_max = new_max == -INFINITY ? 0.0f : new_max;  // no visible key yet
-        const float rescale = __builtin_amdgcn_exp2f(run_max - safe_max);
+        // 1 also for a column without a query: its sum and accumulators are zero
+        const float rescale = new_max == run_max ? 1.0f : __builtin_amdgcn_exp2f(run_max - safe_max);
         run_max = new_max;
         run_sum *= rescale;
 #pragma unroll

@@ -1,4 +1,4 @@
-// Fused causal attention of a context-decoder layer for fp16 heads of 128 or 64 elements: one kernel in place of
+// Fused causal attention of a context-decoder layer for fp16 heads of 128, 96 or 64 elements: one kernel in place of
 // KV broadcast, q x k^T, masked softmax, p x v and the transpose back to packed tokens.  It reads the padded
 // queries [batch, head_num, max_q_len, hs], the layer's slice of the KV cache [batch, kv_head_num,
 // max_seq_len, hs] (keys and values of the history and of this call's tokens) and writes the packed
@@ -61,7 +61,15 @@ __device__ __forceinline__ float halves_sum(float x) {
     return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
-template <int HS>  // head size: 128 or 64
+// x >= 0 as the sum of two halves: the upper one cut off, so that the lower one has no sign of its own, and neither is 0
+// where x is not (an infinite value times either has to stay that infinity).
+__device__ __forceinline__ _Float16 upper_half(float x) { return (_Float16)__builtin_amdgcn_cvt_pkrtz(x, 0.0f)[0]; }
+__device__ __forceinline__ _Float16 lower_half(float x, _Float16 upper) {
+    const float least = 0x1p-24f;  // fp16's smallest
+    return upper_half(__builtin_amdgcn_fmed3f(x - (float)upper, least, x));
+}
+
+template <int HS>  // head size: 128, 96 or 64
 __global__ __launch_bounds__(256, 2) void context_attention_f16(
     const _Float16* __restrict__ q_buf, const _Float16* __restrict__ k_cache, const _Float16* __restrict__ v_cache,
     _Float16* __restrict__ out, const int* history_length, const int* input_length, const int* context_length,
@@ -70,7 +78,12 @@ __global__ __launch_bounds__(256, 2) void context_attention_f16(
     constexpr int kDSteps = HS / 16;    // products over d per 32 x 32 block of scores
     constexpr int kDBlocks = HS / 32;   // 32-row blocks of O^T
     constexpr int kChunks = HS / 8;     // 16-byte pieces of a key or value row
-    constexpr int kMoves = HS / 64;     // key pairs a thread moves per tile
+    constexpr int kUnits = kChunks * kKeyTile / 2, kMoves = (kUnits + 255) / 256;  // key pairs of 8 d a tile has, a thread moves
+    // Heads of 96: the probabilities as the sum of two halves, each a factor of its own product, so that they keep 21 bits (they
+    // were fp32 in the kernel that served these heads before).  Scaled by 2^15 -- the sum that divides the result is, too -- so
+    // that the lower halves are normal numbers down to probabilities of 2^-18.
+    constexpr bool kTwoHalves = HS == 96;
+    constexpr float kProbabilityExponent = kTwoHalves ? 15.0f : 0.0f;
     __shared__ __align__(16) _Float16 k_tiles[2][kKeyTile * kKStride];
     __shared__ __align__(16) uint32_t vt_tiles[2][kHeadSize * kKeyTile / 2];  // [d][key], two keys per dword
 
@@ -138,7 +151,8 @@ __global__ __launch_bounds__(256, 2) void context_attention_f16(
     auto fetch = [&](int kt) {
 #pragma unroll
         for (int i = 0; i < kMoves; i++) {
-            const int unit = tid + 256 * i, d0 = (unit % kChunks) * 8, key = 2 * (unit / kChunks);
+            // heads of 96 leave half of the second moves idle: they re-read the first
+            const int unit = tid + 256 * i < kUnits ? tid + 256 * i : tid, d0 = (unit % kChunks) * 8, key = 2 * (unit / kChunks);
 #pragma unroll
             for (int j = 0; j < 2; j++) {
                 const size_t at = (size_t)min(kt + key + j, wg_visible - 1) * kHeadSize + d0;
@@ -155,6 +169,7 @@ __global__ __launch_bounds__(256, 2) void context_attention_f16(
 #pragma unroll
         for (int i = 0; i < kMoves; i++) {
             const int unit = tid + 256 * i, pair = unit / kChunks, d0 = (unit % kChunks) * 8, key = 2 * pair;
+            if (unit >= kUnits) break;  // wavefront-uniform
             uint32_t lo[4], hi[4];
 #pragma unroll
             for (int j = 0; j < 2; j++) {
@@ -223,7 +238,7 @@ __global__ __launch_bounds__(256, 2) void context_attention_f16(
             const float safe_max = new_max == -INFINITY ? 0.0f : new_max;  // a query with no visible key yet
             // 1 also for a column that sees no key (padded queries): its sum and accumulators are zero
             const float rescale = new_max == run_max ? 1.0f : __builtin_amdgcn_exp2f((run_max - safe_max) * scale_log2e);
-            const float mc = safe_max * scale_log2e;
+            const float mc = safe_max * scale_log2e - kProbabilityExponent;
             float tile_sum = 0.0f;
 #pragma unroll
             for (int rb = 0; rb < 2; rb++)
@@ -249,12 +264,19 @@ __global__ __launch_bounds__(256, 2) void context_attention_f16(
 #pragma unroll
                 for (int db = 0; db < kDBlocks; db++)
                     va[db] = *reinterpret_cast<const half8*>(&vt_lds[vt_unit(32 * db + col, 2 * t + half_id)]);
-                half8 p;
+                half8 p, low;
 #pragma unroll
-                for (int e = 0; e < 8; e++) p[e] = (_Float16)s[rb][4 * (g0 + e / 4) + (e % 4)];
+                for (int e = 0; e < 8; e++) {
+                    const float x = s[rb][4 * (g0 + e / 4) + (e % 4)];
+                    p[e] = kTwoHalves ? upper_half(x) : (_Float16)x;
+                    if (kTwoHalves) low[e] = lower_half(x, p[e]);
+                }
                 __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                for (int db = 0; db < kDBlocks; db++) acc[db] = __builtin_amdgcn_mfma_f32_32x32x16_f16(va[db], p, acc[db], 0, 0, 0);
+                for (int db = 0; db < kDBlocks; db++) {
+                    acc[db] = __builtin_amdgcn_mfma_f32_32x32x16_f16(va[db], p, acc[db], 0, 0, 0);
+                    if (kTwoHalves) acc[db] = __builtin_amdgcn_mfma_f32_32x32x16_f16(va[db], low, acc[db], 0, 0, 0);
+                }
             }
         }
         // the next tile (its loads were issued before this tile's products) goes into the other buffer, which every
@@ -567,6 +589,16 @@ int context_attention_f16_96(const __half* q, const __half* k_cache, const __hal
                              int batch, int head_num, int kv_head_num, int max_q_len, int max_k_len, int max_seq_len,
                              int token_num, float scale, hipStream_t stream);
 
+// Heads of 96 elements have two kernels.  The fp32 one splits a sequence's keys over the four wavefronts of a workgroup, which has 16
+// queries; it serves the few queries of a decode step, and prompts while its workgroups all run at once.  Beyond that the
+// matrix rate counts, and the tiled one here has four to five times its: 500 ... 8000 keys, one workgroup per compute unit or less
+// 17 ... 216 against 23 ... 254 us, at 384 workgroups 27 ... 305 against 23 ... 254, 2 x 2048 tokens with 32 heads 535 against 113 (the
+// padded form: 379).
+static bool attention_96_in_fp32(int batch, int head_num, int kv_head_num, int max_q_len) {
+    return (long long)(head_num / kv_head_num) * max_q_len <= kSlots ||
+           (long long)batch * head_num * ((max_q_len + 15) / 16) <= resident_waves() / 32;
+}
+
 // `workspace` NULL: a sequence's keys are not split.
 int context_attention(const _Float16* q, const _Float16* k_cache, const _Float16* v_cache, _Float16* out,
                       const int32_t* history_length, const int32_t* input_length, const int32_t* context_length,
@@ -575,12 +607,12 @@ int context_attention(const _Float16* q, const _Float16* k_cache, const _Float16
     if (layer < 0 || batch < 0 || head_num <= 0 || kv_head_num <= 0 || head_num % kv_head_num != 0 || max_q_len < 0 ||
         max_k_len < 0 || max_seq_len < 0 || token_num < 0 || !(scale > 0.0f))
         return ISP_ERR_BAD_SHAPE;
-    if (head_size == 96)
+    if (head_size == 96 && attention_96_in_fp32(batch, head_num, kv_head_num, max_q_len))
         return context_attention_f16_96(reinterpret_cast<const __half*>(q), reinterpret_cast<const __half*>(k_cache),
                                         reinterpret_cast<const __half*>(v_cache), reinterpret_cast<__half*>(out), history_length,
                                         input_length, context_length, layer, batch, head_num, kv_head_num, max_q_len, max_k_len,
                                         max_seq_len, token_num, scale, stream);
-    if (head_size != 128 && head_size != 64) return ISP_ERR_UNSUPPORTED;
+    if (head_size != 128 && head_size != 96 && head_size != 64) return ISP_ERR_UNSUPPORTED;
     if (batch == 0 || max_q_len == 0 || token_num == 0) return ISP_OK;
     if (max_k_len == 0 || max_seq_len == 0) return ISP_ERR_BAD_SHAPE;
     const int tiles = (max_q_len + kQueryTile - 1) / kQueryTile;
@@ -628,6 +660,7 @@ int context_attention(const _Float16* q, const _Float16* k_cache, const _Float16
                        history_length, input_length, context_length, head_num, kv_head_num, max_q_len, max_k_len,   \
                        max_seq_len, token_num, scale_log2e)
     if (head_size == 128) ISP_LAUNCH_ATTENTION(128);
+    else if (head_size == 96) ISP_LAUNCH_ATTENTION(96);
     else ISP_LAUNCH_ATTENTION(64);
 #undef ISP_LAUNCH_ATTENTION
     return note_launch(hipGetLastError());

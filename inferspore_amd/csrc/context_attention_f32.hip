@@ -1,5 +1,5 @@
-// Fused causal attention for fp32 heads of 64, 96 or 128 elements, and for fp16 heads of 96 (the tiles of the fp16 kernels want
-// multiples of 64), which are converted when they are loaded: what context_attention.hip does for fp16, in fp32 throughout
+// Fused causal attention for fp32 heads of 64, 96 or 128 elements, and for fp16 heads of 96 with few queries (the decode kernel of
+// context_attention.hip wants powers of two), which are converted when they are loaded: what that file does for fp16, in fp32 throughout
 // (v_mfma_f32_16x16x4_f32 multiplies and adds fp32; probabilities and sums stay fp32).  In place of KV broadcast, a mask tensor,
 // torch's attention, two layout copies and the transpose to packed rows.
 //
@@ -14,8 +14,8 @@
 // Against those five launches, us: 4 prompts of 100 tokens, 16 heads of 128: 11.0, 46.7; 1000 and 700 tokens, 32 heads over 8 key
 // heads: 225, 887; 8 x 300 tokens on a history of 700, 32 heads: 650, 860; decode, 16 sequences of 1000 keys, 32 heads: 117, 449;
 // 64 of 400, 32 heads of 96 over 8: 34, 343.  fp16 heads of 96: decode, 16 x 1000 keys, 32 heads 47, 140; 64 x 400, 32 over 8
-// 26, 234; 8 prompts of 100 tokens 19, 51; 4 of 1000 291, 352; 4 of 2000 1086, 1164; 12 x 200 on a history of 800, 40 heads 415, 401
-// (16 queries per tile: the keys come from the caches once per tile), the one measured extent where it is not ahead.  Error against 64 bits 1.5e-7 ... 3.7e-7 (2-norm), there 2.1e-7 ... 6.9e-7.
+// 26, 234; prompts beyond one workgroup per compute unit are the tiled kernel's.  Error against 64 bits 1.5e-7 ... 3.7e-7 (2-norm),
+// there 2.1e-7 ... 6.9e-7.
 #include <type_traits>
 
 #include "isp_common.h"

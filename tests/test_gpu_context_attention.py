@@ -26,7 +26,10 @@ CASES = [([5], [0], 2, 2, 5, 8),
          ([1, 0, 1], [300, 200, 700], 8, 2, 1, 1024),   # an empty sequence among split keys (fp16)
          ([0, 1, 0], [3, 20, 0], 4, 4, 2, 32),          # and among whole ones
          ([1] * 50 + [0] + [1] * 250, [b % 37 for b in range(301)], 4, 4, 1, 40),   # more sequences than a workgroup has threads,
-         ([20, 3, 0, 17] * 75, [b % 5 for b in range(300)], 2, 1, 20, 25)]          # which add up the lengths before a sequence's
+         ([20, 3, 0, 17] * 75, [b % 5 for b in range(300)], 2, 1, 20, 25),          # which add up the lengths before a sequence's
+         ([129, 64], [0, 64], 32, 4, 130, 200),         # from here on more than 256 tiles of 16 queries: fp16 heads of 96 take
+         ([31, 0, 17], [97, 5, 9], 64, 8, 33, 130),     # the tiled kernel
+         ([33, 32], [31, 96], 64, 64, 33, 128)]
 
 
 def reference(q, k, v, lens, hist, out):
@@ -70,14 +73,15 @@ def test_attention_matches_float64(isp, dtype, hs, case):
 
 @pytest.mark.parametrize("dtype,hs", [(torch.float16, 128), (torch.float16, 96), (torch.float16, 64), (torch.float32, 128),
                                       (torch.float32, 96), (torch.float32, 64)])
-@pytest.mark.parametrize("lens,hist", [([1, 1, 1], [40, 100, 2]), ([20, 5], [0, 13])])
-def test_an_infinite_value_reaches_only_its_own_sum(isp, dtype, hs, lens, hist):
+@pytest.mark.parametrize("even", [False, True])   # equal probabilities: powers of two before the division
+@pytest.mark.parametrize("lens,hist,heads", [([1, 1, 1], [40, 100, 2], 4), ([20, 5], [0, 13], 4), ([121, 40], [0, 13], 32)])
+def test_an_infinite_value_reaches_only_its_own_sum(isp, dtype, hs, lens, hist, heads, even):
     """An infinite element of a sequence's last visible value row, where no block of keys ends: the queries that see it get
     infinity in that element (not NaN: the rest of the block counts as nothing), and no other element is touched."""
     print("[case] infinite value %s hs %d %s" % (dtype, hs, lens), flush=True)
     g = torch.Generator().manual_seed(hs)
-    batch, heads, max_seq = len(lens), 4, 128
-    q = torch.randn(batch, heads, max(lens), hs, generator=g).to(dtype)
+    batch, max_seq = len(lens), 128
+    q = (0 if even else 1) * torch.randn(batch, heads, max(lens), hs, generator=g).to(dtype)
     k, v = (torch.randn(1, batch, 2, max_seq, hs, generator=g).to(dtype) for _ in range(2))
     context = [a + b for a, b in zip(lens, hist)]
     expect = reference(q, k[0], v[0], lens, hist, torch.zeros(sum(lens), heads, hs, dtype=torch.float64))
@@ -109,3 +113,18 @@ def test_more_short_prompts_than_a_grid_row(isp, hs):
                        torch.zeros(sum(lens[b] for b in some), 1, hs, dtype=torch.float64))
     got = torch.cat([out[first[b]:first[b + 1]] for b in some]).cpu().double()
     assert (got - expect).abs().max() <= 2e-3 * expect.abs().max()
+
+
+@pytest.mark.parametrize("lens,hist,heads,kv,max_seq", [([300, 77], [0, 0], 16, 2, 320), ([65, 130], [900, 30], 32, 8, 1000), ([24], [3000], 2, 2, 3100)])
+def test_float16_heads_of_96_keep_their_probabilities(isp, lens, hist, heads, kv, max_seq):
+    """The probabilities of 96-element heads are not rounded to fp16 (two halves, 21 bits): the error is the result's own rounding, 2^-11,
+    and 2e-5 of the largest output for the scores, as in float32."""
+    g = torch.Generator().manual_seed(7)
+    batch, context = len(lens), [a + b for a, b in zip(lens, hist)]
+    q = 2 * torch.randn(batch, heads, max(lens), 96, generator=g).half()
+    k, v = (torch.randn(1, batch, kv, max_seq, 96, generator=g).half() for _ in range(2))
+    expect = reference(q, k[0], v[0], lens, hist, torch.zeros(sum(lens), heads, 96, dtype=torch.float64))
+    ints = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")   # noqa: E731
+    out = torch.zeros(sum(lens), heads, 96, dtype=torch.float16, device="cuda")
+    isp.context_attention(q.cuda(), k.cuda(), v.cuda(), 0, ints(hist), ints(lens), ints(context), max(context), out)
+    assert ((out.cpu().double() - expect).abs() <= 2.0 ** -11 * expect.abs() + 2e-5 * expect.abs().max()).all()

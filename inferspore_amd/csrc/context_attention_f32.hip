@@ -113,7 +113,7 @@ __global__ __launch_bounds__(256) void context_attention_f32(
     float run_max = -INFINITY, run_sum = 0.0f;  // run_sum: this lane's keys only
 
     const auto block = [&](int s, auto tail) {
-        // a key past the visible ones (in a tail only) re-reads the last visible row: its score is masked, its value counts as zero
+        // a key past the visible ones (in the last block only) re-reads the last visible row: its score is masked, its value counts as zero
         float kf[kQuarter], vf[4][kChunk];
         const T* k_row = keys + (size_t)min(s * kBlockKeys + j, wg_visible - 1) * HS + kQuarter * g;
         load_row<kQuarter>(k_row, kf);
@@ -158,9 +158,10 @@ __global__ __launch_bounds__(256) void context_attention_f32(
                 acc[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(exists ? vf[r][c] : 0.0f, p[r], acc[c], 0, 0, 0);
         }
     };
-    const int whole = wg_visible / kBlockKeys, blocks = (wg_visible + kBlockKeys - 1) / kBlockKeys;
+    // every wavefront's last block is treated as a tail: contexts of a few blocks then run one copy of the code only
+    const int blocks = (wg_visible + kBlockKeys - 1) / kBlockKeys;
     int s = wave;
-    for (; s < whole; s += kWaves) block(s, std::false_type{});
+    for (; s + kWaves < blocks; s += kWaves) block(s, std::false_type{});
     if (s < blocks) block(s, std::true_type{});
 
     // O^T row 4 g + r of product c is d = kChunk (4 g + r) + c

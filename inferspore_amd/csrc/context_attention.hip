@@ -589,14 +589,13 @@ int context_attention_f16_96(const __half* q, const __half* k_cache, const __hal
                              int batch, int head_num, int kv_head_num, int max_q_len, int max_k_len, int max_seq_len,
                              int token_num, float scale, hipStream_t stream);
 
-// Heads of 96 elements have two kernels.  The fp32 one splits a sequence's keys over the four wavefronts of a workgroup, which has 16
-// queries; it serves the few queries of a decode step, and prompts while its workgroups all run at once.  Beyond that the
-// matrix rate counts, and the tiled one here has four to five times its: 500 ... 8000 keys, one workgroup per compute unit or less
-// 17 ... 216 against 23 ... 254 us, at 384 workgroups 27 ... 305 against 23 ... 254, 2 x 2048 tokens with 32 heads 535 against 113 (the
-// padded form: 379).
-static bool attention_96_in_fp32(int batch, int head_num, int kv_head_num, int max_q_len) {
-    return (long long)(head_num / kv_head_num) * max_q_len <= kSlots ||
-           (long long)batch * head_num * ((max_q_len + 15) / 16) <= resident_waves() / 32;
+// Heads of 96 elements have two kernels.  The fp32 one has 16 queries per workgroup, whose four wavefronts split a sequence's keys; it
+// serves up to 16 queries, and more while its workgroups all run at once.  Beyond that the matrix rate counts, and the
+// tiled one here has four to five times its.  500 ... 8000 keys, at most one workgroup per compute unit: 17 ... 216 against 23 ... 254
+// us; at 384 workgroups 27 ... 305 against 23 ... 254; 2 x 2048 tokens with 32 heads 535 against 113 (the padded form: 379).  256
+// sequences, 32 heads, 8 and 16 queries on 50 keys 58 and 75 against 88 and 121, 20 queries 134 against 122.
+static bool attention_96_in_fp32(int batch, int head_num, int max_q_len) {
+    return max_q_len <= 16 || (long long)batch * head_num * ((max_q_len + 15) / 16) <= resident_waves() / 32;
 }
 
 // `workspace` NULL: a sequence's keys are not split.
@@ -607,7 +606,7 @@ int context_attention(const _Float16* q, const _Float16* k_cache, const _Float16
     if (layer < 0 || batch < 0 || head_num <= 0 || kv_head_num <= 0 || head_num % kv_head_num != 0 || max_q_len < 0 ||
         max_k_len < 0 || max_seq_len < 0 || token_num < 0 || !(scale > 0.0f))
         return ISP_ERR_BAD_SHAPE;
-    if (head_size == 96 && attention_96_in_fp32(batch, head_num, kv_head_num, max_q_len))
+    if (head_size == 96 && attention_96_in_fp32(batch, head_num, max_q_len))
         return context_attention_f16_96(reinterpret_cast<const __half*>(q), reinterpret_cast<const __half*>(k_cache),
                                         reinterpret_cast<const __half*>(v_cache), reinterpret_cast<__half*>(out), history_length,
                                         input_length, context_length, layer, batch, head_num, kv_head_num, max_q_len, max_k_len,

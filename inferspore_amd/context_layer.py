@@ -47,6 +47,27 @@ class LayerWeights:
         self.ffn_norm = (0.5 + torch.rand(hidden, device=device, generator=generator)).to(dtype)
 
 
+def _padded_is_faster(dtype, batch, max_q_len, max_k_len, head_num, kv_head_num, head_size):
+    """Thousands of contexts of a few keys.  A workgroup of the fused kernels costs 5 to 10 ns of the chip even then, one per key
+    head (up to 16 queries per group) or per query head; torch's kernel works in tiles of 16 keys and takes 2.5 to 9 ns per head.
+    float16, 128 elements, us fused and padded: 1000 prompts of 7 / 12 / 16 tokens, 32 heads over 8 313 and 172 / 331 and 240 / 340
+    and 296, of 24 363 and 673; 4000 decode rows of 8 keys, 8 heads 193 and 123, 8 over 2 below it.  Beyond ten thousand
+    sequences the lengths that every workgroup adds up count as well: 16000 decode rows of 8 keys, 8 heads 959 and 470; in float32
+    60000 of 1 / 8 / 12 keys 5359 and 3141 / 5585 and 4017 / level.  Heads of 96 in float16 lie in between (4000 rows of 2 keys
+    132 and 117, 16000 of 12 876 and 808).  Fewer workgroups are over before torch's launches are: 1000 rows of 4 keys, 8 heads of
+    64, 30 and 41."""
+    if max_k_len > 16 or batch * head_num * head_size < 1000000:
+        return False
+    tiled = head_num // max(kv_head_num, 1) * max_q_len > 16
+    if not tiled and head_num != kv_head_num:
+        return False
+    if dtype == torch.float32:
+        return max_k_len <= batch // 7000
+    if head_size == 96:
+        return batch >= 4000 and max_k_len <= min(12, batch // 2000)
+    return tiled or batch >= 16000 or max_k_len <= 8
+
+
 class BatchState:
     """Padding bookkeeping of one ragged prefill batch plus the buffers a layer needs."""
 
@@ -73,7 +94,9 @@ class BatchState:
         self.act = z(self.tokens, inter)
 
         self._attended = None   # the layer whose attention ran last without the buffers below
-        if not ops.context_attention_supports(dtype, head_size):
+        if (not ops.context_attention_supports(dtype, head_size) or
+                (self.tokens > 64 and _padded_is_faster(dtype, self.batch, max_q_len, self.max_k_len, head_num, kv_head_num,
+                                                        head_size))):
             self._padded_buffers()
 
     def _padded_buffers(self):

@@ -130,3 +130,29 @@ def test_context_lengths_of_another_batch_are_refused(isp, dtype, rows):
 
     with pytest.raises(RuntimeError, match="batch extents"):
         layers(edit, dtype, rows)
+
+
+@pytest.mark.parametrize("dtype,hs,lens,heads,kv", [(torch.float16, 64, [7, 3] * 500, 8, 2), (torch.float16, 128, [1] * 4000, 2, 2),
+                                                    (torch.float16, 96, [2, 1] * 2500, 2, 2), (torch.float32, 64, [1, 2] * 8000, 1, 1)])
+def test_thousands_of_tiny_contexts_take_the_padded_form(isp, dtype, hs, lens, heads, kv):
+    from inferspore_amd import context_layer as cl
+    hidden = 64
+    g = torch.Generator(device="cuda").manual_seed(2)
+    st = cl.BatchState(lens, max(lens), heads, kv, hs, 32, max(lens), 1, dtype)
+    assert "k_all" in st.__dict__
+    w = cl.LayerWeights(hidden, 32, dtype, generator=g)
+    width = (heads + 2 * kv) * hs
+    w.qkv = (torch.randn(hidden, width, device="cuda", generator=g) * hidden ** -0.5).to(dtype)
+    w.o = (torch.randn(heads * hs, hidden, device="cuda", generator=g) * hidden ** -0.5).to(dtype)
+    x = torch.randn(sum(lens), hidden, device="cuda", generator=g).to(dtype)
+    cl.context_decoder_layer(x, x.clone(), w, st, 0, w.attn_norm, rotary_dim=hs)
+    padded = st.packed_ctx.clone()
+    isp.context_attention(st.q, st.k_cache, st.v_cache, 0, st.history, st.lengths, st.context, st.max_k_len, st.packed_ctx)
+    assert (padded.float() - st.packed_ctx.float()).abs().max() <= (4e-3 if dtype == torch.float16 else 4e-5) * padded.abs().max()
+
+
+@pytest.mark.parametrize("lens,history", [([7] * 200, 0), ([24] * 1000, 0), ([1] * 4000, 31)])
+def test_other_batches_build_no_padded_buffers(isp, lens, history):
+    from inferspore_amd import context_layer as cl
+    st = cl.BatchState(lens, max(lens), 8, 2, 64, 32, max(lens) + history, 1, torch.float16, history=[history] * len(lens))
+    assert "k_all" not in st.__dict__ and "mask" not in st.__dict__

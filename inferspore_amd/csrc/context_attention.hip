@@ -113,8 +113,9 @@ __global__ __launch_bounds__(256, 2) void context_attention_f16(
     const int my_visible = real ? min(hist + my_q + 1, ctx) : 0;
 
     __shared__ int length_shares[kWaves];
-    sum_lengths_share(input_length, b, length_shares);
+    const int length_share = sum_lengths_thread(input_length, b);
     if (wg_visible <= 0) {  // workgroup-uniform: a context of no keys (inconsistent lengths); nothing to attend to
+        sum_lengths_wave(length_share, b, length_shares);
         __syncthreads();
         const long long token = (long long)sum_lengths_total(length_shares) + my_q;
         if (real && token < tokens) {
@@ -194,6 +195,7 @@ __global__ __launch_bounds__(256, 2) void context_attention_f16(
     fetch(0);
     store(0, 0);
     fetch(kKeyTile);  // past the last tile a fetch re-reads the last visible row; what it brings is stored as zeros
+    sum_lengths_wave(length_share, b, length_shares);
     __syncthreads();
 
     int cur = 0;
@@ -496,7 +498,7 @@ __global__ __launch_bounds__(256, 2) void decode_attention_f16(
                     float4w{acc[c][r], acc[c + 1][r], acc[c + 2][r], acc[c + 3][r]};
     }
     __shared__ int length_shares[kWaves];
-    if (!SPLIT) sum_lengths_share(input_length, b, length_shares);
+    if (!SPLIT) sum_lengths_wave(sum_lengths_thread(input_length, b), b, length_shares);
     __syncthreads();
     const int first_token = SPLIT ? 0 : sum_lengths_total(length_shares);
     for (int at = tid; at < used * (HS / 4); at += 256) {

@@ -180,7 +180,7 @@ __global__ __launch_bounds__(256) void context_attention_f32(
                 *reinterpret_cast<float2*>(&o_lds[wave][j][kChunk * (4 * g + r) + c]) = make_float2(acc[c][r], acc[c + 1][r]);
     }
     __shared__ int length_shares[kWaves];
-    sum_lengths_share(input_length, b, length_shares);
+    sum_lengths_wave(sum_lengths_thread(input_length, b), b, length_shares);
     __syncthreads();
     const int first_token = sum_lengths_total(length_shares);
     for (int at = tid; at < used * (HS / 4); at += 256) {

@@ -255,14 +255,18 @@ __device__ __forceinline__ int32_t read_only_i32(const int32_t* p, int i) {
     return reinterpret_cast<constant_ints>((unsigned long long)p)[i];
 }
 
-// Sum of lengths[0 .. n) over a workgroup of kBlock threads, in two steps around a barrier that the kernel has anyway: every
-// wavefront leaves its share in waves[wave], and after the barrier the shares are added.  One lane that added them up
-// alone, one scalar load after another, took 60 % of an attention over 1000 prompts of 20 tokens.
-__device__ __forceinline__ void sum_lengths_share(const int32_t* lengths, int n, int* waves) {
+// Sum of lengths[0 .. n) over a workgroup of kBlock threads, around a barrier that the kernel has anyway: every thread reads its
+// share early, every wavefront leaves its own in waves[wave] before the barrier, and after it they are added.  One lane that
+// added them up alone, one scalar load after another, took 60 % of an attention over 1000 prompts of 20 tokens.
+__device__ __forceinline__ int sum_lengths_thread(const int32_t* lengths, int n) {
     int share = 0;
 #pragma unroll 4
     for (int i = (int)threadIdx.x; i < n; i += kBlock) share += read_only_i32(lengths, i);
-    for (int off = 32; off > 0; off >>= 1) share += __shfl_xor(share, off, kWave);
+    return share;
+}
+__device__ __forceinline__ void sum_lengths_wave(int share, int n, int* waves) {
+    if (n > 0)  // workgroup-uniform
+        for (int off = 32; off > 0; off >>= 1) share += __shfl_xor(share, off, kWave);
     if (threadIdx.x % kWave == 0) waves[threadIdx.x / kWave] = share;
 }
 __device__ __forceinline__ int sum_lengths_total(const int* waves) {

@@ -100,8 +100,9 @@ __global__ __launch_bounds__(256) void context_attention_f32(
     const size_t kv_offset = ((size_t)b * kv_head_num + kv_head) * (size_t)max_seq_len * HS;
     const T *keys = k_cache + kv_offset, *values = v_cache + kv_offset;
 
+    const int blocks = (wg_visible + kBlockKeys - 1) / kBlockKeys;
     float qf[kQuarter];
-    {
+    if (wave < blocks) {  // a wavefront without keys has no use for the queries
         const T* q_row = q_buf + (((size_t)b * head_num + my_head) * (size_t)max_q_len + my_q) * HS + kQuarter * g;
         load_row<kQuarter>(q_row, qf);
 #pragma unroll
@@ -159,7 +160,6 @@ __global__ __launch_bounds__(256) void context_attention_f32(
         }
     };
     // every wavefront's last block is treated as a tail: contexts of a few blocks then run one copy of the code only
-    const int blocks = (wg_visible + kBlockKeys - 1) / kBlockKeys;
     int s = wave;
     for (; s + kWaves < blocks; s += kWaves) block(s, std::false_type{});
     if (s < blocks) block(s, std::true_type{});

@@ -7,19 +7,20 @@ src/weights/llama/layer_weights.cc:19-62), so that the kernels can be exercised 
 order a model runs them:
 
     normed, residual                       (packed [tokens, H]; `normed` = RMSNorm(residual) by attn_norm)
-    qkv      = normed @ Wqkv                                 library GEMM (out of this library's scope)
+    qkv      = normed @ Wqkv                                 product
     q, cache += k, v = add_fused_qkv_bias_transpose_rope_and_append(qkv)    * this library
-    packed   = context_attention(q, cache)                   * this library (heads of 64, 96 or 128 elements; others:
-                                                               repeat_kv_cache, torch's attention, transpose_out_remove_padding)
-    attn_out = packed @ Wo                                   library GEMM
+    packed   = context_attention(q, cache)                   * this library (heads of 64, 96 or 128 elements; others, and
+                                                               a state with a mask of its own: repeat_kv_cache, torch's
+                                                               attention, transpose_out_remove_padding)
+    attn_out = packed @ Wo                                   product
     residual, normed2 = fused_add_bias_residual_rmsnorm(residual, attn_out, ffn_norm)      * this library
-    act      = SwiGLU(normed2 @ Wgate_up)                    library GEMM + * this library
-    ffn_out  = act @ Wdown                                   library GEMM
+    act      = SwiGLU(normed2 @ Wgate_up)                    product + * this library
+    ffn_out  = act @ Wdown                                   product
     residual, normed_next = fused_add_bias_residual_rmsnorm(residual, ffn_out, next attn_norm)   * this library
 
-Dense contractions of more than 64 rows are left to torch's library calls (hipBLASLt GEMMs), those of fewer float16 rows go to
-ops.linear, and a layer of such rows is one call of the C ABI (isp_context_layer_f16); everything marked * goes through the
-C ABI.  All work is issued on torch's current stream.
+Products of more than 64 rows, and those in float32, are left to torch's library calls (hipBLASLt GEMMs), those of up to 64 float16
+rows go to ops.linear, and a layer of such rows is one call of the C ABI (isp_context_layer_f16); everything marked * goes
+through the C ABI.  All work is issued on torch's current stream.
 """
 import math
 

@@ -42,7 +42,9 @@ static int layer_shape(int layer, int batch, int tokens, int hidden, int head_nu
         inter % 8 != 0 || batch > 65535 || max_q_len > 65535 * 16 || (long long)batch * max_q_len > 0x7fffffffll ||
         ((long long)head_num + 2ll * kv_head_num) * head_size > (1 << 24) || inter > (1 << 24))
         return ISP_ERR_UNSUPPORTED;
-    // wide products of many rows are the library's (5120 x 40928, 64 rows: 85 us there, 124 here)
+    // wide products of many rows are the library's (5120 x 40928, 64 rows: 85 us there, 124 here); below the line a whole layer is
+    // ahead of its steps, with the library's products or with these (4096 wide, 64 rows, 2 x inter 20480 ... 32768: 159 ... 172 us
+    // against 163 ... 174, 166 ... 188 with the library for gate / up and 244 ... 293 with it for all four)
     if (tokens > 16 && (2 * inter > 32768 || (head_num + 2 * kv_head_num) * head_size > 32768)) return ISP_ERR_UNSUPPORTED;
     return ISP_OK;
 }

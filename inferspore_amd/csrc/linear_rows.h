@@ -144,10 +144,12 @@ __global__ __launch_bounds__(kBlock) void linear_skinny_f16(const __half* __rest
 
 // How many workgroups share a strip of columns.  Two costs are weighed: the rounds of one workgroup per compute unit that
 // strips x splits make, over those that whole rounds would make (idle units at the end), and the partial sums, whose bytes
-// are 4 m splits / k of the weights' and count twice (they are written and read back by a dependent kernel).  Measured with 16
+// are 2 m splits / k of the weights', written once and read back once.  The factor 4 in front of that ratio (2 would be the
+// bytes alone) is what the measured plans want: the reading kernel depends on the last of them.  Measured with 16
 // rows: 96 strips of 4096 rows (100.7 MB) 1, 2, 3, 4, 5, 8 splits 30.0, 19.4, 24.7, 20.5, 18.5, 19.0 us (taken: 5); 32
 // strips (33.6 MB) 4, 8, 16 splits 9.9, 7.8, 7.7 (8); 172 strips 1, 2, 4 splits 34.7, 37.9, 32.5 (4).  With 64 rows: 32
-// strips 4, 8, 16 splits 14.7, 11.3, 15.9 (8); 224 strips 1, 2 splits 49.7, 57.2 (1).  Every wavefront keeps a step.
+// strips 4, 8, 16 splits 14.7, 11.3, 15.9 (8); 224 strips 1, 2 splits 49.7, 57.2 (1).  Every wavefront keeps a step, except in a
+// last split that rounding up the others' steps leaves short.
 struct SkinnyPlan {
     int strips, splits, steps_per_split;
     size_t partial_floats(int m, int n) const { return (size_t)splits * (size_t)m * (size_t)n; }

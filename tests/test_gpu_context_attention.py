@@ -97,6 +97,30 @@ def test_an_infinite_value_reaches_only_its_own_sum(isp, dtype, hs, lens, hist, 
     assert (got - expect)[:, :, others].abs().max() <= (2e-3 if dtype == torch.float16 else 2e-5) * expect.abs().max()
 
 
+@pytest.mark.parametrize("dtype,hs", [(torch.float16, 128), (torch.float16, 96), (torch.float16, 64), (torch.float32, 128),
+                                      (torch.float32, 96), (torch.float32, 64)])
+@pytest.mark.parametrize("lens,heads", [([1, 1, 1], 2), ([1] * 90, 8), ([20, 33, 40], 2), ([130, 33, 40], 64)])
+def test_a_context_of_no_keys_gives_zeros(isp, dtype, hs, lens, heads):
+    """context_length 0 for one sequence (inconsistent lengths): nothing to attend to, zeros -- with split keys, whole ones and
+    in the prompt kernels; its neighbours are untouched."""
+    print("[case] no keys %s hs %d %s" % (dtype, hs, lens[:3]), flush=True)
+    g = torch.Generator().manual_seed(hs)
+    batch, max_seq = len(lens), 600 if max(lens) == 1 else max(lens)
+    hist = [max_seq - n for n in lens]
+    q = torch.randn(batch, heads, max(lens), hs, generator=g).to(dtype)
+    k, v = (torch.randn(1, batch, heads, max_seq, hs, generator=g).to(dtype) for _ in range(2))
+    ints = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")   # noqa: E731
+    out = torch.full((sum(lens), heads, hs), float("nan"), dtype=dtype, device="cuda")
+    isp.context_attention(q.cuda(), k.cuda(), v.cuda(), 0, ints(hist), ints(lens), ints([max_seq, 0] + [max_seq] * (batch - 2)), max_seq, out)
+    first = lens[0]
+    assert not out[first:first + lens[1]].any()
+    rest = [0, batch - 1]
+    expect = reference(q[rest], k[0][rest], v[0][rest], [lens[b] for b in rest], [hist[b] for b in rest],
+                       torch.zeros(lens[0] + lens[-1], heads, hs, dtype=torch.float64))
+    got = torch.cat([out[:first], out[-lens[-1]:]]).cpu().double()
+    assert (got - expect).abs().max() <= (2e-3 if dtype == torch.float16 else 2e-5) * expect.abs().max()
+
+
 @pytest.mark.parametrize("hs", [128, 64])
 def test_more_short_prompts_than_a_grid_row(isp, hs):
     """4200 sequences of up to 16 tokens: more than 65535 query rows, and few enough queries per group for the decode kernel."""

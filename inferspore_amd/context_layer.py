@@ -210,7 +210,7 @@ def context_decoder_layer(normed, residual, w, state, layer_id, next_norm_gamma,
                                                      w.qkv_bias, st.padding_offset, st.history, st.lengths,
                                                      rotary_dim, rotary_base)
     if _fused_attention(st):
-        ops._expect(st.context.shape[0] == st.k_cache.shape[1], "batch extents differ")
+        ops._expect(st.context.shape[0] == st.batch, "batch extents differ")
         ops.context_attention(st.q, st.k_cache, st.v_cache, layer_id, st.history, st.lengths, st.context, st.max_k_len,
                               st.packed_ctx)
         if isinstance(st, BatchState):

@@ -305,12 +305,13 @@ def context_attention_supports(dtype, head_size):
 def context_attention_takes(q_buf, k_cache, v_cache, out):
     """Whether context_attention takes these operands: heads that it supports, extents that its grids hold, 16-byte aligned buffers,
     and an output that does not lie in the queries' memory (workgroups still read queries while others write)."""
-    if not context_attention_supports(q_buf.dtype, q_buf.shape[-1]) or q_buf.shape[0] > 65535 or q_buf.shape[2] > 65535 * 16:
+    batch, _, max_q_len, head_size = q_buf.shape
+    if not context_attention_supports(q_buf.dtype, head_size) or batch > 65535 or max_q_len > 65535 * 16:
         return False
     q, o = q_buf.data_ptr(), out.data_ptr()
     if (q | o | k_cache.data_ptr() | v_cache.data_ptr()) % 16:
         return False
-    return o >= q + q_buf.numel() * q_buf.element_size() or q >= o + out.numel() * out.element_size()
+    return o - q >= q_buf.nbytes if o >= q else q - o >= out.nbytes
 
 
 def context_attention(q_buf, k_cache, v_cache, layer_id, history_length, input_length, context_length, max_k_len, out,
@@ -323,27 +324,28 @@ def context_attention(q_buf, k_cache, v_cache, layer_id, history_length, input_l
             "attention takes q [batch, heads, max_q_len, head_size], caches [layers, batch, kv_heads, max_seq_len, head_size] "
             "and out [tokens, heads, head_size]")
     batch, head_num, max_q_len, head_size = q_buf.shape
-    kv_head_num, max_seq_len = k_cache.shape[2], k_cache.shape[3]
-    _expect(k_cache.shape == v_cache.shape and k_cache.shape[1] == batch and k_cache.shape[4] == head_size,
+    cache, (token_num, out_heads, out_size) = k_cache.shape, out.shape
+    layers, cache_batch, kv_head_num, max_seq_len, cache_size = cache
+    _expect(cache == v_cache.shape and cache_batch == batch and cache_size == head_size,
             "caches must be [layers, batch, kv_head_num, max_seq_len, head_size]")
     _expect(context_attention_supports(q_buf.dtype, head_size), "attention takes float16 or float32 heads of 64, 96 or 128 elements")
     _expect(kv_head_num > 0 and head_num % kv_head_num == 0, "head_num must be a multiple of kv_head_num")
-    _expect(out.shape[1:] == (head_num, head_size), "out must be [tokens, heads, head_size]")
-    _expect(0 <= int(layer_id) < k_cache.shape[0], "layer_id outside the cache")
+    _expect(out_heads == head_num and out_size == head_size, "out must be [tokens, heads, head_size]")
+    _expect(0 <= int(layer_id) < layers, "layer_id outside the cache")
     _expect(min(history_length.numel(), input_length.numel(), context_length.numel()) >= batch,
             "length tensors are shorter than the batch")
     _dev(q_buf, k_cache, v_cache, history_length, input_length, context_length, out)
     if q_buf.dtype == torch.float32:
         capi.check(capi.lib().isp_context_attention_f32(
             _p(q_buf), _p(k_cache), _p(v_cache), _p(out), _p(history_length), _p(input_length), _p(context_length),
-            int(layer_id), batch, head_num, kv_head_num, head_size, max_q_len, int(max_k_len), max_seq_len, out.shape[0],
+            int(layer_id), batch, head_num, kv_head_num, head_size, max_q_len, int(max_k_len), max_seq_len, token_num,
             float(head_size ** -0.5 if scale is None else scale), _stream()), "isp_context_attention")
         return out
     need = capi.lib().isp_context_attention_f16_workspace(batch, head_num, kv_head_num, head_size, max_q_len, int(max_k_len))
     workspace = torch.empty(need, dtype=torch.uint8, device=q_buf.device) if need else None
     capi.check(capi.lib().isp_context_attention_split_f16(
         _p(q_buf), _p(k_cache), _p(v_cache), _p(out), _p(history_length), _p(input_length), _p(context_length),
-        int(layer_id), batch, head_num, kv_head_num, head_size, max_q_len, int(max_k_len), max_seq_len, out.shape[0],
+        int(layer_id), batch, head_num, kv_head_num, head_size, max_q_len, int(max_k_len), max_seq_len, token_num,
         float(head_size ** -0.5 if scale is None else scale), _p(workspace), _stream()), "isp_context_attention")
     return out
 

@@ -106,8 +106,9 @@ class BatchState:
         missing = [name for name in ("k_all", "v_all") if name not in self.__dict__]
         for name in missing:
             self.__dict__[name] = torch.zeros(shape, dtype=self.q.dtype, device=self.q.device)
-        if missing and self._attended is not None:
-            ops.repeat_kv_cache(self.k_cache, self.v_cache, self.context, self._attended, self.k_all, self.v_all)
+        attended = self.__dict__.get("_attended")   # missing in a state saved before layers left a note
+        if missing and attended is not None:
+            ops.repeat_kv_cache(self.k_cache, self.v_cache, self.context, attended, self.k_all, self.v_all)
         if "mask" not in self.__dict__:
             self.mask = self._build_mask()
 
@@ -140,6 +141,7 @@ def _fused_attention(st):
     program's own cache, say), nor where a program has set or asked for the padded form's mask or buffers."""
     if not ops.context_attention_takes(st.q, st.k_cache, st.v_cache, st.packed_ctx) or hasattr(type(st), "mask"):
         return False
+    # a program's own state object has the mask that the padded form needs, or was made for this one
     return _PADDED.isdisjoint(st.__dict__) if isinstance(st, BatchState) else not hasattr(st, "mask")
 
 
@@ -147,6 +149,8 @@ def _layer_in_one_call(normed, residual, w, st, layer_id, gamma, rotary_dim, rot
     """The whole layer as one call of the C ABI, or None where it is not the plain case of a few float16 rows: everything
     that the steps below accept or refuse otherwise stays with them."""
     if normed.dtype != torch.float16 or normed.dim() != 2 or not 0 < normed.shape[0] <= 64:
+        return None
+    if not isinstance(st, BatchState) and hasattr(st, "mask"):   # a program's own state: it may have nothing else of what follows
         return None
     (tokens, hidden), batch, heads, kv, hs = normed.shape, st.batch, st.head_num, st.kv_head_num, st.head_size
     inter, width, max_seq = st.act.shape[-1], (heads + 2 * kv) * hs, st.k_cache.shape[3]
@@ -210,7 +214,7 @@ def context_decoder_layer(normed, residual, w, state, layer_id, next_norm_gamma,
                                                      w.qkv_bias, st.padding_offset, st.history, st.lengths,
                                                      rotary_dim, rotary_base)
     if _fused_attention(st):
-        ops._expect(st.context.shape[0] == st.batch, "batch extents differ")
+        ops._expect(st.context.shape[0] == st.q.shape[0], "batch extents differ")
         ops.context_attention(st.q, st.k_cache, st.v_cache, layer_id, st.history, st.lengths, st.context, st.max_k_len,
                               st.packed_ctx)
         if isinstance(st, BatchState):

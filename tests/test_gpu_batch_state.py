@@ -156,3 +156,33 @@ def test_other_batches_build_no_padded_buffers(isp, lens, history):
     from inferspore_amd import context_layer as cl
     st = cl.BatchState(lens, max(lens), 8, 2, 64, 32, max(lens) + history, 1, torch.float16, history=[history] * len(lens))
     assert "k_all" not in st.__dict__ and "mask" not in st.__dict__
+
+
+@pytest.mark.parametrize("rows", ["few", "many"])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+def test_a_programs_own_state_object(isp, dtype, rows):
+    """An object with the attributes that the steps of a layer read, and no others."""
+    from types import SimpleNamespace
+    from inferspore_amd import context_layer as cl
+    lens = LENS[rows]
+    st = cl.BatchState(lens, max(lens), HEADS, KV, HS, INTER, 64, 1, dtype)
+    names = ("tokens", "head_num", "kv_head_num", "head_size", "q", "k_cache", "v_cache", "padding_offset", "history", "lengths",
+             "context", "packed_ctx", "act", "k_all", "v_all", "mask")
+    own = SimpleNamespace(**{n: getattr(st, n) for n in names})
+    g = torch.Generator(device="cuda").manual_seed(9)
+    w = cl.LayerWeights(HIDDEN, INTER, dtype, generator=g)
+    w.qkv = w.qkv[:, :(HEADS + 2 * KV) * HS].contiguous()
+    x = torch.randn(sum(lens), HIDDEN, device="cuda", generator=g).to(dtype)
+    out = cl.context_decoder_layer(x, x.clone(), w, own, 0, w.attn_norm, rotary_dim=HS)
+    expect = attention64(own, lens, None)
+    assert torch.isfinite(out).all()
+    assert (own.packed_ctx.double() - expect).abs().max() <= (2e-3 if dtype == torch.float16 else 2e-5) * expect.abs().max()
+
+
+def test_a_state_saved_before(isp):
+    """A copy without what a layer notes in it still builds its buffers."""
+    import copy
+    from inferspore_amd import context_layer as cl
+    st = copy.copy(cl.BatchState([3, 2], 3, HEADS, KV, HS, INTER, 8, 1, torch.float16))
+    del st.__dict__["_attended"]
+    assert st.mask.shape == (2, 1, 3, 3) and not st.k_all.any()

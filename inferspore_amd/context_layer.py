@@ -136,21 +136,24 @@ class BatchState:
         return mask
 
 
+def _padded_asked(st):
+    """Whether a program has set or asked for the padded form's mask or buffers.  Its own state object has the mask that the padded
+    form needs, or was made for the fused one."""
+    if not isinstance(st, BatchState):
+        return hasattr(st, "mask")
+    return not _PADDED.isdisjoint(st.__dict__) or hasattr(type(st), "mask")
+
+
 def _fused_attention(st):
     """Whether a layer's attention is the fused kernel's: not where that does not take the state's buffers (an unaligned view in a
-    program's own cache, say), nor where a program has set or asked for the padded form's mask or buffers."""
-    if not ops.context_attention_takes(st.q, st.k_cache, st.v_cache, st.packed_ctx) or hasattr(type(st), "mask"):
-        return False
-    # a program's own state object has the mask that the padded form needs, or was made for this one
-    return _PADDED.isdisjoint(st.__dict__) if isinstance(st, BatchState) else not hasattr(st, "mask")
+    program's own cache, say), nor where a program has asked for the padded form."""
+    return not _padded_asked(st) and ops.context_attention_takes(st.q, st.k_cache, st.v_cache, st.packed_ctx)
 
 
 def _layer_in_one_call(normed, residual, w, st, layer_id, gamma, rotary_dim, rotary_base, eps):
     """The whole layer as one call of the C ABI, or None where it is not the plain case of a few float16 rows: everything
     that the steps below accept or refuse otherwise stays with them."""
-    if normed.dtype != torch.float16 or normed.dim() != 2 or not 0 < normed.shape[0] <= 64:
-        return None
-    if not isinstance(st, BatchState) and hasattr(st, "mask"):   # a program's own state: it may have nothing else of what follows
+    if normed.dtype != torch.float16 or normed.dim() != 2 or not 0 < normed.shape[0] <= 64 or _padded_asked(st):
         return None
     (tokens, hidden), batch, heads, kv, hs = normed.shape, st.batch, st.head_num, st.kv_head_num, st.head_size
     inter, width, max_seq = st.act.shape[-1], (heads + 2 * kv) * hs, st.k_cache.shape[3]
@@ -175,7 +178,7 @@ def _layer_in_one_call(normed, residual, w, st, layer_id, gamma, rotary_dim, rot
     if not (st.tokens == tokens and st.context.shape[0] == batch and 0 <= int(layer_id) < st.k_cache.shape[0] and
             0 <= int(rotary_dim) <= hs and int(rotary_dim) % 2 == 0) or normed.data_ptr() == residual.data_ptr():
         return None
-    if not _fused_attention(st):
+    if not ops.apart(st.q, st.packed_ctx):
         return None
     lib = capi.lib()
     need = lib.isp_context_layer_f16_workspace(batch, tokens, hidden, heads, kv, hs, st.max_q_len, st.max_k_len, max_seq, inter)

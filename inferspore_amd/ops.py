@@ -302,16 +302,21 @@ def context_attention_supports(dtype, head_size):
     return head_size in (64, 96, 128) and dtype in (torch.float16, torch.float32)
 
 
+def apart(a, b):
+    """Whether two contiguous tensors share no memory."""
+    p, q = a.data_ptr(), b.data_ptr()
+    return q - p >= a.nbytes if q >= p else p - q >= b.nbytes
+
+
 def context_attention_takes(q_buf, k_cache, v_cache, out):
     """Whether context_attention takes these operands: heads that it supports, extents that its grids hold, 16-byte aligned buffers,
     and an output that does not lie in the queries' memory (workgroups still read queries while others write)."""
     batch, _, max_q_len, head_size = q_buf.shape
     if not context_attention_supports(q_buf.dtype, head_size) or batch > 65535 or max_q_len > 65535 * 16:
         return False
-    q, o = q_buf.data_ptr(), out.data_ptr()
-    if (q | o | k_cache.data_ptr() | v_cache.data_ptr()) % 16:
+    if (q_buf.data_ptr() | out.data_ptr() | k_cache.data_ptr() | v_cache.data_ptr()) % 16:
         return False
-    return o - q >= q_buf.nbytes if o >= q else q - o >= out.nbytes
+    return apart(q_buf, out)
 
 
 def context_attention(q_buf, k_cache, v_cache, layer_id, history_length, input_length, context_length, max_k_len, out,

@@ -111,7 +111,8 @@ def test_a_context_of_no_keys_gives_zeros(isp, dtype, hs, lens, heads):
     k, v = (torch.randn(1, batch, heads, max_seq, hs, generator=g).to(dtype) for _ in range(2))
     ints = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")   # noqa: E731
     out = torch.full((sum(lens), heads, hs), float("nan"), dtype=dtype, device="cuda")
-    isp.context_attention(q.cuda(), k.cuda(), v.cuda(), 0, ints(hist), ints(lens), ints([max_seq, 0] + [max_seq] * (batch - 2)), max_seq, out)
+    context = [max_seq, 0] + [max_seq] * (batch - 2)
+    isp.context_attention(q.cuda(), k.cuda(), v.cuda(), 0, ints(hist), ints(lens), ints(context), max_seq, out)
     first = lens[0]
     assert not out[first:first + lens[1]].any()
     rest = [0, batch - 1]
@@ -139,7 +140,8 @@ def test_more_short_prompts_than_a_grid_row(isp, hs):
     assert (got - expect).abs().max() <= 2e-3 * expect.abs().max()
 
 
-@pytest.mark.parametrize("lens,hist,heads,kv,max_seq", [([300, 77], [0, 0], 16, 2, 320), ([65, 130], [900, 30], 32, 8, 1000), ([24], [3000], 2, 2, 3100)])
+@pytest.mark.parametrize("lens,hist,heads,kv,max_seq", [([300, 77], [0, 0], 16, 2, 320), ([65, 130], [900, 30], 32, 8, 1000),
+                                                          ([24], [3000], 2, 2, 3100)])
 def test_float16_heads_of_96_keep_their_probabilities(isp, lens, hist, heads, kv, max_seq):
     """The probabilities of 96-element heads are not rounded to fp16 (two halves, 21 bits): the error is the result's own rounding, 2^-11,
     and 2e-5 of the largest output for the scores, as in float32."""

@@ -18,9 +18,9 @@ order a model runs them:
     ffn_out  = act @ Wdown                                   product
     residual, normed_next = fused_add_bias_residual_rmsnorm(residual, ffn_out, next attn_norm)   * this library
 
-Products of more than 64 rows, and those in float32, are left to torch's library calls (hipBLASLt GEMMs), those of up to 64 float16
-rows go to ops.linear, and a layer of such rows is one call of the C ABI (isp_context_layer_f16); everything marked * goes
-through the C ABI.  All work is issued on torch's current stream.
+A layer of float16 rows is one call of the C ABI (isp_context_layer_rows_f16), products included.  Where a layer runs step by step (a mask of
+its own, unaligned buffers, gradients, float32), products of up to 64 float16 rows go to ops.linear and the others to torch's library
+calls (hipBLASLt GEMMs); everything marked * goes through the C ABI.  All work is issued on torch's current stream.
 """
 import math
 
@@ -151,9 +151,9 @@ def _fused_attention(st):
 
 
 def _layer_in_one_call(normed, residual, w, st, layer_id, gamma, rotary_dim, rotary_base, eps):
-    """The whole layer as one call of the C ABI, or None where it is not the plain case of a few float16 rows: everything
+    """The whole layer as one call of the C ABI, or None where it is not the plain case of float16 rows: everything
     that the steps below accept or refuse otherwise stays with them."""
-    if normed.dtype != torch.float16 or normed.dim() != 2 or not 0 < normed.shape[0] <= 64 or _padded_asked(st):
+    if normed.dtype != torch.float16 or normed.dim() != 2 or normed.shape[0] == 0 or _padded_asked(st):
         return None
     (tokens, hidden), batch, heads, kv, hs = normed.shape, st.batch, st.head_num, st.kv_head_num, st.head_size
     inter, width, max_seq = st.act.shape[-1], (heads + 2 * kv) * hs, st.k_cache.shape[3]
@@ -181,13 +181,13 @@ def _layer_in_one_call(normed, residual, w, st, layer_id, gamma, rotary_dim, rot
     if not ops.apart(st.q, st.packed_ctx):
         return None
     lib = capi.lib()
-    need = lib.isp_context_layer_f16_workspace(batch, tokens, hidden, heads, kv, hs, st.max_q_len, st.max_k_len, max_seq, inter)
+    need = lib.isp_context_layer_rows_f16_workspace(batch, tokens, hidden, heads, kv, hs, st.max_q_len, st.max_k_len, max_seq, inter)
     if need == 0:
         return None
     workspace = torch.empty(need, dtype=torch.uint8, device=device)
     out = torch.empty_like(normed)
     p = torch.Tensor.data_ptr
-    capi.check(lib.isp_context_layer_f16(
+    capi.check(lib.isp_context_layer_rows_f16(
         p(normed), p(residual), p(out), p(w.qkv), None if w.qkv_bias is None else p(w.qkv_bias), p(w.o), p(w.gate_up),
         p(w.down), p(w.ffn_norm), p(gamma), p(st.q), p(st.k_cache), p(st.v_cache), p(st.packed_ctx), p(st.act),
         p(st.padding_offset), p(st.history), p(st.lengths), p(st.context), p(workspace), int(layer_id), batch, tokens, hidden,

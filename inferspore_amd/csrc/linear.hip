@@ -1,7 +1,8 @@
-// isp_linear_f16: the product of a few activation rows with a weight matrix (see linear_rows.h for the kernel).
+// isp_linear_rows_f16: the product of activation rows with a weight matrix, up to 16 rows by the kernel in linear_rows.h, more by the tiles in
+// linear_tiled.h; isp_linear_f16: up to 64 of them.
 // The reference calls cuBLAS for it (src/kernels/linear.cu:7-66); the library here, hipBLASLt, reads the weights of a
-// 16-row product at 1.4-3.8 TB/s and those of a 64-row product at 1.2-1.8 (4.9 for the widest), this kernel at 4.3-5.5
-// and 3.0-4.7.
+// 16-row product at 1.4-3.8 TB/s and those of a 64-row product at 1.2-1.8 (4.9 for the widest), these kernels at 4.3-5.5
+// and 3.1-5.4.
 #include "linear_rows.h"
 
 namespace isp {
@@ -36,28 +37,31 @@ __global__ __launch_bounds__(kBlock) void linear_add_splits(const float* __restr
     reinterpret_cast<uint2*>(out)[i] = make_uint2(*reinterpret_cast<const uint32_t*>(&lo), *reinterpret_cast<const uint32_t*>(&hi));
 }
 
+// Extents that the kernels can count: a few rows, or any number of them (the addition below indexes four values in 32 bits).
+static bool linear_shape(int m, int n, int k) {
+    const int most = m <= kSkinnyMaxRows ? kSkinnyMaxExtent : kTiledMaxExtent;
+    return k > 0 && n % 8 == 0 && k % 8 == 0 && n <= most && k <= most && (long long)m * n < 0x3ffffff00ll;
+}
+
 static int linear(const __half* a, const __half* w, __half* out, float* workspace, int m, int n, int k, hipStream_t stream) {
     if (m < 0 || n < 0 || k < 0) return ISP_ERR_BAD_SHAPE;
     if (m == 0 || n == 0) return ISP_OK;
-    if (k == 0 || m > kSkinnyMaxRows || n % 8 != 0 || k % 8 != 0 || n > kSkinnyMaxExtent || k > kSkinnyMaxExtent)
-        return ISP_ERR_UNSUPPORTED;
+    if (!linear_shape(m, n, k)) return ISP_ERR_UNSUPPORTED;
     ISP_REQUIRE_PTR(a);
     ISP_REQUIRE_PTR(w);
     ISP_REQUIRE_PTR(out);
     if (!aligned16(a) || !aligned16(w) || !aligned16(out)) return ISP_ERR_UNSUPPORTED;
-    const SkinnyPlan plan = skinny_plan(m, n, k);
-    if (plan.splits == 1) {
-        launch_skinny(plan, a, w, out, nullptr, m, n, k, stream);
-        return note_launch(hipGetLastError());
+    const ProductPlan plan = product_plan(m, n, k);
+    if (plan.splits() > 1) {
+        ISP_REQUIRE_PTR(workspace);
+        if (!aligned16(workspace)) return ISP_ERR_UNSUPPORTED;
     }
-    ISP_REQUIRE_PTR(workspace);
-    if (!aligned16(workspace)) return ISP_ERR_UNSUPPORTED;
-    launch_skinny(plan, a, w, nullptr, workspace, m, n, k, stream);
+    launch_product(plan, a, w, out, workspace, m, n, k, stream);
     const int status = note_launch(hipGetLastError());
-    if (status != ISP_OK) return status;
+    if (status != ISP_OK || plan.splits() == 1) return status;
     const unsigned quads = (unsigned)((size_t)m * (size_t)n / 4);
     hipLaunchKernelGGL(linear_add_splits, dim3((quads + kBlock - 1) / kBlock), dim3(kBlock), 0, stream, workspace, out, quads,
-                       plan.splits);
+                       plan.splits());
     return note_launch(hipGetLastError());
 }
 
@@ -65,15 +69,34 @@ static int linear(const __half* a, const __half* w, __half* out, float* workspac
 
 extern "C" {
 
+size_t isp_linear_rows_f16_workspace(int m, int n, int k) {
+    if (m <= 0 || n <= 0 || k <= 0 || !isp::linear_shape(m, n, k)) return 0;
+    const isp::ProductPlan plan = isp::product_plan(m, n, k);
+    return plan.splits() == 1 ? 0 : plan.bytes(m, n);
+}
+
+int isp_linear_rows_f16(const void* a, const void* w, void* out, void* workspace, int m, int n, int k, isp_stream_t stream) {
+    return isp::linear(static_cast<const __half*>(a), static_cast<const __half*>(w), static_cast<__half*>(out),
+                       static_cast<float*>(workspace), m, n, k, static_cast<hipStream_t>(stream));
+}
+
+int isp_linear_rows_f16_plan(int m, int n, int k, int* tile_rows, int* tile_cols, int* splits) {
+    if (m <= 0 || n <= 0 || k <= 0 || !isp::linear_shape(m, n, k)) return ISP_ERR_BAD_SHAPE;
+    const isp::ProductPlan plan = isp::product_plan(m, n, k);
+    *tile_rows = *tile_cols = 0;
+    if (plan.tiled) isp::tiled_extents(plan.tile, tile_rows, tile_cols);
+    *splits = plan.splits();
+    return ISP_OK;
+}
+
 size_t isp_linear_f16_workspace(int m, int n, int k) {
-    if (m <= 0 || n <= 0 || k <= 0 || m > isp::kSkinnyMaxRows || n > isp::kSkinnyMaxExtent || k > isp::kSkinnyMaxExtent) return 0;
-    const isp::SkinnyPlan plan = isp::skinny_plan(m, n, k);
-    return plan.splits == 1 ? 0 : plan.partial_floats(m, n) * sizeof(float);
+    if (m > isp::kSkinnyMaxRows) return 0;
+    return isp_linear_rows_f16_workspace(m, n, k);
 }
 
 int isp_linear_f16(const void* a, const void* w, void* out, void* workspace, int m, int n, int k, isp_stream_t stream) {
-    return isp::linear(static_cast<const __half*>(a), static_cast<const __half*>(w), static_cast<__half*>(out),
-                       static_cast<float*>(workspace), m, n, k, static_cast<hipStream_t>(stream));
+    if (m > isp::kSkinnyMaxRows && n > 0 && k >= 0) return ISP_ERR_UNSUPPORTED;
+    return isp_linear_rows_f16(a, w, out, workspace, m, n, k, stream);
 }
 
 }  // extern "C"

@@ -178,6 +178,47 @@ inline SkinnyPlan skinny_plan(int m, int n, int k) {
 void launch_skinny(const SkinnyPlan& plan, const __half* a, const __half* w, __half* out, float* partial, int m, int n, int k,
                    hipStream_t stream);
 
+// Products of more rows (linear_tiled.h): which of the tiles, and how many workgroups share a tile's k.
+struct TiledPlan {
+    int tile, splits, steps_per_split;
+};
+TiledPlan tiled_plan(int m, int n, int k, int max_splits);
+void tiled_extents(const TiledPlan& plan, int* rows, int* cols);
+constexpr int kTiledMaxSplits = 16;
+constexpr int kTiledMaxExtent = 1 << 22;  // of n and k: a tile's rows of A and of W are addressed in 32 bits
+// With plan.splits > 1 partial sums to `partial`, else the fp16 product to `out`.  Operands checked by the caller.
+void launch_tiled(const TiledPlan& plan, const __half* a, const __half* w, __half* out, float* partial, int m, int n, int k,
+                  hipStream_t stream);
+// out[m, inter] = SwiGLU of the product with gate_up [k, 2 inter]; a plan without splits
+void launch_tiled_swiglu(const TiledPlan& plan, const __half* a, const __half* gate_up, __half* out, int m, int inter, int k,
+                         hipStream_t stream);
+
+// Either, for the rows that it is made for.  A skinny product's sums end in the order of its wavefronts, a tiled one's in the order of k.
+struct ProductPlan {
+    bool tiled;
+    SkinnyPlan skinny;
+    TiledPlan tile;
+    int splits() const { return tiled ? tile.splits : skinny.splits; }
+    // what the product leaves for its consumer: fp16, or the splits' partial sums
+    size_t bytes(int m, int n) const {
+        const size_t values = (size_t)m * (size_t)n;
+        return splits() == 1 ? values * sizeof(__half) : (size_t)splits() * values * sizeof(float);
+    }
+};
+constexpr int kSkinnyRows = 16;  // up to here
+inline ProductPlan product_plan(int m, int n, int k, int max_splits = kTiledMaxSplits) {
+    ProductPlan p = {m > kSkinnyRows, {}, {}};
+    if (p.tiled) p.tile = tiled_plan(m, n, k, max_splits);
+    else p.skinny = skinny_plan(m, n, k);
+    return p;
+}
+// With several splits their sums to `partial`, else the fp16 product to `out`.
+inline void launch_product(const ProductPlan& plan, const __half* a, const __half* w, __half* out, float* partial, int m, int n, int k,
+                           hipStream_t stream) {
+    if (plan.tiled) launch_tiled(plan.tile, a, w, out, partial, m, n, k, stream);
+    else launch_skinny(plan.skinny, a, w, plan.skinny.splits == 1 ? out : nullptr, partial, m, n, k, stream);
+}
+
 // Eight neighbouring columns of a product left as partial sums: the splits added in their order and rounded to fp16 once, the
 // value linear_add_splits would have stored.  `stride`: floats between two splits.
 __device__ __forceinline__ vec16 add_splits8(const float* p, size_t stride, int splits) {

@@ -9,23 +9,6 @@
 
 namespace isp {
 
-__device__ __forceinline__ float silu_exact(float x) { return x / (1.0f + expf(-x)); }
-
-// exp through the hardware exp2 and a hardware reciprocal: relative error of a few 1e-7, three
-// orders of magnitude below half an fp16 ulp, so the rounded fp16 result matches the exact form
-// except on rounding ties.
-__device__ __forceinline__ float silu_fast(float x) {
-    const float e = __builtin_amdgcn_exp2f(-1.4426950408889634f * x);
-    return x * __builtin_amdgcn_rcpf(1.0f + e);
-}
-
-template <typename T>
-__device__ __forceinline__ float silu_for(float x);
-template <>
-__device__ __forceinline__ float silu_for<float>(float x) { return silu_exact(x); }
-template <>
-__device__ __forceinline__ float silu_for<__half>(float x) { return silu_fast(x); }
-
 // Single-wave workgroups: 80.8 against 83.2 us with 256 threads at 8192 x 11008 fp16, equal from 2977 rows down.
 template <typename T, int UNROLL, int ST>
 __global__ __launch_bounds__(kWave) void swiglu_vec(const T* __restrict__ in, T* __restrict__ out,

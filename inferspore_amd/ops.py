@@ -269,12 +269,7 @@ def transpose_out_remove_padding(qkv_buf_w_pad, padding_offset, qkv_buf_wo_pad):
 
 
 def linear_supports(x, w):
-    """Whether linear() takes this product: a few contiguous float16 rows outside autograd.  Above 32768 columns more
-    than one round of workgroups is needed, and from 17 rows on the library is faster there (5120 x 40928: 37 rows 88
-    against 112 us, 64 rows 85 against 124; 8 rows 80 against 85).  By itself the kernel is level with the library from 17 rows and
-    20480 columns on where its strips do not fill the compute units (4096 x 22016, 32 rows 43 against 40 us, 64 rows 47 against 45;
-    x 28672 42 against 46, 49 against 49); in a layer, whose other products and additions run around it, it stays
-    ahead (64 rows, gate / up of 22016 columns: 164 us a layer, 169 with the library there; 28672: 171 and 180)."""
+    """Whether linear() takes this product: up to 64 contiguous float16 rows outside autograd, above 16 rows up to 32768 columns."""
     return (x.dtype == torch.float16 and w.dtype == torch.float16 and x.dim() == 2 and w.dim() == 2 and x.is_cuda and
             0 < x.shape[0] <= 64 and (x.shape[0] <= 16 or w.shape[1] <= 32768) and x.shape[1] == w.shape[0] and w.device == x.device and
             w.shape[0] % 8 == 0 and w.shape[1] % 8 == 0 and w.numel() > 0 and max(w.shape) <= 1 << 24 and

@@ -312,6 +312,10 @@ int isp_linear_rows_f16(const void* a, const void* w, void* out, void* workspace
 /* The tile of a workgroup (0 x 0: the kernel for up to 16 rows, whose workgroups take 128 columns) and the number of workgroups that
  * share its k. */
 int isp_linear_rows_f16_plan(int m, int n, int k, int* tile_rows, int* tile_cols, int* splits);
+/* The same in fp32 throughout: n and k multiples of 4 up to 2^22. */
+size_t isp_linear_rows_f32_workspace(int m, int n, int k);
+int isp_linear_rows_f32(const void* a, const void* w, void* out, void* workspace, int m, int n, int k, isp_stream_t stream);
+int isp_linear_rows_f32_plan(int m, int n, int k, int* tile_rows, int* tile_cols, int* splits);
 
 /*
  * A whole context-decoder layer for up to 64 packed fp16 rows (a decode step, a short prompt) in one call: QKV product,
@@ -340,6 +344,16 @@ int isp_context_layer_f16(const void* normed, void* residual, void* out, const v
 size_t isp_context_layer_rows_f16_workspace(int batch, int token_num, int hidden, int head_num, int kv_head_num, int head_size,
                                             int max_q_len, int max_k_len, int max_seq_len, int inter);
 int isp_context_layer_rows_f16(const void* normed, void* residual, void* out, const void* qkv_weight, const void* qkv_bias,
+                               const void* o_weight, const void* gate_up_weight, const void* down_weight, const void* ffn_norm,
+                               const void* next_norm, void* q, void* k_cache, void* v_cache, void* context, void* act,
+                               const int32_t* padding_offset, const int32_t* history_length, const int32_t* input_length,
+                               const int32_t* context_length, void* workspace, int layer, int batch, int token_num, int hidden,
+                               int head_num, int kv_head_num, int head_size, int max_q_len, int max_k_len, int max_seq_len, int inter,
+                               int rotary_dim, float rotary_base, float eps, isp_stream_t stream);
+/* The same in fp32 throughout, hidden and inter multiples of 4. */
+size_t isp_context_layer_rows_f32_workspace(int batch, int token_num, int hidden, int head_num, int kv_head_num, int head_size,
+                                            int max_q_len, int max_k_len, int max_seq_len, int inter);
+int isp_context_layer_rows_f32(const void* normed, void* residual, void* out, const void* qkv_weight, const void* qkv_bias,
                                const void* o_weight, const void* gate_up_weight, const void* down_weight, const void* ffn_norm,
                                const void* next_norm, void* q, void* k_cache, void* v_cache, void* context, void* act,
                                const int32_t* padding_offset, const int32_t* history_length, const int32_t* input_length,

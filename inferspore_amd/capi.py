@@ -56,10 +56,15 @@ SIGNATURES = {
     "isp_linear_rows_f16_workspace": (C.c_size_t, [_i, _i, _i]),
     "isp_linear_rows_f16": (_i, [_vp] * 4 + [_i] * 3 + [_vp]),
     "isp_linear_rows_f16_plan": (_i, [_i] * 3 + [C.POINTER(C.c_int)] * 3),
+    "isp_linear_rows_f32_workspace": (C.c_size_t, [_i, _i, _i]),
+    "isp_linear_rows_f32": (_i, [_vp] * 4 + [_i] * 3 + [_vp]),
+    "isp_linear_rows_f32_plan": (_i, [_i] * 3 + [C.POINTER(C.c_int)] * 3),
     "isp_context_layer_f16_workspace": (C.c_size_t, [_i] * 10),
     "isp_context_layer_f16": (_i, [_vp] * 20 + [_i] * 12 + [_f, _f, _vp]),
     "isp_context_layer_rows_f16_workspace": (C.c_size_t, [_i] * 10),
     "isp_context_layer_rows_f16": (_i, [_vp] * 20 + [_i] * 12 + [_f, _f, _vp]),
+    "isp_context_layer_rows_f32_workspace": (C.c_size_t, [_i] * 10),
+    "isp_context_layer_rows_f32": (_i, [_vp] * 20 + [_i] * 12 + [_f, _f, _vp]),
     "isp_tuning_set": (_i, [_i, _i]),
     "isp_calibration_copy": (_i, [_vp, _vp, C.c_size_t, _vp]),
     "isp_norm_launch_config": (_i, [_i, _i, _i, _i] + [C.POINTER(C.c_int)] * 4),

@@ -1,4 +1,5 @@
-// isp_context_layer_rows_f16: a whole context-decoder layer of packed fp16 rows in one call (isp_context_layer_f16: up to 64 of them).
+// isp_context_layer_rows_f16: a whole context-decoder layer of packed fp16 rows in one call (isp_context_layer_f16: up to 64 of them);
+// isp_context_layer_rows_f32: of fp32 rows.
 // Seven to ten launches.  A product whose k is split over workgroups leaves fp32 partial sums, and the step that follows adds them where it
 // would have read the product -- QKV bias + RoPE + KV append, residual + RMSNorm (twice), SwiGLU; a gate / up product that is not
 // split computes SwiGLU itself.  As separate calls a layer
@@ -35,16 +36,16 @@ static LayerPlans layer_plans(int batch, int tokens, int hidden, int head_num, i
     return p;
 }
 
-// ISP_OK where the layer runs here.
+// ISP_OK where the layer runs here.  `vector`: elements of 16 bytes, of which rows are whole numbers.
 static int layer_shape(int layer, int batch, int tokens, int hidden, int head_num, int kv_head_num, int head_size, int max_q_len,
-                       int max_k_len, int max_seq_len, int inter, int rotary_dim) {
+                       int max_k_len, int max_seq_len, int inter, int rotary_dim, int vector = 8) {
     if (layer < 0 || batch <= 0 || tokens <= 0 || hidden <= 0 || head_num <= 0 || kv_head_num <= 0 || head_size <= 0 ||
         max_q_len <= 0 || max_k_len <= 0 || max_seq_len <= 0 || inter <= 0 || rotary_dim < 0 || head_num % kv_head_num != 0 ||
         rotary_dim % 2 != 0 || rotary_dim > head_size)
         return ISP_ERR_BAD_SHAPE;
     const long long widest = ((long long)head_num + 2ll * kv_head_num) * head_size;
-    const int most = tokens <= kSkinnyMaxRows ? kSkinnyMaxExtent : kTiledMaxExtent;
-    if ((head_size != 64 && head_size != 96 && head_size != 128) || hidden % 8 != 0 || inter % 8 != 0 || batch > 65535 ||
+    const int most = tokens <= kSkinnyMaxRows && vector == 8 ? kSkinnyMaxExtent : kTiledMaxExtent;
+    if ((head_size != 64 && head_size != 96 && head_size != 128) || hidden % vector != 0 || inter % vector != 0 || batch > 65535 ||
         max_q_len > 65535 * 16 || (long long)batch * max_q_len > 0x7fffffffll || hidden > most || inter > most || widest > most)
         return ISP_ERR_UNSUPPORTED;
     // the steps between the products index vectors of 16 bytes in 32 bits
@@ -133,6 +134,64 @@ static int context_layer(const void* normed, void* residual, void* out, const vo
     return layer_norm(plan.down, sums, residual, out, next_norm, eps, tokens, hidden, stream);
 }
 
+// The same steps in fp32: products, their additions of splits and the entry points of the other steps, on a workspace that holds the
+// wider of the two products stored on the way and, behind it, partial sums.  Nine to thirteen launches.
+struct LayerSpaceF32 {
+    size_t product, bytes;
+};
+static LayerSpaceF32 layer_space_f32(int tokens, int hidden, int head_num, int kv_head_num, int head_size, int inter) {
+    const int width = (head_num + 2 * kv_head_num) * head_size, ctx = head_num * head_size, widest = width > 2 * inter ? width : 2 * inter;
+    const int extents[][2] = {{width, hidden}, {hidden, ctx}, {2 * inter, hidden}, {hidden, inter}};
+    size_t sums = 0;
+    for (const auto& e : extents) {
+        const size_t need = isp_linear_rows_f32_workspace(tokens, e[0], e[1]);
+        sums = need > sums ? need : sums;
+    }
+    const size_t product = (size_t)tokens * (size_t)widest * sizeof(float);  // rows of whole 16 bytes
+    return {product, product + sums};
+}
+
+static int context_layer_f32(const void* normed, void* residual, void* out, const void* qkv_weight, const void* qkv_bias,
+                             const void* o_weight, const void* gate_up_weight, const void* down_weight, const void* ffn_norm,
+                             const void* next_norm, void* q, void* k_cache, void* v_cache, void* context, void* act,
+                             const int32_t* padding_offset, const int32_t* history_length, const int32_t* input_length,
+                             const int32_t* context_length, void* workspace, int layer, int batch, int tokens, int hidden, int head_num,
+                             int kv_head_num, int head_size, int max_q_len, int max_k_len, int max_seq_len, int inter, int rotary_dim,
+                             float rotary_base, float eps, hipStream_t stream) {
+    const void* needed[] = {normed, residual, out, qkv_weight, o_weight, gate_up_weight, down_weight, ffn_norm, next_norm,
+                            q, k_cache, v_cache, context, act, padding_offset, history_length, input_length, context_length, workspace};
+    for (const void* p : needed) ISP_REQUIRE_PTR(p);
+    const void* vectors[] = {normed, residual, out, qkv_weight, qkv_bias, o_weight, gate_up_weight, down_weight, ffn_norm,
+                             next_norm, q, k_cache, v_cache, context, act, workspace};
+    for (const void* p : vectors)
+        if (!aligned16(p)) return ISP_ERR_UNSUPPORTED;
+    const int width = (head_num + 2 * kv_head_num) * head_size, ctx = head_num * head_size;
+    void* product = workspace;
+    void* sums = static_cast<char*>(workspace) + layer_space_f32(tokens, hidden, head_num, kv_head_num, head_size, inter).product;
+
+    int status = isp_linear_rows_f32(normed, qkv_weight, product, sums, tokens, width, hidden, stream);
+    if (status != ISP_OK) return status;
+    status = isp_qkv_bias_rope_transpose_append_f32(q, nullptr, nullptr, k_cache, v_cache, layer, max_seq_len, product, qkv_bias,
+                                                    padding_offset, history_length, input_length, batch, max_q_len, tokens, head_num,
+                                                    kv_head_num, head_size, rotary_dim, rotary_base, stream);
+    if (status != ISP_OK) return status;
+    status = isp_context_attention_f32(q, k_cache, v_cache, context, history_length, input_length, context_length, layer, batch,
+                                       head_num, kv_head_num, head_size, max_q_len, max_k_len, max_seq_len, tokens,
+                                       (float)(1.0 / sqrt((double)head_size)), stream);
+    if (status != ISP_OK) return status;
+    status = isp_linear_rows_f32(context, o_weight, out, sums, tokens, hidden, ctx, stream);
+    if (status != ISP_OK) return status;
+    status = isp_fused_add_bias_residual_rmsnorm_f32(residual, out, nullptr, ffn_norm, eps, tokens, hidden, 0, stream);
+    if (status != ISP_OK) return status;
+    status = isp_linear_rows_f32(out, gate_up_weight, product, sums, tokens, 2 * inter, hidden, stream);
+    if (status != ISP_OK) return status;
+    status = isp_swiglu_f32(product, act, tokens, inter, stream);
+    if (status != ISP_OK) return status;
+    status = isp_linear_rows_f32(act, down_weight, out, sums, tokens, hidden, inter, stream);
+    if (status != ISP_OK) return status;
+    return isp_fused_add_bias_residual_rmsnorm_f32(residual, out, nullptr, next_norm, eps, tokens, hidden, 0, stream);
+}
+
 }  // namespace isp
 
 extern "C" {
@@ -184,6 +243,31 @@ int isp_context_layer_f16(const void* normed, void* residual, void* out, const v
                                       next_norm, q, k_cache, v_cache, context, act, padding_offset, history_length, input_length,
                                       context_length, workspace, layer, batch, token_num, hidden, head_num, kv_head_num, head_size,
                                       max_q_len, max_k_len, max_seq_len, inter, rotary_dim, rotary_base, eps, stream);
+}
+
+size_t isp_context_layer_rows_f32_workspace(int batch, int token_num, int hidden, int head_num, int kv_head_num, int head_size,
+                                            int max_q_len, int max_k_len, int max_seq_len, int inter) {
+    if (isp::layer_shape(0, batch, token_num, hidden, head_num, kv_head_num, head_size, max_q_len, max_k_len, max_seq_len, inter, 0,
+                         4) != ISP_OK)
+        return 0;
+    return isp::layer_space_f32(token_num, hidden, head_num, kv_head_num, head_size, inter).bytes;
+}
+
+int isp_context_layer_rows_f32(const void* normed, void* residual, void* out, const void* qkv_weight, const void* qkv_bias,
+                               const void* o_weight, const void* gate_up_weight, const void* down_weight, const void* ffn_norm,
+                               const void* next_norm, void* q, void* k_cache, void* v_cache, void* context, void* act,
+                               const int32_t* padding_offset, const int32_t* history_length, const int32_t* input_length,
+                               const int32_t* context_length, void* workspace, int layer, int batch, int token_num, int hidden,
+                               int head_num, int kv_head_num, int head_size, int max_q_len, int max_k_len, int max_seq_len, int inter,
+                               int rotary_dim, float rotary_base, float eps, isp_stream_t stream) {
+    const int shape = isp::layer_shape(layer, batch, token_num, hidden, head_num, kv_head_num, head_size, max_q_len, max_k_len,
+                                       max_seq_len, inter, rotary_dim, 4);
+    if (shape != ISP_OK) return shape;
+    return isp::context_layer_f32(normed, residual, out, qkv_weight, qkv_bias, o_weight, gate_up_weight, down_weight, ffn_norm,
+                                  next_norm, q, k_cache, v_cache, context, act, padding_offset, history_length, input_length,
+                                  context_length, workspace, layer, batch, token_num, hidden, head_num, kv_head_num, head_size,
+                                  max_q_len, max_k_len, max_seq_len, inter, rotary_dim, rotary_base, eps,
+                                  static_cast<hipStream_t>(stream));
 }
 
 }  // extern "C"

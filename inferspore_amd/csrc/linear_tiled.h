@@ -21,35 +21,13 @@
 // 12288 66, 54; 462 x 11008 x 4096 98, 49; 660 x 1024 x 3072 17.5, 11.2; 2610 x 4096 x 22016 487, 411; 6460 x 4096 x 22016 1062, 940.
 #pragma once
 
-#include <type_traits>
-
-#include "isp_common.h"
+#include "tile_loads.h"
 
 namespace isp {
 
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef _Float16 half4 __attribute__((ext_vector_type(4)));
-typedef float float4v __attribute__((ext_vector_type(4)));
 
-template <int N, int I = 0, typename F>
-__device__ __forceinline__ void static_for(F&& f) {
-    if constexpr (I < N) {
-        f(std::integral_constant<int, I>{});
-        static_for<N, I + 1>(f);
-    }
-}
-
-// 16 bytes per lane from base + off into LDS, lane i's to lds + 16 i.  An asm statement because the compiler would make every later
-// LDS read wait for all such loads; the kernel waits by itself (wait_loads).  Nothing is written but LDS: no register is in flight.
-// s_nop: M0 must not be written in the instruction right before.
-__device__ __forceinline__ void load_to_lds(uint32_t lds, const void* base, uint32_t off) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(lds), "v"(off), "s"(base) : "memory");
-}
-// until at most N of this wavefront's loads are outstanding (they arrive in order)
-template <int N>
-__device__ __forceinline__ void wait_loads() {
-    asm volatile("s_waitcnt vmcnt(%0)" : : "n"(N) : "memory");
-}
 __device__ __forceinline__ half4 lds_read_transposed(uint32_t at) {
     typedef short short4v __attribute__((ext_vector_type(4)));
     typedef __attribute__((address_space(3))) short4v* lds_ptr;
@@ -60,11 +38,6 @@ __device__ __forceinline__ half8 lds_read_row(uint32_t at) {
     typedef __attribute__((address_space(3))) const half8* lds_ptr;
     return *(lds_ptr)(uintptr_t)at;
 }
-__device__ __forceinline__ void lds_clear16(uint32_t at) {
-    typedef __attribute__((address_space(3))) float4v* lds_ptr;
-    *(lds_ptr)(uintptr_t)at = float4v{0.0f, 0.0f, 0.0f, 0.0f};
-}
-
 // What becomes of the sums: fp16 to `out`; fp32 to partial[split], for the consumer to add up; or, with W's columns [0, n / 2) gates and
 // [n / 2, n) up projections, SwiGLU of the two products rounded to fp16 -- what the separate kernel computes from the stored product, same
 // bits -- to `out` [m, n / 2].
@@ -92,16 +65,9 @@ __global__ __launch_bounds__(kWave* WAVES_M* WAVES_N, 2) void linear_tiled_f16(c
     const int tid = threadIdx.x, lane = tid % kWave, wave = __builtin_amdgcn_readfirstlane(tid / kWave), j = lane % 16, g = lane / 16;
     const int wm = wave / WAVES_N, wn = wave % WAVES_N;
 
-    // Workgroups are handed to the eight XCDs in turn; each XCD gets a contiguous run of tiles, four rows of tiles at a time, so that
-    // its L2 holds what its workgroups share.  (Eight rows of tiles: within 2 % of it either way.)
-    constexpr int kXcds = 8, kTileRows = 4;
     const int cols = RESULT == kTiledSwiglu ? BN / 2 : BN, width = RESULT == kTiledSwiglu ? n / 2 : n;  // result columns
-    const int rows_of_tiles = (m + BM - 1) / BM, cols_of_tiles = (width + cols - 1) / cols, tiles = rows_of_tiles * cols_of_tiles;
-    const int per_xcd = tiles / kXcds, xcd = (int)blockIdx.x % kXcds;
-    const int index = xcd * per_xcd + min(xcd, tiles % kXcds) + (int)blockIdx.x / kXcds;
-    const int band = index / (kTileRows * cols_of_tiles), in_band = index - band * kTileRows * cols_of_tiles;
-    const int band_rows = min(kTileRows, rows_of_tiles - band * kTileRows);
-    const int m0 = (band * kTileRows + in_band % band_rows) * BM, n0 = in_band / band_rows * cols;
+    const TilePlace place = place_tile((m + BM - 1) / BM, (width + cols - 1) / cols);
+    const int m0 = place.row * BM, n0 = place.col * cols;
 
     const int steps = (k + kTiledStep - 1) / kTiledStep;
     const int first = (int)blockIdx.y * steps_per_split, last = min(steps, first + steps_per_split), count = last - first;

@@ -5,16 +5,19 @@
 
 Outputs (git-ignored, but they travel with the source tree to a GPU machine):
     inferspore_amd/lib/libinferspore_amd.so     HIP kernels + the C ABI (include/inferspore_amd.h)
+    inferspore_amd/lib/_torch_calls.so          the calls of ops.py from torch's tensors to the C ABI
     inferspore_amd/lib/libinferspore_launch.so  the C++ `launch*` shims over the C ABI
     inferspore_amd/lib/libinferspore_layers.so  the C++ context-decoder layer (launch* + hipBLASLt GEMMs)
     build/bin/test_*                            reference-style C++ call-site programs
 """
 import argparse
 import concurrent.futures as cf
+import importlib.util
 import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 
 PKG = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(PKG)
@@ -35,6 +38,7 @@ HIPCC_FLAGS = [
 LIB_KERNELS = os.path.join(LIBDIR, "libinferspore_amd.so")
 LIB_LAUNCH = os.path.join(LIBDIR, "libinferspore_launch.so")
 LIB_LAYERS = os.path.join(LIBDIR, "libinferspore_layers.so")
+CALLS = os.path.join(LIBDIR, "_torch_calls.so")
 LAYERS = os.path.join(CSRC, "layers")
 
 
@@ -71,6 +75,17 @@ def _compile(src):
     return obj, out
 
 
+def _compile_calls():
+    """Host code only: torch's headers and libraries, the C ABI."""
+    torch_dir = os.path.dirname(importlib.util.find_spec("torch").origin)
+    include, libs = os.path.join(torch_dir, "include"), os.path.join(torch_dir, "lib")
+    return _run(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", "-I" + INCLUDE,
+                 "-isystem", include, "-isystem", os.path.join(include, "torch", "csrc", "api", "include"),
+                 "-isystem", sysconfig.get_paths()["include"], "-isystem", "/opt/rocm/include",
+                 os.path.join(CSRC, "torch_calls.cc"), "-o", CALLS, "-L" + LIBDIR, "-linferspore_amd", "-L" + libs, "-lc10", "-lc10_hip",
+                 "-ltorch_cpu", "-ltorch_python", "-Wl,-rpath,$ORIGIN"])
+
+
 def build(verbose=False, jobs=8, cpp_tests=True):
     for d in (LIBDIR, OBJDIR, BINDIR):
         os.makedirs(d, exist_ok=True)
@@ -83,6 +98,15 @@ def build(verbose=False, jobs=8, cpp_tests=True):
     objs = [o for o, _ in results]
     _run([hipcc(), "--offload-arch=" + ARCH, "-shared", "-fPIC", "-o", LIB_KERNELS] + objs)
 
+    with cf.ThreadPoolExecutor(max_workers=1) as ex:
+        calls = ex.submit(_compile_calls)
+        _build_callers(jobs, cpp_tests)
+        calls.result()
+    return LIB_KERNELS
+
+
+def _build_callers(jobs, cpp_tests):
+    """The C++ libraries and programs over the C ABI."""
     launch_src = os.path.join(CSRC, "launchers.cc")
     if os.path.exists(launch_src):
         _run([hipcc()] + HIPCC_FLAGS + ["-x", "hip", "-shared", launch_src, "-o", LIB_LAUNCH,
@@ -117,11 +141,10 @@ def build(verbose=False, jobs=8, cpp_tests=True):
 
             with cf.ThreadPoolExecutor(max_workers=jobs) as ex:
                 list(ex.map(one, srcs))
-    return LIB_KERNELS
 
 
 def clean():
-    for p in (LIB_KERNELS, LIB_LAUNCH, LIB_LAYERS):
+    for p in (LIB_KERNELS, LIB_LAUNCH, LIB_LAYERS, CALLS):
         if os.path.exists(p):
             os.remove(p)
     shutil.rmtree(os.path.join(ROOT, "build"), ignore_errors=True)

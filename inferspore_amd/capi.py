@@ -1,9 +1,12 @@
 """ctypes view of include/inferspore_amd.h.  Loading fails loudly when the library is not built."""
 import ctypes as C
+import importlib.machinery
+import importlib.util
 import os
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "lib", "libinferspore_amd.so")
+CALLS_PATH = os.path.join(_HERE, "lib", "_torch_calls.so")
 
 OK = 0
 ERR_NULL_POINTER = -1
@@ -72,6 +75,7 @@ SIGNATURES = {
 }
 
 _lib = None
+_calls = None
 
 
 class IspError(RuntimeError):
@@ -98,6 +102,30 @@ def lib():
             fn.argtypes = args
         _lib = l
     return _lib
+
+
+class _NoCalls:
+    """Stands for the module below where nothing has been built: every call is left to its general path, which raises."""
+
+    def __getattr__(self, name):
+        return lambda *args: None
+
+
+def calls():
+    """The native module that takes the calls on plain tensors (csrc/torch_calls.cc)."""
+    global _calls
+    if _calls is None:
+        if not os.path.exists(CALLS_PATH):
+            if os.path.exists(LIB_PATH):
+                raise RuntimeError("inferspore_amd: %s is missing -- build it with `python -m inferspore_amd.build`" % CALLS_PATH)
+            return _NoCalls()
+        lib()
+        import torch  # noqa: F401  the module links to its libraries
+        loader = importlib.machinery.ExtensionFileLoader("_torch_calls", CALLS_PATH)
+        module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_torch_calls", loader))
+        loader.exec_module(module)
+        _calls = module
+    return _calls
 
 
 def check(status, where):

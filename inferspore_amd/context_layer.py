@@ -28,8 +28,6 @@ import torch
 
 from . import capi, ops
 
-_PLAIN = (torch.Tensor, torch.nn.Parameter)
-_ONE_CALL = {torch.float16: "isp_context_layer_rows_f16", torch.float32: "isp_context_layer_rows_f32"}
 _PADDED = frozenset(("mask", "k_all", "v_all"))
 
 
@@ -154,49 +152,15 @@ def _fused_attention(st):
 def _layer_in_one_call(normed, residual, w, st, layer_id, gamma, rotary_dim, rotary_base, eps):
     """The whole layer as one call of the C ABI, or None where it is not the plain case of float16 or float32 rows: everything
     that the steps below accept or refuse otherwise stays with them."""
-    dtype = normed.dtype
-    if dtype not in _ONE_CALL or normed.dim() != 2 or normed.shape[0] == 0 or _padded_asked(st):
+    if normed.dtype not in (torch.float16, torch.float32) or _padded_asked(st):
         return None
-    (tokens, hidden), batch, heads, kv, hs = normed.shape, st.batch, st.head_num, st.kv_head_num, st.head_size
-    inter, width, max_seq = st.act.shape[-1], (heads + 2 * kv) * hs, st.k_cache.shape[3]
-    operands = ((normed, (tokens, hidden)), (residual, (tokens, hidden)), (w.qkv, (hidden, width)), (w.qkv_bias, (width,)),
-                (w.o, (heads * hs, hidden)), (w.gate_up, (hidden, 2 * inter)), (w.down, (inter, hidden)), (w.ffn_norm, (hidden,)),
-                (gamma, (hidden,)), (st.q, (batch, heads, st.max_q_len, hs)),
-                (st.k_cache, (st.k_cache.shape[0], batch, kv, max_seq, hs)), (st.v_cache, tuple(st.k_cache.shape)),
-                (st.packed_ctx, (tokens, heads, hs)), (st.act, (tokens, inter)))
-    grad, device = torch.is_grad_enabled(), normed.device
-    if not normed.is_cuda or torch.is_autocast_enabled():
-        return None
-    for t, shape in operands:
-        if t is None and shape == (width,):
-            continue
-        if (type(t) not in _PLAIN or t.dtype != dtype or t.shape != shape or not t.is_contiguous() or
-                t.device != device or t.data_ptr() % 16 or (grad and t.requires_grad)):
-            return None
-    for t, most in ((st.padding_offset, tokens), (st.history, batch), (st.lengths, batch), (st.context, batch)):
-        if (type(t) not in _PLAIN or t.dtype != torch.int32 or t.numel() < most or not t.is_contiguous() or
-                t.device != device):
-            return None
-    if not (st.tokens == tokens and st.context.shape[0] == batch and 0 <= int(layer_id) < st.k_cache.shape[0] and
-            0 <= int(rotary_dim) <= hs and int(rotary_dim) % 2 == 0) or normed.data_ptr() == residual.data_ptr():
-        return None
-    if not ops.apart(st.q, st.packed_ctx):
-        return None
-    lib = capi.lib()
-    name = _ONE_CALL[dtype]
-    need = getattr(lib, name + "_workspace")(batch, tokens, hidden, heads, kv, hs, st.max_q_len, st.max_k_len, max_seq, inter)
-    if need == 0:
-        return None
-    workspace = torch.empty(need, dtype=torch.uint8, device=device)
-    out = torch.empty_like(normed)
-    p = torch.Tensor.data_ptr
-    capi.check(getattr(lib, name)(
-        p(normed), p(residual), p(out), p(w.qkv), None if w.qkv_bias is None else p(w.qkv_bias), p(w.o), p(w.gate_up),
-        p(w.down), p(w.ffn_norm), p(gamma), p(st.q), p(st.k_cache), p(st.v_cache), p(st.packed_ctx), p(st.act),
-        p(st.padding_offset), p(st.history), p(st.lengths), p(st.context), p(workspace), int(layer_id), batch, tokens, hidden,
-        heads, kv, hs, st.max_q_len, st.max_k_len, max_seq, inter, int(rotary_dim), float(rotary_base), float(eps),
-        ops._stream()), "isp_context_layer")
-    if isinstance(st, BatchState):
+    out = capi.calls().context_layer(
+        normed, residual, w.qkv, w.qkv_bias, w.o, w.gate_up, w.down, w.ffn_norm, gamma, st.q, st.k_cache, st.v_cache, st.packed_ctx,
+        st.act, st.padding_offset, st.history, st.lengths, st.context, int(layer_id), int(st.tokens), int(st.head_num),
+        int(st.kv_head_num), int(st.head_size), int(st.max_k_len), int(rotary_dim), float(rotary_base), float(eps))
+    if type(out) is int:
+        capi.check(out, "isp_context_layer")
+    if out is not None and isinstance(st, BatchState):
         st._attended = int(layer_id)
     return out
 

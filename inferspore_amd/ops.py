@@ -59,8 +59,19 @@ def _stream():
     return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
+def _done(status, where):
+    """Whether the native module has taken a call (capi.calls()): not where it answers None.  What follows in each function is the general
+    path: the checks that name what is wrong, and the operands that are more than plain tensors."""
+    if status is None:
+        return False
+    capi.check(status, where)
+    return True
+
+
 def input_embedding(input_ids, output, embed_table, check_bounds=True):
     """launchInputEmbedding: output[t, :] = embed_table[input_ids[t], :]."""
+    if _done(capi.calls().input_embedding(input_ids, output, embed_table, check_bounds), "isp_embedding"):
+        return output
     _int32(input_ids)
     _suffix(output)
     _expect(output.dim() == 2 and embed_table.dim() == 2 and input_ids.dim() == 1,
@@ -80,6 +91,8 @@ def input_embedding(input_ids, output, embed_table, check_bounds=True):
 
 def cal_padding_offset(padding_offset, cum_seqlens, input_lengths):
     """launchCalPaddingoffset: padding_offset [batch, max_q_len], cum_seqlens [batch + 1]."""
+    if _done(capi.calls().cal_padding_offset(padding_offset, cum_seqlens, input_lengths), "isp_cal_padding_offset"):
+        return padding_offset, cum_seqlens
     _expect(padding_offset.dim() == 2 and cum_seqlens.dim() == 1 and input_lengths.dim() == 1,
             "cal_padding_offset takes padding_offset [batch, max_q_len], cum_seqlens [batch + 1], lengths [batch]")
     batch, max_q_len = padding_offset.shape
@@ -99,6 +112,8 @@ def cal_padding_offset(padding_offset, cum_seqlens, input_lengths):
 
 def rmsnorm(x, gamma, eps):
     """In-place RMSNorm of x [tokens, hidden]."""
+    if _done(capi.calls().rmsnorm(x, gamma, eps), "isp_rmsnorm"):
+        return x
     _same_dtype(x, gamma)
     _expect(x.dim() == 2, "rmsnorm takes x [tokens, hidden]")
     _expect(gamma.numel() == x.shape[1], "gamma must hold one value per hidden column")
@@ -110,6 +125,9 @@ def rmsnorm(x, gamma, eps):
 
 def fused_add_bias_residual_rmsnorm(residual, decoder_out, bias, gamma, eps, flags=0):
     """launchFusedAddBiasResidualRMSNorm: in place on residual (may be None) and decoder_out."""
+    if _done(capi.calls().fused_add_bias_residual_rmsnorm(residual, decoder_out, bias, gamma, eps, flags),
+             "isp_fused_add_bias_residual_rmsnorm"):
+        return residual, decoder_out
     _same_dtype(decoder_out, residual, bias, gamma)
     _expect(decoder_out.dim() == 2, "fused norm takes decoder_out [tokens, hidden]")
     hidden = decoder_out.shape[1]
@@ -156,6 +174,10 @@ def add_fused_qkv_bias_transpose_and_rope(q_buf, k_buf, v_buf, qkv, qkv_bias, pa
                                           use_dynamic_ntk=False):
     """launchAddFusedQKVBiasTransposeAndRoPE; shapes as the reference derives them
     (qkv_bias_and_RoPE.cu:298-304)."""
+    if _done(capi.calls().qkv_bias_rope_transpose(q_buf, k_buf, v_buf, qkv, qkv_bias, padding_offset, history_length, input_length,
+                                                  rotary_embedding_dim, rotary_embedding_base, max_position_embeddings,
+                                                  use_dynamic_ntk), "isp_qkv_bias_rope_transpose"):
+        return q_buf, k_buf, v_buf
     _same_dtype(qkv, q_buf, k_buf, v_buf, qkv_bias)
     _int32(padding_offset, history_length, input_length)
     token_num, head_size, batch, head_num, seq_len, kv_head_num = _qkv_shapes(
@@ -176,6 +198,10 @@ def add_fused_qkv_bias_transpose_rope_and_append(q_buf, k_buf, v_buf, k_cache, v
     """launchAddFusedQKVBiasTransposeAndRoPE with launchConcatKVCache fused in: k_buf / v_buf may both be
     None (the k and v rows then go to the cache only).
     k_cache, v_cache [layers, batch, kv_head_num, max_seq_len, head_size]."""
+    if _done(capi.calls().qkv_bias_rope_transpose_append(q_buf, k_buf, v_buf, k_cache, v_cache, layer_id, qkv, qkv_bias,
+                                                         padding_offset, history_length, input_length, rotary_embedding_dim,
+                                                         rotary_embedding_base), "isp_qkv_bias_rope_transpose_append"):
+        return q_buf, k_cache, v_cache
     _same_dtype(qkv, q_buf, k_buf, v_buf, k_cache, v_cache, qkv_bias)
     _int32(padding_offset, history_length, input_length)
     _expect(input_length is not None, "input_length is required")
@@ -196,6 +222,8 @@ def add_fused_qkv_bias_transpose_rope_and_append(q_buf, k_buf, v_buf, k_cache, v
 
 def act(input, out):
     """launchAct (SwiGLU): input [tokens, 2, inter] -> out [tokens, inter]."""
+    if _done(capi.calls().act(input, out), "isp_swiglu"):
+        return out
     _same_dtype(input, out)
     _expect(input.dim() == 3, "SwiGLU input must have shape [tokens, 2, inter]")
     if input.shape[1] != 2:
@@ -229,6 +257,9 @@ def rope_decode_and_append(qkv_buf, qkv_bias, k_cache, v_cache, layer_id, histor
     the v row of sequence b go to cache[layer][b, head, history_length[b], :] (as launchConcatKVCache with one
     query token).  qkv_bias may be None.  step = 0: every sequence is rotated at its own history_length[b] instead
     (a batch whose sequences have different histories)."""
+    if _done(capi.calls().rope_decode_append(qkv_buf, qkv_bias, k_cache, v_cache, layer_id, history_length, step, head_num,
+                                             rotary_embedding_dim, rotary_embedding_base), "isp_rope_decode_append"):
+        return qkv_buf, k_cache, v_cache
     _same_dtype(qkv_buf, qkv_bias, k_cache, v_cache)
     _int32(history_length)
     _expect(qkv_buf.dim() == 3, "qkv_buf must be [batch, heads, head_size]")
@@ -253,6 +284,8 @@ def rope_decode_and_append(qkv_buf, qkv_bias, k_cache, v_cache, layer_id, histor
 
 def transpose_out_remove_padding(qkv_buf_w_pad, padding_offset, qkv_buf_wo_pad):
     """launchTransposeOutRemovePadding: [batch, heads, seq, hs] -> [tokens, heads, hs]."""
+    if _done(capi.calls().transpose_out_remove_padding(qkv_buf_w_pad, padding_offset, qkv_buf_wo_pad), "isp_transpose_remove_padding"):
+        return qkv_buf_wo_pad
     _same_dtype(qkv_buf_w_pad, qkv_buf_wo_pad)
     _int32(padding_offset)
     _expect(qkv_buf_w_pad.dim() == 4 and qkv_buf_wo_pad.dim() == 3,
@@ -352,6 +385,9 @@ def context_attention(q_buf, k_cache, v_cache, layer_id, history_length, input_l
 
 def concat_kv_cache(k_src, v_src, layer_id, cur_query_length, history_length, k_dst, v_dst):
     """launchConcatKVCache; shapes as the reference derives them (concat_past_kv.cu:84-90)."""
+    if _done(capi.calls().concat_kv_cache(k_src, v_src, layer_id, cur_query_length, history_length, k_dst, v_dst),
+             "isp_concat_kv_cache"):
+        return k_dst, v_dst
     _same_dtype(k_src, v_src, k_dst, v_dst)
     _int32(cur_query_length, history_length)
     _expect(k_src.dim() == 4 and k_src.shape == v_src.shape,
@@ -374,6 +410,9 @@ def concat_kv_cache(k_src, v_src, layer_id, cur_query_length, history_length, k_
 
 def repeat_kv_cache(k_cache_src, v_cache_src, context_length, layer_id, k_cache_dst, v_cache_dst):
     """launchRepeatKVCache; shapes as the reference derives them (repeat_kv.cu:59-70)."""
+    if _done(capi.calls().repeat_kv_cache(k_cache_src, v_cache_src, context_length, layer_id, k_cache_dst, v_cache_dst),
+             "isp_repeat_kv_cache"):
+        return k_cache_dst, v_cache_dst
     _same_dtype(k_cache_src, v_cache_src, k_cache_dst, v_cache_dst)
     _int32(context_length)
     _expect(k_cache_src.dim() == 5 and k_cache_src.shape == v_cache_src.shape,

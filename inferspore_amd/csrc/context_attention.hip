@@ -551,12 +551,29 @@ __global__ __launch_bounds__(64) void combine_splits_f16(const float* __restrict
     }
     const float safe = m == -INFINITY ? 0.0f : m;
     float o[HS / 64] = {};
-    for (int z = 0; z < splits; z++) {
-        const float* pz = p + z * partial_floats(HS);
-        const float e = __builtin_amdgcn_exp2f(pz[HS] - safe);
-        l += e * pz[HS + 1];
+    constexpr int kAtOnce = 8;  // splits whose loads are on their way together; those past the last re-read it
+    for (int z0 = 0; z0 < splits; z0 += kAtOnce) {
+        float part[kAtOnce][HS / 64 + 2];
 #pragma unroll
-        for (int i = 0; i < HS / 64; i++) o[i] += e * pz[HS / 64 * lane + i];
+        for (int i = 0; i < kAtOnce; i++) {
+            const float* pz = p + min(z0 + i, splits - 1) * partial_floats(HS);
+            part[i][0] = pz[HS];
+            part[i][1] = pz[HS + 1];
+#pragma unroll
+            for (int d = 0; d < HS / 64; d++) part[i][2 + d] = pz[HS / 64 * lane + d];
+        }
+#pragma unroll
+        for (int i = 0; i < kAtOnce; i++)
+#pragma unroll
+            for (int d = 0; d < HS / 64 + 2; d++) asm volatile("" : "+v"(part[i][d]));  // or the loads move behind the test below
+#pragma unroll
+        for (int i = 0; i < kAtOnce; i++) {
+            if (z0 + i >= splits) break;  // uniform
+            const float e = __builtin_amdgcn_exp2f(part[i][0] - safe);
+            l += e * part[i][1];
+#pragma unroll
+            for (int d = 0; d < HS / 64; d++) o[d] += e * part[i][2 + d];
+        }
     }
     const long long token = (long long)n + q;
     if (token >= tokens) return;

@@ -29,10 +29,10 @@ __global__ __launch_bounds__(kBlock) void linear_add_splits(const float* __restr
                                                             unsigned quads, int splits) {
     const unsigned i = blockIdx.x * kBlock + threadIdx.x;
     if (i >= quads) return;
-    const float4v* p = reinterpret_cast<const float4v*>(partial) + i;
-    float4v sum = p[0];
-#pragma unroll 8
-    for (int s = 1; s < splits; s++) sum += p[(size_t)s * quads];
+    const float* const at[1] = {partial + 4 * (size_t)i};
+    float4v sums[1];
+    add_splits(at, 4 * (size_t)quads, splits, sums);
+    const float4v sum = sums[0];
     const __half2 lo = __floats2half2_rn(sum[0], sum[1]), hi = __floats2half2_rn(sum[2], sum[3]);
     reinterpret_cast<uint2*>(out)[i] = make_uint2(*reinterpret_cast<const uint32_t*>(&lo), *reinterpret_cast<const uint32_t*>(&hi));
 }

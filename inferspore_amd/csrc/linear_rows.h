@@ -219,17 +219,51 @@ inline void launch_product(const ProductPlan& plan, const __half* a, const __hal
     else launch_skinny(plan.skinny, a, w, plan.skinny.splits == 1 ? out : nullptr, partial, m, n, k, stream);
 }
 
-// Eight neighbouring columns of a product left as partial sums: the splits added in their order and rounded to fp16 once, the
-// value linear_add_splits would have stored.  `stride`: floats between two splits.
-__device__ __forceinline__ vec16 add_splits8(const float* p, size_t stride, int splits) {
-    float4v a = *reinterpret_cast<const float4v*>(p), b = *reinterpret_cast<const float4v*>(p + 4);
-#pragma unroll 4
-    for (int s = 1; s < splits; s++) {
-        a += *reinterpret_cast<const float4v*>(p + s * stride);
-        b += *reinterpret_cast<const float4v*>(p + s * stride + 4);
+// Values of a product left as partial sums, four neighbouring ones at each of p[0 ... PIECES): the splits added in their order.  `stride`:
+// floats between two splits.  All loads of up to eight splits are on their way before the first is added (those past the last re-read
+// it): the sums were just written by other XCDs, and a loop that waits for one load after the other took most of its kernel's time.
+template <int CHUNK, int PIECES>
+__device__ __forceinline__ void add_split_chunks(const float* const (&p)[PIECES], size_t stride, int splits, float4v (&sum)[PIECES]) {
+    for (int s0 = 0; s0 < splits; s0 += CHUNK) {
+        float4v v[CHUNK][PIECES];
+#pragma unroll
+        for (int s = 0; s < CHUNK; s++)
+#pragma unroll
+            for (int i = 0; i < PIECES; i++) v[s][i] = *reinterpret_cast<const float4v*>(p[i] + (size_t)min(s0 + s, splits - 1) * stride);
+#pragma unroll
+        for (int s = 0; s < CHUNK; s++)
+#pragma unroll
+            for (int i = 0; i < PIECES; i++) asm volatile("" : "+v"(v[s][i]));  // or the compiler moves each load behind the test below
+#pragma unroll
+        for (int s = 0; s < CHUNK; s++) {
+            if (s0 + s >= splits) break;  // uniform
+#pragma unroll
+            for (int i = 0; i < PIECES; i++) sum[i] = s0 + s == 0 ? v[s][i] : sum[i] + v[s][i];
+        }
     }
+}
+template <int PIECES>
+__device__ __forceinline__ void add_splits(const float* const (&p)[PIECES], size_t stride, int splits, float4v (&sum)[PIECES]) {
+    if (splits <= 4) add_split_chunks<4>(p, stride, splits, sum);  // uniform
+    else add_split_chunks<8>(p, stride, splits, sum);
+}
+// Eight neighbouring columns rounded to fp16 once, the value linear_add_splits would have stored.
+__device__ __forceinline__ vec16 pack_sums(const float4v& a, const float4v& b) {
     const float f[8] = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
     return Elem<__half>::pack(f);
+}
+__device__ __forceinline__ vec16 add_splits8(const float* p, size_t stride, int splits) {
+    const float* const at[2] = {p, p + 4};
+    float4v sum[2];
+    add_splits(at, stride, splits, sum);
+    return pack_sums(sum[0], sum[1]);
+}
+__device__ __forceinline__ void add_splits8(const float* p, const float* q, size_t stride, int splits, vec16& first, vec16& second) {
+    const float* const at[4] = {p, p + 4, q, q + 4};
+    float4v sum[4];
+    add_splits(at, stride, splits, sum);
+    first = pack_sums(sum[0], sum[1]);
+    second = pack_sums(sum[2], sum[3]);
 }
 
 // Consumers of partial sums: what the entry points of the same step do with a stored fp16 product (same bits), with that

@@ -63,11 +63,10 @@ __global__ __launch_bounds__(kBlock) void linear_add_splits_f32(const float* __r
                                                                 unsigned quads, int splits) {
     const unsigned i = blockIdx.x * kBlock + threadIdx.x;
     if (i >= quads) return;
-    const float4v* p = reinterpret_cast<const float4v*>(partial) + i;
-    float4v sum = p[0];
-#pragma unroll 8
-    for (int s = 1; s < splits; s++) sum += p[(size_t)s * quads];
-    reinterpret_cast<float4v*>(out)[i] = sum;
+    const float* const at[1] = {partial + 4 * (size_t)i};
+    float4v sum[1];
+    add_splits(at, 4 * (size_t)quads, splits, sum);
+    reinterpret_cast<float4v*>(out)[i] = sum[0];
 }
 
 // Extents that the kernels can count (the addition indexes four values in 32 bits).

@@ -1266,14 +1266,15 @@ __global__ __launch_bounds__(kBlock) void qkv_rope_sums_f16(RopeDivisors tab, co
     half_units.divmod(live ? unit : 0u, h, g);
     const size_t col = (size_t)h * hs + (size_t)g * 8u, width = (size_t)heads * hs;
     const float* src = partial + (size_t)token * width + col;
-    const vec16 lo = add_splits8(src, (size_t)tokens * width, splits);
-    const vec16 hi = add_splits8(src + half, (size_t)tokens * width, splits);
+    const int32_t offset = read_only_i32(padding_offset, token);
     vec16 blo, bhi;
     if (bias) {
         blo = load16(bias + col);
         bhi = load16(bias + col + half);
     }
-    const long long p = (long long)token + (long long)read_only_i32(padding_offset, token);
+    vec16 lo, hi;
+    add_splits8(src, src + half, (size_t)tokens * width, splits, lo, hi);
+    const long long p = (long long)token + (long long)offset;
     if (p < 0 || p >= (long long)positions) return;  // workgroup-uniform
     unsigned b, s;
     seq.divmod((unsigned)p, b, s);

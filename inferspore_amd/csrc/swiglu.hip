@@ -108,7 +108,8 @@ __global__ __launch_bounds__(kWave) void swiglu_sums_f16(const float* __restrict
     if (unit * 8 >= inter) return;
     const size_t stride = (size_t)tokens * 2u * (size_t)inter;
     const float* gate = partial + (size_t)token * 2u * (size_t)inter + (size_t)unit * 8u;
-    const vec16 g = add_splits8(gate, stride, splits), u = add_splits8(gate + inter, stride, splits);
+    vec16 g, u;
+    add_splits8(gate, gate + inter, stride, splits, g, u);
     float a[8], b[8], y[8];
     Elem<__half>::unpack(g, a);
     Elem<__half>::unpack(u, b);

@@ -19,36 +19,26 @@
 // accumulators, the B operand of the second product O^T[d, query] = V^T x P^T -- no exchange between lanes.
 // The B operand's 16 contraction indices are matched to the accumulator rows by reading V^T's keys in the
 // order (4 h + j, 8 + 4 h + j), h = lane / 32: a contraction does not care about the order of its terms as
-// long as both operands agree.  K tiles sit in LDS as stored ([key][d], padded rows), V tiles transposed
-// ([d][key], written two keys at a time, the keys of a row in the operand's order) so that the A operand of the
-// second product is one 16-byte read.
-#include "isp_common.h"
+// long as both operands agree.  K and V tiles go from memory straight into LDS, as stored ([key][d]); the A operand of the
+// second product is read by the transposing LDS load (ds_read_b64_tr_b16: sixteen lanes hand in four keys of sixteen d and get four
+// keys of one d each).  Against tiles moved
+// through registers and transposed on the way, us: 4 prompts of up to 2048 tokens, 32 heads of 128, 149 and 132 (680 TFLOP/s); one of
+// 4096 on 8 key heads 188 and 165 (830); 8 of up to 512 32.7 and 29.8; 2 of 2000 and 1500, 16 heads of 64, 47.4 and 44.4.  What
+// bounds it then is the wavefronts' own instructions: reads ahead of the softmax, products in turn and priorities changed nothing.
+// Bank conflicts: the 16-byte chunks of a row are permuted by an exclusive or with its
+// row number, by choosing which chunk each lane of a load brings.
+#include "tile_loads.h"
 
 namespace isp {
 
 namespace {
 
-typedef _Float16 half8 __attribute__((ext_vector_type(8)));
-typedef _Float16 half4 __attribute__((ext_vector_type(4)));
 typedef float float16v __attribute__((ext_vector_type(16)));
 
 constexpr int kQueriesPerWave = 32;
 constexpr int kWaves = 4;
 constexpr int kQueryTile = kQueriesPerWave * kWaves;  // queries per workgroup
 constexpr int kKeyTile = 64;
-constexpr int kKPad = 8;  // halfs added to a key row in LDS (272 bytes for 128-element heads): spreads the rows over the banks
-
-// The transposed value tile: row d holds the tile's 64 keys as 8 units of 16 bytes, and a unit is exactly what one
-// lane needs for one product: unit 2 t + h holds the keys 16 t + 4 h + 0..3 followed by 16 t + 8 + 4 h + 0..3 (the
-// order in which the accumulator rows of the scores meet the operand's contraction index).  Unit u of row d sits
-// at position u ^ (d % 8) ^ ((d / 8) % 8): the 64 lanes of an operand read (32 rows d, two units) then touch every
-// bank equally, and the transposing writes (two neighbouring keys, 4 bytes) are spread over half of the banks.
-__device__ __forceinline__ int vt_unit(int d, int unit) { return d * (kKeyTile / 2) + 4 * (unit ^ (d & 7) ^ ((d >> 3) & 7)); }
-// dword that holds the keys `pair * 2` and `pair * 2 + 1` of row d
-__device__ __forceinline__ int vt_pair(int d, int pair) {
-    const int key = 2 * pair, step = key / 16, quad = (key % 16) / 4;  // quads 0..3 of a step: h = quad % 2, second half = quad / 2
-    return vt_unit(d, 2 * step + quad % 2) + 2 * (quad / 2) + (key % 4) / 2;
-}
 
 // Maximum / sum of a value with the one in the other half of the wavefront (lane ^ 32), without a trip through LDS:
 // the swap leaves the lower half's value in every lane of one register and the upper half's in the other.
@@ -74,20 +64,27 @@ __global__ __launch_bounds__(256, 2) void context_attention_f16(
     const _Float16* __restrict__ q_buf, const _Float16* __restrict__ k_cache, const _Float16* __restrict__ v_cache,
     _Float16* __restrict__ out, const int* history_length, const int* input_length, const int* context_length,
     int head_num, int kv_head_num, int max_q_len, int max_k_len, int max_seq_len, int tokens, float scale_log2e) {
-    constexpr int kHeadSize = HS, kKStride = HS + kKPad;
+    constexpr int kHeadSize = HS;
     constexpr int kDSteps = HS / 16;    // products over d per 32 x 32 block of scores
     constexpr int kDBlocks = HS / 32;   // 32-row blocks of O^T
-    constexpr int kChunks = HS / 8;     // 16-byte pieces of a key or value row
-    constexpr int kUnits = kChunks * kKeyTile / 2, kMoves = (kUnits + 255) / 256;  // key pairs of 8 d a tile has, a thread moves
+    constexpr int kChunks = HS / 8;                      // 16-byte chunks of a key or value row
+    constexpr int kRow = HS == 64 ? 8 : 16;              // and of a row in LDS: heads of 96 leave four unused
+    constexpr int kLoads = kKeyTile * kRow / 256;        // of a lane per tile, of either operand
+    constexpr uint32_t kTileBytes = kKeyTile * kRow * 16, kStage = 2 * kTileBytes;  // keys, then values
+    // chunk c of key row r lies at c ^ key_swizzle(r), so that sixteen neighbouring rows' chunks touch every bank once; of value row
+    // r at c ^ value_swizzle(r): four chunks of four neighbouring rows
+    constexpr auto key_swizzle = [](int r) { return kRow == 16 ? r % 16 : r / 2 % 8; };
+    constexpr auto value_swizzle = [](int r) { return kRow == 16 ? r % 4 * 4 : r / 2 % 2 * 4; };
     // Heads of 96: the probabilities as the sum of two halves, each a factor of its own product, so that they keep 21 bits (they
     // were fp32 in the kernel that served these heads before).  Scaled by 2^15 -- the sum that divides the result is, too -- so
     // that the lower halves are normal numbers down to probabilities of 2^-18.
     constexpr bool kTwoHalves = HS == 96;
     constexpr float kProbabilityExponent = kTwoHalves ? 15.0f : 0.0f;
-    __shared__ __align__(16) _Float16 k_tiles[2][kKeyTile * kKStride];
-    __shared__ __align__(16) uint32_t vt_tiles[2][kHeadSize * kKeyTile / 2];  // [d][key], two keys per dword
+    __shared__ __align__(1024) char tiles[2 * kStage];
+    typedef __attribute__((address_space(3))) char* lds_ptr;
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_ptr)tiles;
 
-    const int tid = threadIdx.x, lane = tid % 64, wave = tid / 64, half_id = lane / 32, col = lane % 32;
+    const int tid = threadIdx.x, lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64), half_id = lane / 32, col = lane % 32;
     // grid: x = head (fastest), y = sequence, z = query tile in DESCENDING order -- the tiles far down the causal
     // triangle visit the most key tiles, and workgroups are handed out in grid order, so the long ones start first
     // (the kernel takes as long as its longest workgroup: pinning the query tiles of a (sequence, head) pair to one
@@ -143,65 +140,53 @@ __global__ __launch_bounds__(256, 2) void context_attention_f16(
         for (int i = 0; i < 16; i++) acc[db][i] = 0.0f;
     float run_max = -INFINITY, run_sum = 0.0f;
 
-    // A thread moves two pairs of neighbouring keys per tile (pairs, so that V^T is written two keys -- one dword --
-    // at a time).  The eight loads of a tile are issued together and unconditionally: a row past the visible keys
-    // re-reads the last visible one and is masked to zero when it is stored (loads or register writes under a
-    // branch would each be waited for before the next is issued).  The loads of tile n + 1 are in flight while
-    // tile n is computed.
-    uint4 kraw[kMoves][2], vraw[kMoves][2];
-    auto fetch = [&](int kt) {
+    // Two tiles are in LDS: one is computed while the loads of the other are in flight.  Rows past the visible ones re-read the last of
+    // them; their scores are masked, their values cleared (a zero probability times infinity is NaN).
+    uint32_t k_chunk[kLoads], v_chunk[kLoads];  // byte offsets of the chunks that this lane brings, in their rows
 #pragma unroll
-        for (int i = 0; i < kMoves; i++) {
-            // heads of 96 leave half of the second moves idle: they re-read the first
-            const int unit = tid + 256 * i < kUnits ? tid + 256 * i : tid, d0 = (unit % kChunks) * 8, key = 2 * (unit / kChunks);
+    for (int i = 0; i < kLoads; i++) {
+        const int at = (wave * kLoads + i) * 64 + lane, r = at / kRow;
+        const int kc = at % kRow ^ key_swizzle(r), vc = at % kRow ^ value_swizzle(r);
+        k_chunk[i] = 16 * (kc < kChunks ? kc : kc - kChunks);
+        v_chunk[i] = 16 * (vc < kChunks ? vc : vc - kChunks);
+    }
+    const auto load = [&](uint32_t stage_at, int kt) __attribute__((always_inline)) {
+        const _Float16 *k_tile = keys + (size_t)kt * kHeadSize, *v_tile = values + (size_t)kt * kHeadSize;
 #pragma unroll
-            for (int j = 0; j < 2; j++) {
-                const size_t at = (size_t)min(kt + key + j, wg_visible - 1) * kHeadSize + d0;
-                kraw[i][j] = *reinterpret_cast<const uint4*>(keys + at);
-                vraw[i][j] = *reinterpret_cast<const uint4*>(values + at);
-            }
+        for (int i = 0; i < kLoads; i++) {
+            const uint32_t row = (uint32_t)min(((wave * kLoads + i) * 64 + lane) / kRow, wg_visible - 1 - kt) * (kHeadSize * 2);
+            load_to_lds(stage_at + (wave * kLoads + i) * 1024, k_tile, row + k_chunk[i]);
+            load_to_lds(stage_at + kTileBytes + (wave * kLoads + i) * 1024, v_tile, row + v_chunk[i]);
         }
     };
-    auto store = [&](int buf, int kt) {
-        _Float16* k_lds = k_tiles[buf];
-        uint32_t* vt_lds = vt_tiles[buf];
-        // ---- the tile into LDS: 64 keys x 128 d of K as stored, of V transposed; keys past the visible ones as zeros
-        //      (a zero probability times whatever an unwritten cache row holds could be NaN)
-#pragma unroll
-        for (int i = 0; i < kMoves; i++) {
-            const int unit = tid + 256 * i, pair = unit / kChunks, d0 = (unit % kChunks) * 8, key = 2 * pair;
-            if (unit >= kUnits) break;  // wavefront-uniform
-            uint32_t lo[4], hi[4];
-#pragma unroll
-            for (int j = 0; j < 2; j++) {
-                uint4 kk = kraw[i][j], vv = vraw[i][j];
-                if (kt + kKeyTile > wg_visible) {  // workgroup-uniform: only the last tile has rows to blank
-                    const uint32_t keep = kt + key + j < wg_visible ? 0xffffffffu : 0u;
-                    kk = make_uint4(kk.x & keep, kk.y & keep, kk.z & keep, kk.w & keep);
-                    vv = make_uint4(vv.x & keep, vv.y & keep, vv.z & keep, vv.w & keep);
-                }
-                *reinterpret_cast<uint4*>(&k_lds[(key + j) * kKStride + d0]) = kk;
-                uint32_t* v = j == 0 ? lo : hi;
-                v[0] = vv.x, v[1] = vv.y, v[2] = vv.z, v[3] = vv.w;
-            }
-#pragma unroll
-            for (int e = 0; e < 8; e++) {
-                // low half: v[key][d0 + e], high half: v[key + 1][d0 + e]  (one byte-permute of the two source dwords)
-                vt_lds[vt_pair(d0 + e, pair)] =
-                    __builtin_amdgcn_perm(hi[e / 2], lo[e / 2], e % 2 ? 0x07060302u : 0x05040100u);
-            }
-        }
-    };
-    fetch(0);
-    store(0, 0);
-    fetch(kKeyTile);  // past the last tile a fetch re-reads the last visible row; what it brings is stored as zeros
+    load(lds0, 0);
+    if (kKeyTile < wg_visible) load(lds0 + kStage, kKeyTile);
     sum_lengths_wave(length_share, b, length_shares);
-    __syncthreads();
 
-    int cur = 0;
-    for (int kt = 0; kt < wg_visible; kt += kKeyTile, cur ^= 1) {
-        const _Float16* k_lds = k_tiles[cur];
-        const uint32_t* vt_lds = vt_tiles[cur];
+    // where a lane reads: row col of 32 keys; of V rows 4 half_id ... of eight, four columns, for the lane that they end in
+    uint32_t k_at[kDSteps], v_at[kDBlocks];
+#pragma unroll
+    for (int st = 0; st < kDSteps; st++) k_at[st] = lds0 + col * (kRow * 16) + 16 * ((2 * st + half_id) ^ key_swizzle(col));
+#pragma unroll
+    for (int db = 0; db < kDBlocks; db++) {
+        const int r = 4 * half_id + lane % 16 / 4, c = 4 * db + lane / 16 % 2 * 2 + lane % 4 / 2;
+        v_at[db] = lds0 + kTileBytes + r * (kRow * 16) + 16 * (c ^ value_swizzle(r)) + 8 * (lane % 2);
+    }
+
+    uint32_t stage_at = lds0;
+    for (int kt = 0; kt < wg_visible; kt += kKeyTile) {
+        const bool more = kt + kKeyTile < wg_visible;
+        if (more) {
+            wait_loads<2 * kLoads>();
+        } else {
+            wait_loads<0>();
+#pragma unroll
+            for (int i = 0; i < kLoads; i++) {
+                const int at = (wave * kLoads + i) * 64 + lane;
+                if (kt + at / kRow >= wg_visible) lds_clear16(stage_at + kTileBytes + at * 16);
+            }
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" : : : "memory");
 
         if (kt < wave_visible) {  // wavefront-uniform: tiles behind this wavefront's diagonal are skipped
             // ---- S^T[key, query] for the 64 keys: two 32-row blocks, 8 steps over d each
@@ -215,7 +200,7 @@ __global__ __launch_bounds__(256, 2) void context_attention_f16(
                 half8 ka[kDSteps];
 #pragma unroll
                 for (int st = 0; st < kDSteps; st++)
-                    ka[st] = *reinterpret_cast<const half8*>(&k_lds[(32 * rb + col) * kKStride + 16 * st + 8 * half_id]);
+                    ka[st] = lds_read_row(k_at[st] + 32 * rb * (kRow * 16));
                 __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
                 for (int st = 0; st < kDSteps; st++) s[rb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ka[st], qf[st], s[rb], 0, 0, 0);
@@ -265,7 +250,8 @@ __global__ __launch_bounds__(256, 2) void context_attention_f16(
                 half8 va[kDBlocks];
 #pragma unroll
                 for (int db = 0; db < kDBlocks; db++)
-                    va[db] = *reinterpret_cast<const half8*>(&vt_lds[vt_unit(32 * db + col, 2 * t + half_id)]);
+                    va[db] = __builtin_shufflevector(lds_read_transposed(v_at[db] + 16 * t * (kRow * 16)),
+                                                     lds_read_transposed(v_at[db] + (16 * t + 8) * (kRow * 16)), 0, 1, 2, 3, 4, 5, 6, 7);
                 half8 p, low;
 #pragma unroll
                 for (int e = 0; e < 8; e++) {
@@ -281,12 +267,15 @@ __global__ __launch_bounds__(256, 2) void context_attention_f16(
                 }
             }
         }
-        // the next tile (its loads were issued before this tile's products) goes into the other buffer, which every
-        // wavefront finished reading before the barrier that ended the previous iteration; then the loads of the
-        // tile after it are started: one barrier per tile, and no load is waited for right after it was issued
-        store(cur ^ 1, kt + kKeyTile);
-        fetch(kt + 2 * kKeyTile);
-        __syncthreads();
+        // once every wavefront has read this tile its place is free for the one after the next
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" : : : "memory");
+        if (kt + 2 * kKeyTile < wg_visible) load(stage_at, kt + 2 * kKeyTile);
+        const uint32_t by = stage_at == lds0 ? kStage : 0u - kStage;
+        stage_at += by;
+#pragma unroll
+        for (int st = 0; st < kDSteps; st++) k_at[st] += by;
+#pragma unroll
+        for (int db = 0; db < kDBlocks; db++) v_at[db] += by;
     }
 
     const long long token = (long long)sum_lengths_total(length_shares) + my_q;

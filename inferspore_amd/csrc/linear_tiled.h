@@ -25,19 +25,6 @@
 
 namespace isp {
 
-typedef _Float16 half8 __attribute__((ext_vector_type(8)));
-typedef _Float16 half4 __attribute__((ext_vector_type(4)));
-
-__device__ __forceinline__ half4 lds_read_transposed(uint32_t at) {
-    typedef short short4v __attribute__((ext_vector_type(4)));
-    typedef __attribute__((address_space(3))) short4v* lds_ptr;
-    const short4v r = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)(uintptr_t)at);
-    return __builtin_bit_cast(half4, r);
-}
-__device__ __forceinline__ half8 lds_read_row(uint32_t at) {
-    typedef __attribute__((address_space(3))) const half8* lds_ptr;
-    return *(lds_ptr)(uintptr_t)at;
-}
 // What becomes of the sums: fp16 to `out`; fp32 to partial[split], for the consumer to add up; or, with W's columns [0, n / 2) gates and
 // [n / 2, n) up projections, SwiGLU of the two products rounded to fp16 -- what the separate kernel computes from the stored product, same
 // bits -- to `out` [m, n / 2].

@@ -1,5 +1,5 @@
-// What the tiled products (linear_tiled.h, linear_tiled_f32.h) share: loads from memory straight into LDS and loops whose index is a
-// constant.
+// What the tiled products (linear_tiled.h, linear_tiled_f32.h) and the attention of prompts share: loads from memory straight into LDS,
+// reads of matrix operands from there, and loops whose index is a constant.
 #pragma once
 
 #include <type_traits>
@@ -8,6 +8,8 @@
 
 namespace isp {
 
+typedef _Float16 half8 __attribute__((ext_vector_type(8)));
+typedef _Float16 half4 __attribute__((ext_vector_type(4)));
 typedef float float4v __attribute__((ext_vector_type(4)));
 
 template <int N, int I = 0, typename F>
@@ -28,6 +30,16 @@ __device__ __forceinline__ void load_to_lds(uint32_t lds, const void* base, uint
 template <int N>
 __device__ __forceinline__ void wait_loads() {
     asm volatile("s_waitcnt vmcnt(%0)" : : "n"(N) : "memory");
+}
+__device__ __forceinline__ half4 lds_read_transposed(uint32_t at) {
+    typedef short short4v __attribute__((ext_vector_type(4)));
+    typedef __attribute__((address_space(3))) short4v* lds_ptr;
+    const short4v r = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)(uintptr_t)at);
+    return __builtin_bit_cast(half4, r);
+}
+__device__ __forceinline__ half8 lds_read_row(uint32_t at) {
+    typedef __attribute__((address_space(3))) const half8* lds_ptr;
+    return *(lds_ptr)(uintptr_t)at;
 }
 __device__ __forceinline__ void lds_clear16(uint32_t at) {
     typedef __attribute__((address_space(3))) float4v* lds_ptr;

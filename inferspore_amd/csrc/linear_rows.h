@@ -193,6 +193,13 @@ void launch_tiled(const TiledPlan& plan, const __half* a, const __half* w, __hal
 void launch_tiled_swiglu(const TiledPlan& plan, const __half* a, const __half* gate_up, __half* out, int m, int inter, int k,
                          hipStream_t stream);
 
+// The same in fp32 (linear_tiled_f32.h).  `us`: what the plan is estimated to take, the addition of its splits included.
+TiledPlan tiled_plan_f32(int m, int n, int k, int max_splits, double* us);
+void launch_tiled_f32(const TiledPlan& plan, const float* a, const float* w, float* out_or_partial, int m, int n, int k, hipStream_t stream);
+// out[m, inter] = SwiGLU of the product with gate_up [k, 2 inter]; a plan without splits
+void launch_tiled_swiglu_f32(const TiledPlan& plan, const float* a, const float* gate_up, float* out, int m, int inter, int k,
+                             hipStream_t stream);
+
 // Either, for the rows that it is made for.  A skinny product's sums end in the order of its wavefronts, a tiled one's in the order of k.
 struct ProductPlan {
     bool tiled;
@@ -258,6 +265,19 @@ __device__ __forceinline__ vec16 add_splits8(const float* p, size_t stride, int 
     add_splits(at, stride, splits, sum);
     return pack_sums(sum[0], sum[1]);
 }
+// 16 bytes of the product that the splits make up
+template <typename T>
+__device__ __forceinline__ vec16 add_splits_vector(const float* p, size_t stride, int splits) {
+    if constexpr (sizeof(T) == 2) {
+        return add_splits8(p, stride, splits);
+    } else {
+        const float* const at[1] = {p};
+        float4v sum[1];
+        add_splits(at, stride, splits, sum);
+        const float f[4] = {sum[0][0], sum[0][1], sum[0][2], sum[0][3]};
+        return Elem<float>::pack(f);
+    }
+}
 __device__ __forceinline__ void add_splits8(const float* p, const float* q, size_t stride, int splits, vec16& first, vec16& second) {
     const float* const at[4] = {p, p + 4, q, q + 4};
     float4v sum[4];
@@ -272,9 +292,10 @@ void launch_qkv_sums(const float* partial, int splits, const __half* bias, __hal
                      const int32_t* padding_offset, const int32_t* history_length, const int32_t* input_length, int batch,
                      int seq_len, int tokens, int head_num, int kv_head_num, int head_size, int max_seq_len, int rot, float base,
                      hipStream_t stream);
-void launch_norm_sums(const float* partial, int splits, __half* residual, __half* out, const __half* gamma, float eps,
-                      int tokens, int hidden, hipStream_t stream);
-constexpr int kNormSumsMaxHidden = 8192;
+template <typename T>
+void launch_norm_sums(const float* partial, int splits, T* residual, T* out, const T* gamma, float eps, int tokens, int hidden,
+                      hipStream_t stream);
+constexpr int kNormSumsMaxHidden = 8192;  // in fp16: a vector per lane
 void launch_swiglu_sums(const float* partial, int splits, __half* out, int tokens, int inter, hipStream_t stream);
 
 // csrc/context_attention.hip

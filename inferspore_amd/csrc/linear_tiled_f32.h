@@ -20,8 +20,9 @@ namespace isp {
 
 constexpr int kTiledStepF32 = 32;  // k per step
 
-// Sums of steps [blockIdx.y * steps_per_split, ...) to out[blockIdx.y][m][n].
-template <int BM, int BN, int WAVES_M, int WAVES_N, int STAGES>
+// Sums of steps [blockIdx.y * steps_per_split, ...) to out[blockIdx.y][m][n]; or, with W's columns [0, n / 2) gates and [n / 2, n) up
+// projections, SwiGLU of the two products -- what the separate kernel computes from the stored product, same bits -- to out [m, n / 2].
+template <int BM, int BN, int WAVES_M, int WAVES_N, int STAGES, bool SWIGLU>
 __global__ __launch_bounds__(kWave* WAVES_M* WAVES_N, 2) void linear_tiled_f32(const float* __restrict__ a, const float* __restrict__ w,
                                                                                float* __restrict__ out, int m, int n, int k,
                                                                                int steps_per_split) {
@@ -39,8 +40,9 @@ __global__ __launch_bounds__(kWave* WAVES_M* WAVES_N, 2) void linear_tiled_f32(c
 
     const int tid = threadIdx.x, lane = tid % kWave, wave = __builtin_amdgcn_readfirstlane(tid / kWave), j = lane % 16, g = lane / 16;
     const int wm = wave / WAVES_N, wn = wave % WAVES_N;
-    const TilePlace place = place_tile((m + BM - 1) / BM, (n + BN - 1) / BN);
-    const int m0 = place.row * BM, n0 = place.col * BN;
+    const int result_cols = SWIGLU ? BN / 2 : BN, width = SWIGLU ? n / 2 : n;
+    const TilePlace place = place_tile((m + BM - 1) / BM, (width + result_cols - 1) / result_cols);
+    const int m0 = place.row * BM, n0 = place.col * result_cols;
 
     const int steps = (k + kTiledStepF32 - 1) / kTiledStepF32;
     const int first = (int)blockIdx.y * steps_per_split, last = min(steps, first + steps_per_split), count = last - first;
@@ -58,7 +60,12 @@ __global__ __launch_bounds__(kWave* WAVES_M* WAVES_N, 2) void linear_tiled_f32(c
 #pragma unroll
     for (int i = 0; i < LW; i++) {
         const int at = (wave * LW + i) * kWave + lane, r = at / CW, c = at % CW ^ w_swizzle(r);
-        w_off[i] = ((uint32_t)r * (uint32_t)n + (uint32_t)min(n0 + 4 * c, n - 4)) * 4u;
+        int col = min(n0 + 4 * c, width - 4);
+        if constexpr (SWIGLU) {  // a wavefront's columns: half of them gates, then the same columns' up projections
+            const int of_wave = c / (TN / 4), in_wave = c % (TN / 4), half = in_wave / (TN / 8);
+            col = min(n0 + of_wave * (TN / 2) + 4 * (in_wave % (TN / 8)), width - 4) + half * width;
+        }
+        w_off[i] = ((uint32_t)r * (uint32_t)n + (uint32_t)col) * 4u;
     }
     const char* a_next = reinterpret_cast<const char*>(a + (size_t)m0 * (size_t)k + (size_t)first * kTiledStepF32);
     const char* w_next = reinterpret_cast<const char*>(w + (size_t)first * kTiledStepF32 * (size_t)n);
@@ -198,6 +205,34 @@ __global__ __launch_bounds__(kWave* WAVES_M* WAVES_N, 2) void linear_tiled_f32(c
 
     // ---- lane (j, g) holds rows 4 g ... 4 g + 3 of every block and its NI neighbouring columns
     typedef float cols __attribute__((ext_vector_type(NI)));
+    if constexpr (SWIGLU) {  // lane j has eight lanes' gates, lane j ^ 8 the up projections: each computes two of the four rows
+        static_assert(NI >= 2, "sixteen columns would hold no whole chunk of both");
+        const bool gates = j < 8;
+        const int col = n0 + wn * (TN / 2) + NI * (j % 8);
+#pragma unroll
+        for (int x = 0; x < MI; x++) {
+            float own[4][NI], other[4][NI];
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+#pragma unroll
+                for (int y = 0; y < NI; y++) {
+                    own[r][y] = acc[0][x][y][r] + acc[1][x][y][r];
+                    other[r][y] = dpp_mov<0x128>(own[r][y]);  // row_ror:8
+                }
+#pragma unroll
+            for (int r = 0; r < 2; r++) {
+                const int row = m0 + wm * TM + 16 * x + 4 * g + (gates ? r : r + 2);
+                cols v;
+#pragma unroll
+                for (int y = 0; y < NI; y++) {
+                    const float gate = gates ? own[r][y] : other[r + 2][y], up = gates ? other[r][y] : own[r + 2][y];
+                    v[y] = silu_for<float>(gate) * up;
+                }
+                if (row < m && col < width) *reinterpret_cast<cols*>(out + (size_t)row * (size_t)width + col) = v;
+            }
+        }
+        return;
+    }
     float* mine = out + (size_t)blockIdx.y * (size_t)m * (size_t)n;
     const int col = n0 + wn * TN + NI * j;
     if (col >= n) return;  // n is a multiple of 4: NI columns exist together

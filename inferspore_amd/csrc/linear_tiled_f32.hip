@@ -27,7 +27,7 @@ constexpr TiledTileF32 kTilesF32[] = {
     {160, 64, 2, 3.18f, 1.128f, 1.088f, 2.54f, 6.30f},
 };
 
-static TiledPlan tiled_plan_f32(int m, int n, int k) {
+TiledPlan tiled_plan_f32(int m, int n, int k, int max_splits, double* us_of_plan) {
     const int steps = (k + kTiledStepF32 - 1) / kTiledStepF32, units = resident_waves() / 32;
     const double mn = (double)m * n, weight_bytes = 4.0 * n * k;
     TiledPlan best = {0, 1, steps};
@@ -37,7 +37,7 @@ static TiledPlan tiled_plan_f32(int m, int n, int k) {
         if (tile.rows >= 2 * m && tile.rows > 32) continue;  // rows of a tile that do not exist are work for nothing
         const long long tiles = ((m + tile.rows - 1ll) / tile.rows) * ((n + tile.cols - 1) / tile.cols), slots = (long long)units * tile.per_unit;
         const double stream = 2.0 + weight_bytes / tile.stream_tb * 1e-6;
-        for (int s = 1; s <= kTiledMaxSplits && (s == 1 || (2 * s <= steps && tiles * (s - 1) < slots)); s++) {
+        for (int s = 1; s <= max_splits && (s == 1 || (2 * s <= steps && tiles * (s - 1) < slots)); s++) {
             const int per = (steps + s - 1) / s;
             if (s > 1 && per * (s - 1) >= steps) continue;  // the same as a smaller number
             const long long groups = tiles * s, whole = groups / slots, rest = groups - whole * slots;
@@ -55,6 +55,7 @@ static TiledPlan tiled_plan_f32(int m, int n, int k) {
             }
         }
     }
+    if (us_of_plan) *us_of_plan = best_us;
     return best;
 }
 
@@ -74,14 +75,16 @@ static bool linear_shape_f32(int m, int n, int k) {
     return k > 0 && n % 4 == 0 && k % 4 == 0 && n <= kTiledMaxExtent && k <= kTiledMaxExtent && (long long)m * n < 0x3ffffff00ll;
 }
 
+template <bool SWIGLU>
 static void launch_f32(const TiledPlan& plan, const float* a, const float* w, float* out, int m, int n, int k, hipStream_t stream) {
     const TiledTileF32& tile = kTilesF32[plan.tile];
-    const dim3 grid((unsigned)((m + tile.rows - 1ll) / tile.rows) * (unsigned)((n + tile.cols - 1) / tile.cols), (unsigned)plan.splits);
+    const int cols = SWIGLU ? tile.cols / 2 : tile.cols, width = SWIGLU ? n / 2 : n;
+    const dim3 grid((unsigned)((m + tile.rows - 1ll) / tile.rows) * (unsigned)((width + cols - 1) / cols), (unsigned)plan.splits);
 #define ISP_TILED(INDEX, BM, BN, WM, WN, STAGES)                                                                              \
     case INDEX:                                                                                                               \
         static_assert(kTilesF32[INDEX].rows == BM && kTilesF32[INDEX].cols == BN, "tile");                                    \
-        hipLaunchKernelGGL((linear_tiled_f32<BM, BN, WM, WN, STAGES>), grid, dim3(kWave * WM * WN), 0, stream, a, w, out, m, n, k, \
-                           plan.steps_per_split);                                                                             \
+        hipLaunchKernelGGL((linear_tiled_f32<BM, BN, WM, WN, STAGES, SWIGLU>), grid, dim3(kWave * WM * WN), 0, stream, a, w, out, m,  \
+                           n, k, plan.steps_per_split);                                                                       \
         break
     switch (plan.tile) {
         ISP_TILED(0, 32, 64, 2, 2, 4);
@@ -93,6 +96,15 @@ static void launch_f32(const TiledPlan& plan, const float* a, const float* w, fl
 #undef ISP_TILED
 }
 
+void launch_tiled_f32(const TiledPlan& plan, const float* a, const float* w, float* out_or_partial, int m, int n, int k, hipStream_t stream) {
+    launch_f32<false>(plan, a, w, out_or_partial, m, n, k, stream);
+}
+
+void launch_tiled_swiglu_f32(const TiledPlan& plan, const float* a, const float* gate_up, float* out, int m, int inter, int k,
+                             hipStream_t stream) {
+    launch_f32<true>(plan, a, gate_up, out, m, 2 * inter, k, stream);
+}
+
 static int linear_f32(const float* a, const float* w, float* out, float* workspace, int m, int n, int k, hipStream_t stream) {
     if (m < 0 || n < 0 || k < 0) return ISP_ERR_BAD_SHAPE;
     if (m == 0 || n == 0) return ISP_OK;
@@ -101,12 +113,12 @@ static int linear_f32(const float* a, const float* w, float* out, float* workspa
     ISP_REQUIRE_PTR(w);
     ISP_REQUIRE_PTR(out);
     if (!aligned16(a) || !aligned16(w) || !aligned16(out)) return ISP_ERR_UNSUPPORTED;
-    const TiledPlan plan = tiled_plan_f32(m, n, k);
+    const TiledPlan plan = tiled_plan_f32(m, n, k, kTiledMaxSplits, nullptr);
     if (plan.splits > 1) {
         ISP_REQUIRE_PTR(workspace);
         if (!aligned16(workspace)) return ISP_ERR_UNSUPPORTED;
     }
-    launch_f32(plan, a, w, plan.splits > 1 ? workspace : out, m, n, k, stream);
+    launch_f32<false>(plan, a, w, plan.splits > 1 ? workspace : out, m, n, k, stream);
     const int status = note_launch(hipGetLastError());
     if (status != ISP_OK || plan.splits == 1) return status;
     const unsigned quads = (unsigned)((size_t)m * (size_t)n / 4);
@@ -121,7 +133,7 @@ extern "C" {
 
 size_t isp_linear_rows_f32_workspace(int m, int n, int k) {
     if (m <= 0 || n <= 0 || k <= 0 || !isp::linear_shape_f32(m, n, k)) return 0;
-    const isp::TiledPlan plan = isp::tiled_plan_f32(m, n, k);
+    const isp::TiledPlan plan = isp::tiled_plan_f32(m, n, k, isp::kTiledMaxSplits, nullptr);
     return plan.splits == 1 ? 0 : (size_t)plan.splits * (size_t)m * (size_t)n * sizeof(float);
 }
 
@@ -132,7 +144,7 @@ int isp_linear_rows_f32(const void* a, const void* w, void* out, void* workspace
 
 int isp_linear_rows_f32_plan(int m, int n, int k, int* tile_rows, int* tile_cols, int* splits) {
     if (m <= 0 || n <= 0 || k <= 0 || !isp::linear_shape_f32(m, n, k)) return ISP_ERR_BAD_SHAPE;
-    const isp::TiledPlan plan = isp::tiled_plan_f32(m, n, k);
+    const isp::TiledPlan plan = isp::tiled_plan_f32(m, n, k, isp::kTiledMaxSplits, nullptr);
     *tile_rows = isp::kTilesF32[plan.tile].rows;
     *tile_cols = isp::kTilesF32[plan.tile].cols;
     *splits = plan.splits;

@@ -56,22 +56,24 @@ template NormFewKernel<__half> norm_few_variant<__half>(int, int, int, int);
 
 // Residual + RMSNorm of a product left as partial sums [splits][tokens][hidden]: a row per workgroup, one vector per lane;
 // the operations and their order are norm_rows_body's (absent waves add exact zeros), so the bits are too.
-__global__ __launch_bounds__(1024) void fused_norm_sums_f16(const float* __restrict__ partial, int splits, __half* __restrict__ residual,
-                                                            __half* __restrict__ out, const __half* __restrict__ gamma, float eps,
-                                                            int tokens, int hidden) {
+template <typename T>
+__global__ __launch_bounds__(1024) void fused_norm_sums(const float* __restrict__ partial, int splits, T* __restrict__ residual,
+                                                        T* __restrict__ out, const T* __restrict__ gamma, float eps, int tokens,
+                                                        int hidden) {
+    constexpr int VEC = Elem<T>::kVec;
     __shared__ float sums[16];
     const int tid = threadIdx.x, waves = blockDim.x / kWave;
-    const bool ok = tid * 8 < hidden;
-    const size_t at = (size_t)blockIdx.x * (size_t)hidden + (size_t)(ok ? tid : 0) * 8u;
-    const vec16 vr = load16(residual + at), vg = load16(gamma + (ok ? tid : 0) * 8);
-    const vec16 vo = add_splits8(partial + at, (size_t)tokens * (size_t)hidden, splits);
-    float x[8];
-    Elem<__half>::sum(vo, vr, x);
+    const bool ok = tid * VEC < hidden;
+    const size_t at = (size_t)blockIdx.x * (size_t)hidden + (size_t)(ok ? tid : 0) * (unsigned)VEC;
+    const vec16 vr = load16(residual + at), vg = load16(gamma + (ok ? tid : 0) * VEC);
+    const vec16 vo = add_splits_vector<T>(partial + at, (size_t)tokens * (size_t)hidden, splits);
+    float x[VEC];
+    Elem<T>::sum(vo, vr, x);
 #pragma unroll
-    for (int e = 0; e < 8; e++) x[e] = Elem<__half>::pinned(x[e]);
+    for (int e = 0; e < VEC; e++) x[e] = Elem<T>::pinned(x[e]);
     float p = x[0] * x[0];
 #pragma unroll
-    for (int e = 1; e < 8; e++) p = __fmaf_rn(x[e], x[e], p);
+    for (int e = 1; e < VEC; e++) p = __fmaf_rn(x[e], x[e], p);
     p = wave_sum(ok ? p : 0.0f);
     if (tid % kWave == 0) sums[tid / kWave] = p;
     __syncthreads();
@@ -80,19 +82,22 @@ __global__ __launch_bounds__(1024) void fused_norm_sums_f16(const float* __restr
     for (int w = 0; w < 16; w++) part[w] = w < waves ? sums[w] : 0.0f;
     const float inv = rsqrtf(tree_sum<16>(part) / (float)hidden + eps);
     if (!ok) return;
-    store16(residual + at, Elem<__half>::pack_pinned(x));
-    float y[8];
-    Elem<__half>::scale(vg, x, y);
+    store16(residual + at, Elem<T>::pack_pinned(x));
+    float y[VEC];
+    Elem<T>::scale(vg, x, y);
 #pragma unroll
-    for (int e = 0; e < 8; e++) y[e] *= inv;
-    store16(out + at, Elem<__half>::pack(y));
+    for (int e = 0; e < VEC; e++) y[e] *= inv;
+    store16(out + at, Elem<T>::pack(y));
 }
 
-void launch_norm_sums(const float* partial, int splits, __half* residual, __half* out, const __half* gamma, float eps,
-                      int tokens, int hidden, hipStream_t stream) {
-    const unsigned threads = (unsigned)((hidden / 8 + kWave - 1) / kWave * kWave);
-    hipLaunchKernelGGL(fused_norm_sums_f16, dim3((unsigned)tokens), dim3(threads), 0, stream, partial, splits, residual, out,
-                       gamma, eps, tokens, hidden);
+template <typename T>
+void launch_norm_sums(const float* partial, int splits, T* residual, T* out, const T* gamma, float eps, int tokens, int hidden,
+                      hipStream_t stream) {
+    const unsigned threads = (unsigned)((hidden / Elem<T>::kVec + kWave - 1) / kWave * kWave);
+    hipLaunchKernelGGL(fused_norm_sums<T>, dim3((unsigned)tokens), dim3(threads), 0, stream, partial, splits, residual, out, gamma,
+                       eps, tokens, hidden);
 }
+template void launch_norm_sums<__half>(const float*, int, __half*, __half*, const __half*, float, int, int, hipStream_t);
+template void launch_norm_sums<float>(const float*, int, float*, float*, const float*, float, int, int, hipStream_t);
 
 }  // namespace isp

@@ -73,7 +73,11 @@ def test_what_the_products_refuse(isp):
 LAYERS = [([1], [0], 2, 2, 64, 12, 1, 16, 64, False, 36),
           ([100, 0, 31], [3, 9, 0], 4, 2, 128, 1000, 100, 128, 96, True, 520),
           ([300, 299], [50, 0], 6, 3, 96, 1540, 300, 384, 96, True, 572),
-          ([1] * 70, [7] * 70, 16, 2, 128, 4112, 1, 16, 128, False, 2048)]
+          ([1] * 70, [7] * 70, 16, 2, 128, 4112, 1, 16, 128, False, 2048),
+          # the gate / up product with SwiGLU inside, on each of the tiles; a last one with rows too wide for the norm to add splits
+          ([1], [0], 1, 1, 64, 4, 1, 16, 64, False, 44), ([30, 3], [0, 0], 1, 1, 64, 4124, 30, 32, 64, False, 36),
+          ([100, 63], [0, 0], 1, 1, 64, 4132, 100, 128, 64, False, 36), ([65], [0], 1, 1, 64, 2732, 65, 128, 64, False, 36),
+          ([300, 60], [0, 0], 1, 1, 64, 2716, 300, 320, 64, False, 68), ([5, 4], [0, 3], 33, 3, 128, 200, 5, 16, 128, False, 4224)]
 
 
 @pytest.mark.parametrize("case", range(len(LAYERS)))

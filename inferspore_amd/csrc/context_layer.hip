@@ -26,7 +26,7 @@ static LayerPlans layer_plans(int batch, int tokens, int hidden, int head_num, i
     LayerPlans p;
     p.qkv = product_plan(tokens, width, hidden, splits);
     p.o = product_plan(tokens, hidden, ctx, norm_splits);
-    p.gate_up = product_plan(tokens, 2 * inter, hidden, splits);
+    p.gate_up = product_plan(tokens, 2 * inter, hidden, splits, true);
     p.down = product_plan(tokens, hidden, inter, norm_splits);
     p.bytes = attention_workspace(batch, head_num, kv_head_num, head_size, max_q_len, max_k_len);
     const size_t sizes[] = {p.qkv.bytes(tokens, width), p.o.splits() == 1 ? 0 : p.o.bytes(tokens, hidden),

@@ -182,7 +182,7 @@ void launch_skinny(const SkinnyPlan& plan, const __half* a, const __half* w, __h
 struct TiledPlan {
     int tile, splits, steps_per_split;
 };
-TiledPlan tiled_plan(int m, int n, int k, int max_splits);
+TiledPlan tiled_plan(int m, int n, int k, int max_splits, bool swiglu);
 void tiled_extents(const TiledPlan& plan, int* rows, int* cols);
 constexpr int kTiledMaxSplits = 16;
 constexpr int kTiledMaxExtent = 1 << 22;  // of n and k: a tile's rows of A and of W are addressed in 32 bits
@@ -213,9 +213,10 @@ struct ProductPlan {
     }
 };
 constexpr int kSkinnyRows = 16;  // up to here
-inline ProductPlan product_plan(int m, int n, int k, int max_splits = kTiledMaxSplits) {
+// swiglu: a plan without splits computes SwiGLU
+inline ProductPlan product_plan(int m, int n, int k, int max_splits = kTiledMaxSplits, bool swiglu = false) {
     ProductPlan p = {m > kSkinnyRows, {}, {}};
-    if (p.tiled) p.tile = tiled_plan(m, n, k, max_splits);
+    if (p.tiled) p.tile = tiled_plan(m, n, k, max_splits, swiglu);
     else p.skinny = skinny_plan(m, n, k);
     return p;
 }

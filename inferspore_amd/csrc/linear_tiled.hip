@@ -10,20 +10,25 @@ namespace isp {
 // share one (tiles of up to 80 KiB of LDS); the weights arrive at stream_tb TB/s at most.  Fitted (mean error 7 to 9 %) to 1970
 // products of 17 ... 8192 rows over the layers of models of 512 ... 5120 columns, each with every tile and up to sixteen splits.  The plan
 // that these figures choose is 2 % behind the best of all (geometric mean; 10 % in one of twenty).
+// swiglu: steps of a product with SwiGLU inside take so much longer.  The wavefronts of 128 x 192 own 96 columns, in which gates and up
+// projections alternate 32 bytes at a time, not 64: 1.34 to 1.69 us per step and pair, not 1.22.  Without the factor 660 x 4096 x 22016 took
+// 173 us there (128 x 256: 152), 463 rows 104 (256 x 256: 100), 300 rows 93 (192 x 256: 86).  The 192 x 256 tile's step is not the
+// fit's 1.166: at 200 to 256 workgroups, for which it is mostly taken, it measures 1.21 to 1.26 (2611 x 4096 x 4096 87.1 us, 128 x 192 82.8;
+// x 11008 x 4096 219.6 and 213.1).
 struct TiledTile {
     int rows, cols, threads, per_unit;
-    float start_us, step_us, pair_us, stream_tb, partial_tb;
+    float start_us, step_us, pair_us, stream_tb, partial_tb, swiglu;
 };
 constexpr TiledTile kTiles[] = {
-    {256, 256, 512, 1, 8.38f, 1.301f, 0.0f, 3.62f, 7.59f}, {192, 256, 512, 1, 6.67f, 1.166f, 0.0f, 3.51f, 7.83f},
-    {256, 128, 512, 1, 5.16f, 0.731f, 0.0f, 3.41f, 5.88f}, {128, 256, 512, 1, 5.65f, 0.757f, 0.0f, 3.63f, 6.50f},
-    {128, 192, 256, 2, 4.01f, 0.887f, 1.216f, 4.09f, 5.10f}, {128, 128, 512, 1, 3.65f, 0.493f, 0.0f, 3.46f, 5.76f},
-    {128, 64, 256, 2, 2.21f, 0.382f, 0.645f, 3.59f, 5.15f}, {64, 128, 256, 2, 2.43f, 0.430f, 0.730f, 4.89f, 5.40f},
-    {64, 64, 256, 2, 1.98f, 0.284f, 0.457f, 4.25f, 5.79f}, {32, 128, 256, 2, 2.14f, 0.357f, 0.560f, 4.88f, 5.78f},
+    {256, 256, 512, 1, 8.38f, 1.301f, 0.0f, 3.62f, 7.59f, 1.0f}, {192, 256, 512, 1, 6.67f, 1.21f, 0.0f, 3.51f, 7.83f, 1.0f},
+    {256, 128, 512, 1, 5.16f, 0.731f, 0.0f, 3.41f, 5.88f, 1.0f}, {128, 256, 512, 1, 5.65f, 0.757f, 0.0f, 3.63f, 6.50f, 1.0f},
+    {128, 192, 256, 2, 4.01f, 0.887f, 1.216f, 4.09f, 5.10f, 1.25f}, {128, 128, 512, 1, 3.65f, 0.493f, 0.0f, 3.46f, 5.76f, 1.0f},
+    {128, 64, 256, 2, 2.21f, 0.382f, 0.645f, 3.59f, 5.15f, 1.0f}, {64, 128, 256, 2, 2.43f, 0.430f, 0.730f, 4.89f, 5.40f, 1.0f},
+    {64, 64, 256, 2, 1.98f, 0.284f, 0.457f, 4.25f, 5.79f, 1.0f}, {32, 128, 256, 2, 2.14f, 0.357f, 0.560f, 4.88f, 5.78f, 1.0f},
 };
 constexpr int kTileCount = sizeof(kTiles) / sizeof(kTiles[0]);
 
-TiledPlan tiled_plan(int m, int n, int k, int max_splits) {
+TiledPlan tiled_plan(int m, int n, int k, int max_splits, bool swiglu) {
     const int steps = (k + kTiledStep - 1) / kTiledStep, units = resident_waves() / 32;
     const double mn = (double)m * n, weight_bytes = 2.0 * n * k;
     TiledPlan best = {0, 1, steps};
@@ -38,7 +43,8 @@ TiledPlan tiled_plan(int m, int n, int k, int max_splits) {
             const int per = (steps + s - 1) / s;
             if (s > 1 && per * (s - 1) >= steps) continue;  // the same as a smaller number
             const int groups = tiles * s, whole = groups / slots, rest = groups - whole * slots;
-            const double alone = tile.start_us + per * tile.step_us, paired = tile.start_us + per * tile.pair_us;
+            const double longer = swiglu && s == 1 ? per * tile.swiglu : per;
+            const double alone = tile.start_us + longer * tile.step_us, paired = tile.start_us + longer * tile.pair_us;
             double us;
             if (tile.per_unit == 1) us = (whole + (rest > 0)) * alone;
             else us = whole * paired + (rest > units ? paired : rest > 0 ? alone : 0.0);

@@ -17,7 +17,7 @@ SHAPES = [(17, 16, 8, 32, 128, False), (18, 16, 208, 32, 128, True), (31, 12296,
           (65, 1632, 4488, 64, 128, True), (129, 5984, 224, 128, 64, False), (132, 1832, 1976, 128, 64, True),
           (386, 4752, 584, 128, 128, False), (130, 3624, 3272, 128, 128, True), (644, 6040, 72, 128, 192, False),
           (393, 5384, 7112, 128, 192, True), (1330, 5528, 208, 128, 256, False), (137, 5472, 5232, 128, 256, True),
-          (3369, 3488, 72, 192, 256, False), (3590, 664, 6536, 192, 256, True), (3846, 1056, 464, 256, 128, False),
+          (3369, 3488, 72, 192, 256, False), (517, 6768, 3656, 192, 256, True), (3846, 1056, 464, 256, 128, False),
           (403, 2720, 4784, 256, 128, True), (2752, 4464, 72, 256, 256, False), (904, 4360, 3992, 256, 256, True)]
 
 

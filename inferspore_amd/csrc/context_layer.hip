@@ -21,13 +21,12 @@ struct LayerPlans {
 static LayerPlans layer_plans(int batch, int tokens, int hidden, int head_num, int kv_head_num, int head_size, int max_q_len,
                               int max_k_len, int inter) {
     const int width = (head_num + 2 * kv_head_num) * head_size, ctx = head_num * head_size;
-    // the kernels that add up splits take rows of up to kNormSumsMaxHidden columns and a grid row per token
-    const int splits = tokens > 65535 ? 1 : kTiledMaxSplits, norm_splits = hidden > kNormSumsMaxHidden ? 1 : splits;
+    const int splits = tokens > 65535 ? 1 : kTiledMaxSplits;  // the kernels that add them up have a grid row per token
     LayerPlans p;
     p.qkv = product_plan(tokens, width, hidden, splits);
-    p.o = product_plan(tokens, hidden, ctx, norm_splits);
+    p.o = product_plan(tokens, hidden, ctx, splits);
     p.gate_up = product_plan(tokens, 2 * inter, hidden, splits, true);
-    p.down = product_plan(tokens, hidden, inter, norm_splits);
+    p.down = product_plan(tokens, hidden, inter, splits);
     p.bytes = attention_workspace(batch, head_num, kv_head_num, head_size, max_q_len, max_k_len);
     const size_t sizes[] = {p.qkv.bytes(tokens, width), p.o.splits() == 1 ? 0 : p.o.bytes(tokens, hidden),
                             p.gate_up.tiled && p.gate_up.splits() == 1 ? 0 : p.gate_up.bytes(tokens, 2 * inter),
@@ -60,10 +59,17 @@ static int few_rows_shape(int tokens, int hidden, int head_num, int kv_head_num,
     return ISP_OK;
 }
 
-// residual + RMSNorm of a product: its partial sums, or what it has stored in `out`
+// residual + RMSNorm of a product: its partial sums, or what it has stored in `out`.  Rows of more than kNormSumsMaxHidden columns are wider
+// than the workgroup that adds and normalises one: their sums are added first, as behind a product of its own.
 static int layer_norm(const ProductPlan& plan, const float* sums, void* residual, void* out, const void* gamma, float eps, int tokens,
                       int hidden, hipStream_t stream) {
-    if (plan.splits() == 1)
+    const bool wide = hidden > kNormSumsMaxHidden;
+    if (wide && plan.splits() > 1) {
+        launch_add_splits(sums, plan.splits(), static_cast<__half*>(out), tokens, hidden, stream);
+        const int status = note_launch(hipGetLastError());
+        if (status != ISP_OK) return status;
+    }
+    if (wide || plan.splits() == 1)
         return isp_fused_add_bias_residual_rmsnorm_f16(residual, out, nullptr, gamma, eps, tokens, hidden, 0, stream);
     launch_norm_sums(sums, plan.splits(), static_cast<__half*>(residual), static_cast<__half*>(out), static_cast<const __half*>(gamma), eps,
                      tokens, hidden, stream);

@@ -37,6 +37,11 @@ __global__ __launch_bounds__(kBlock) void linear_add_splits(const float* __restr
     reinterpret_cast<uint2*>(out)[i] = make_uint2(*reinterpret_cast<const uint32_t*>(&lo), *reinterpret_cast<const uint32_t*>(&hi));
 }
 
+void launch_add_splits(const float* partial, int splits, __half* out, int m, int n, hipStream_t stream) {
+    const unsigned quads = (unsigned)((size_t)m * (size_t)n / 4);
+    hipLaunchKernelGGL(linear_add_splits, dim3((quads + kBlock - 1) / kBlock), dim3(kBlock), 0, stream, partial, out, quads, splits);
+}
+
 // Extents that the kernels can count: a few rows, or any number of them (the addition below indexes four values in 32 bits).
 static bool linear_shape(int m, int n, int k) {
     const int most = m <= kSkinnyMaxRows ? kSkinnyMaxExtent : kTiledMaxExtent;
@@ -59,9 +64,7 @@ static int linear(const __half* a, const __half* w, __half* out, float* workspac
     launch_product(plan, a, w, out, workspace, m, n, k, stream);
     const int status = note_launch(hipGetLastError());
     if (status != ISP_OK || plan.splits() == 1) return status;
-    const unsigned quads = (unsigned)((size_t)m * (size_t)n / 4);
-    hipLaunchKernelGGL(linear_add_splits, dim3((quads + kBlock - 1) / kBlock), dim3(kBlock), 0, stream, workspace, out, quads,
-                       plan.splits());
+    launch_add_splits(workspace, plan.splits(), out, m, n, stream);
     return note_launch(hipGetLastError());
 }
 

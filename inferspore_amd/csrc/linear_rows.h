@@ -287,6 +287,9 @@ __device__ __forceinline__ void add_splits8(const float* p, const float* q, size
     second = pack_sums(sum[2], sum[3]);
 }
 
+// out[m][n] = the splits' sum, rounded to fp16.  n is a multiple of 8, m n / 4 fits 32 bits.
+void launch_add_splits(const float* partial, int splits, __half* out, int m, int n, hipStream_t stream);
+
 // Consumers of partial sums: what the entry points of the same step do with a stored fp16 product (same bits), with that
 // product's addition of splits, its store and its read back taken out.  Operands checked by the caller.
 void launch_qkv_sums(const float* partial, int splits, const __half* bias, __half* q, __half* k_cache, __half* v_cache,

@@ -16,7 +16,11 @@ CASES = [([1], [0], 2, 2, 64, 264, 1, 8, 64, False, 128),
          ([1, 4], [50, 0], 6, 3, 96, 392, 4, 64, 96, True, 576),
          ([64], [0], 12, 3, 128, 88, 64, 64, 128, False, 1536),
          ([1, 1, 1], [30, 31, 40], 16, 16, 64, 2816, 1, 32, 0, True, 1024),   # the last two sequences' rows are past the cache
-         ([2, 2], [100, 7], 64, 8, 128, 4096, 2, 128, 128, False, 8192)]
+         ([2, 2], [100, 7], 64, 8, 128, 4096, 2, 128, 128, False, 8192),
+         # rows wider than the kernel that adds splits and normalises takes: the splits are added by themselves
+         ([1], [9], 2, 2, 64, 264, 1, 16, 64, False, 8320),
+         ([1] * 16, list(range(16)), 2, 1, 128, 1040, 1, 32, 128, True, 10240),
+         ([9, 8], [0, 5], 2, 2, 128, 1040, 9, 32, 128, False, 8320)]
 
 
 @pytest.mark.parametrize("case", range(len(CASES)))

@@ -309,7 +309,7 @@ int isp_linear_f16(const void* a, const void* w, void* out, void* workspace, int
 /* The same for any number of rows (above 64: n and k up to 2^22), prompts included. */
 size_t isp_linear_rows_f16_workspace(int m, int n, int k);
 int isp_linear_rows_f16(const void* a, const void* w, void* out, void* workspace, int m, int n, int k, isp_stream_t stream);
-/* The tile of a workgroup (0 x 0: the kernel for up to 16 rows, whose workgroups take 128 columns) and the number of workgroups that
+/* The tile of a workgroup (0 x 0: the kernel for few rows, whose workgroups take all of them and 128 columns) and the number of workgroups that
  * share its k. */
 int isp_linear_rows_f16_plan(int m, int n, int k, int* tile_rows, int* tile_cols, int* splits);
 /* The same in fp32 throughout: n and k multiples of 4 up to 2^22. */

@@ -1,5 +1,5 @@
-// isp_linear_rows_f16: the product of activation rows with a weight matrix, up to 16 rows by the kernel in linear_rows.h, more by the tiles in
-// linear_tiled.h; isp_linear_f16: up to 64 of them.
+// isp_linear_rows_f16: the product of activation rows with a weight matrix, up to 16 rows by the kernel in linear_rows.h, more than 64 by the
+// tiles in linear_tiled.h, between them by whichever is priced lower (product_plan); isp_linear_f16: up to 64 of them.
 // The reference calls cuBLAS for it (src/kernels/linear.cu:7-66); the library here, hipBLASLt, reads the weights of a
 // 16-row product at 1.4-3.8 TB/s and those of a 64-row product at 1.2-1.8 (4.9 for the widest), these kernels at 4.3-5.5
 // and 3.1-5.4.

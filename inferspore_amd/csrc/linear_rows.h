@@ -10,6 +10,8 @@
 // order; workgroups that share a strip of columns write fp32 partial sums [splits][m][n] that the consumer adds in order.
 #pragma once
 
+#include <math.h>
+
 #include "isp_common.h"
 
 namespace isp {
@@ -182,7 +184,8 @@ void launch_skinny(const SkinnyPlan& plan, const __half* a, const __half* w, __h
 struct TiledPlan {
     int tile, splits, steps_per_split;
 };
-TiledPlan tiled_plan(int m, int n, int k, int max_splits, bool swiglu);
+// `us`: what the plan is estimated to take, the reading of its splits by whatever adds them included.
+TiledPlan tiled_plan(int m, int n, int k, int max_splits, bool swiglu, double* us);
 void tiled_extents(const TiledPlan& plan, int* rows, int* cols);
 constexpr int kTiledMaxSplits = 16;
 constexpr int kTiledMaxExtent = 1 << 22;  // of n and k: a tile's rows of A and of W are addressed in 32 bits
@@ -212,12 +215,39 @@ struct ProductPlan {
         return splits() == 1 ? values * sizeof(__half) : (size_t)splits() * values * sizeof(float);
     }
 };
-constexpr int kSkinnyRows = 16;  // up to here
+constexpr int kSkinnyRows = 16;  // the skinny kernel up to here, up to kSkinnyMaxRows whichever is priced lower
+// What a skinny product of 17 ... 64 rows takes, the reading of its splits included: rounds of one workgroup per compute unit, each start +
+// step per 128 k, against the weights' stream.  Fitted (mean error 3 to 4 %) to 1008 products of 17 to 64 rows, 1024 to 32768 columns and
+// 1024 to 14336 k.
+inline double skinny_us(const SkinnyPlan& plan, int m, int n, int k) {
+    constexpr double kStart[] = {4.3, 4.64, 4.93}, kStep[] = {0.648, 1.033, 1.209}, kStream[] = {6.47, 6.75, 6.82};
+    const int t = m <= 32 ? 0 : m <= 48 ? 1 : 2, waves = kBlock / kWave, units = resident_waves() / 32;
+    const double mn = (double)m * n, stream = 2.0 + 2.0 * n * k / kStream[t] * 1e-6;
+    const long long rounds = ((long long)plan.strips * plan.splits + units - 1) / units;
+    const double us = (double)rounds * (kStart[t] + (plan.steps_per_split + waves - 1) / waves * kStep[t]);
+    const double sums = plan.splits == 1 ? 0.0 : 4.0 * plan.splits * mn / 5.5 * 1e-6 + (4.0 * plan.splits - 2.0) * mn / 4.5 * 1e-6;
+    return sqrt(sqrt(us * us * us * us + stream * stream * stream * stream)) + sums;
+}
 // swiglu: a plan without splits computes SwiGLU
 inline ProductPlan product_plan(int m, int n, int k, int max_splits = kTiledMaxSplits, bool swiglu = false) {
     ProductPlan p = {m > kSkinnyRows, {}, {}};
-    if (p.tiled) p.tile = tiled_plan(m, n, k, max_splits, swiglu);
-    else p.skinny = skinny_plan(m, n, k);
+    if (m <= kSkinnyMaxRows) p.skinny = skinny_plan(m, n, k);
+    if (!p.tiled) return p;
+    double us;
+    p.tile = tiled_plan(m, n, k, max_splits, swiglu, &us);
+    if (m > kSkinnyMaxRows) return p;
+    // The skinny kernel reads the weights straight to registers, 5.8 to 6.5 TB/s where its strips fill whole rounds of compute units; the tiled
+    // one needs no whole rounds and feeds more rows.  us, skinny and tiled, additions included: 17 x 4096 x 28672 39.5, 43.1; 32 x 8192 x
+    // 8192 27.6, 30.7; 17 x 8192 x 32768 87.0, 91.2; 48 x 4096 x 12288 26.4, 24.1; 32 x 4096 x 22016 43.3, 36.0; 64 x 4096 x 28672 49.5,
+    // 43.3.  The tiles' prices are 1.11 to 1.18 times what they take here.  SwiGLU inside saves a launch (3 us), but reads two narrower streams, slowest where
+    // rows are whole multiples of 2 KiB: 17 x 4096 x 28672 49.7 against 39.8 and 5.0; a whole layer of 48 rows x 4096, inter 11008, 125 against 131.  With these
+    // factors 102 layers of 512 to 8192 columns are within 1 % of the better of the two in the mean.
+    double tiled = 0.9 * us, skinny = skinny_us(p.skinny, m, n, k);
+    if (swiglu && p.tile.splits == 1) {
+        tiled *= 2ll * n % 2048 == 0 ? 1.33 : 1.11;
+        skinny += 3.0;
+    }
+    p.tiled = tiled < skinny;
     return p;
 }
 // With several splits their sums to `partial`, else the fp16 product to `out`.

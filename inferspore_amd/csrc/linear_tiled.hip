@@ -28,7 +28,7 @@ constexpr TiledTile kTiles[] = {
 };
 constexpr int kTileCount = sizeof(kTiles) / sizeof(kTiles[0]);
 
-TiledPlan tiled_plan(int m, int n, int k, int max_splits, bool swiglu) {
+TiledPlan tiled_plan(int m, int n, int k, int max_splits, bool swiglu, double* us_of_plan) {
     const int steps = (k + kTiledStep - 1) / kTiledStep, units = resident_waves() / 32;
     const double mn = (double)m * n, weight_bytes = 2.0 * n * k;
     TiledPlan best = {0, 1, steps};
@@ -58,6 +58,7 @@ TiledPlan tiled_plan(int m, int n, int k, int max_splits, bool swiglu) {
             }
         }
     }
+    *us_of_plan = best_us;
     return best;
 }
 

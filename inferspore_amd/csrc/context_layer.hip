@@ -52,7 +52,8 @@ static int layer_shape(int layer, int batch, int tokens, int hidden, int head_nu
     return ISP_OK;
 }
 
-// What isp_context_layer_f16 has always been for: a few rows.
+// What isp_context_layer_f16 is for: a few rows, of products whose weights these kernels read faster than the library does (above 16 rows 32768
+// columns: 48 rows of 6144, inter 24576, take 295 us a layer here and 278 with the library's).
 static int few_rows_shape(int tokens, int hidden, int head_num, int kv_head_num, int head_size, int inter) {
     if (tokens > kSkinnyMaxRows || hidden > kNormSumsMaxHidden) return ISP_ERR_UNSUPPORTED;
     if (tokens > 16 && (2ll * inter > 32768 || ((long long)head_num + 2ll * kv_head_num) * head_size > 32768)) return ISP_ERR_UNSUPPORTED;

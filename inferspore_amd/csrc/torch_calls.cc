@@ -288,6 +288,16 @@ ISP_METHOD(repeat_kv_cache) {  // k_cache, v_cache, context_length, layer, k_dst
     });
 }
 
+// float16 layers that are faster step by step, with the library's product for what is wide: 17 to 64 rows where a product has more than 32768
+// columns, 65 to 192 rows where gate and up projections have more than 400 million weights.  us a layer, steps and one call: 48 rows x
+// 6144, inter 24576 278, 295; 40 x 10240, 27648, 8 key heads 411, 464; 96 x 8192, 28672 495, 554; 144 x 12288, 43008 1142, 1421.  Next to the
+// lines: 17 x 6144, 24576 262, 236; 40 x 5120, 13824 162, 159; 80 x 8192, 28672 544, 537; 128 x 8192, 22016 531, 491; 200 x 12288, 43008
+// 1480, 1308; 640 x 8192, 28672, the slowest above 192 rows, 1349, 1437.
+bool steps_are_faster(int rows, int64_t hidden, int64_t width, int64_t inter) {
+    if (rows <= 64) return rows > 16 && (2 * inter > 32768 || width > 32768);
+    return rows <= 192 && 2 * inter * hidden > 400000000;
+}
+
 // A whole layer: its output, a status that is not 0, or None.  normed, residual, qkv, qkv_bias, o, gate_up, down, ffn_norm, next_norm, q,
 // k_cache, v_cache, packed context, act, padding_offset, history, lengths, context lengths; layer, tokens, heads, kv_heads, head_size,
 // longest context, rotary_dim; base, eps.
@@ -316,7 +326,7 @@ ISP_METHOD(context_layer) {
         const Tensor* t = i < 14 ? f[i].t : lens[i - 14].t;
         if (t) c.need(t->device() == f[0].t->device() && (i >= 14 || ((uintptr_t)t->mutable_data_ptr() % 16 == 0 && !(grad && t->requires_grad()))));
     }
-    if (!c.plain || f[0].data() == f[1].data()) Py_RETURN_NONE;
+    if (!c.plain || f[0].data() == f[1].data() || (type == at::kHalf && steps_are_faster(tokens, hidden, width, inter))) Py_RETURN_NONE;
     const char *q = static_cast<const char*>(f[9].data()), *packed = static_cast<const char*>(f[12].data());
     if (packed >= q ? (size_t)(packed - q) < f[9].t->nbytes() : (size_t)(q - packed) < f[12].t->nbytes()) Py_RETURN_NONE;
     const size_t need = ISP_BY_TYPE_WITH(type, isp_context_layer_rows, _workspace)((int)batch, tokens, (int)hidden, heads, kv, hs, (int)max_q,

@@ -80,3 +80,20 @@ def test_a_few_tokens_among_thousands_of_empty_sequences(isp):
     out = cl._layer_in_one_call(x, x.clone(), w, st, 0, w.attn_norm, 64, 1e4, 1e-5)
     assert out is not None and torch.isfinite(out).all()
     assert torch.equal(st.packed_ctx[[0, 5], 0], st.v_cache[0, [0, 4199], 0, 0])   # a first token attends to itself
+
+
+@pytest.mark.parametrize("rows,hidden,inter,kv,one", [(16, 64, 16392, 1, True), (17, 64, 16392, 1, False), (64, 64, 16384, 1, True),
+                                                      (33, 64, 64, 171, False), (64, 64, 64, 170, True), (65, 64, 16392, 1, True),
+                                                      (65, 8192, 24416, 1, False), (192, 8192, 24416, 1, False),
+                                                      (193, 8192, 24416, 1, True), (192, 8192, 24408, 1, True)])
+def test_layers_that_are_faster_step_by_step(isp, rows, hidden, inter, kv, one):
+    """Few rows with wide products keep the library's product for them."""
+    from inferspore_amd import context_layer as cl
+    print("[case] route of %s" % ((rows, hidden, inter, kv),), flush=True)
+    zeros = lambda *s: torch.zeros(s, dtype=torch.float16, device="cuda")   # noqa: E731
+    w = cl.LayerWeights.__new__(cl.LayerWeights)
+    w.qkv, w.qkv_bias, w.o, w.gate_up = zeros(hidden, 3 * kv * 64), None, zeros(kv * 64, hidden), zeros(hidden, 2 * inter)
+    w.down, w.ffn_norm, w.attn_norm = zeros(inter, hidden), zeros(hidden), zeros(hidden)
+    st = cl.BatchState([1] * rows, 1, kv, kv, 64, inter, 1, 1, torch.float16)
+    x = zeros(rows, hidden)
+    assert (cl._layer_in_one_call(x, x.clone(), w, st, 0, w.attn_norm, 64, 1e4, 1e-5) is not None) == one

@@ -49,6 +49,8 @@ static int layer_shape(int layer, int batch, int tokens, int hidden, int head_nu
         return ISP_ERR_UNSUPPORTED;
     // the steps between the products index vectors of 16 bytes in 32 bits
     if ((long long)tokens * (widest > 2ll * inter ? widest : 2ll * inter) > 0xffffffffll) return ISP_ERR_UNSUPPORTED;
+    // the fp32 products are calls of their own: none may refuse once another has run
+    if (vector == 4 && (2ll * inter > kTiledMaxExtent || (long long)tokens * hidden >= kTiledMaxValues)) return ISP_ERR_UNSUPPORTED;
     return ISP_OK;
 }
 

@@ -72,7 +72,7 @@ __global__ __launch_bounds__(kBlock) void linear_add_splits_f32(const float* __r
 
 // Extents that the kernels can count (the addition indexes four values in 32 bits).
 static bool linear_shape_f32(int m, int n, int k) {
-    return k > 0 && n % 4 == 0 && k % 4 == 0 && n <= kTiledMaxExtent && k <= kTiledMaxExtent && (long long)m * n < 0x3ffffff00ll;
+    return k > 0 && n % 4 == 0 && k % 4 == 0 && n <= kTiledMaxExtent && k <= kTiledMaxExtent && (long long)m * n < kTiledMaxValues;
 }
 
 template <bool SWIGLU>

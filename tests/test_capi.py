@@ -196,3 +196,15 @@ def test_few_rows_keep_the_kernel_that_is_faster_for_them(lib, m, n, k):
     rows, cols, splits = ctypes.c_int(), ctypes.c_int(), ctypes.c_int()
     assert lib.isp_linear_rows_f16_plan(m, n, k, ctypes.byref(rows), ctypes.byref(cols), ctypes.byref(splits)) == 0
     assert (rows.value, cols.value) == (0, 0)
+
+
+def test_a_float32_layer_is_taken_only_if_all_its_products_are(lib):
+    """None of them may refuse after the ones before it have run."""
+    most = 2 ** 22
+    layer = lambda tokens, hidden, inter, heads=1: lib.isp_context_layer_rows_f32_workspace(   # noqa: E731
+        1, tokens, hidden, heads, heads, 64, tokens, tokens, tokens, inter)
+    for tokens, hidden, inter in ((1, 64, 64), (1, 64, most // 2), (1, 64, most // 2 + 4), (3, 4, most), (4100, most, 64), (4095, most, 64)):
+        products = ((tokens, 192, hidden), (tokens, hidden, 64), (tokens, 2 * inter, hidden), (tokens, hidden, inter))
+        a, b, s = ctypes.c_int(), ctypes.c_int(), ctypes.c_int()
+        taken = all(lib.isp_linear_rows_f32_plan(*p, ctypes.byref(a), ctypes.byref(b), ctypes.byref(s)) == 0 for p in products)
+        assert (layer(tokens, hidden, inter) != 0) == taken, (tokens, hidden, inter)

@@ -9,6 +9,7 @@
 #include <ATen/ATen.h>
 #include <ATen/autocast_mode.h>
 #include <ATen/PythonTorchFunctionTLS.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPStream.h>
 
 #include <initializer_list>
@@ -311,7 +312,8 @@ ISP_METHOD(context_layer) {
     const int layer = c.integer(18), tokens = c.integer(19), heads = c.integer(20), kv = c.integer(21), hs = c.integer(22),
               longest = c.integer(23), rotary = c.integer(24);
     const float base = c.number(25), eps = c.number(26);
-    c.need(c.plain && f[0].dim() == 2 && f[9].dim() == 4 && f[10].dim() == 5 && f[13].dim() == 2 && heads > 0 && kv > 0 && hs > 0);
+    // a dispatch mode (a counter of operations, a tracer) sees the products of the steps
+    c.need(c.plain && !c10::impl::dispatch_mode_enabled() && f[0].dim() == 2 && f[9].dim() == 4 && f[10].dim() == 5 && f[13].dim() == 2 && heads > 0 && kv > 0 && hs > 0);
     if (!c.plain) Py_RETURN_NONE;
     const int64_t hidden = f[0].size(1), batch = f[9].size(0), max_q = f[9].size(2), max_seq = f[10].size(3), inter = f[13].size(1),
                   width = ((int64_t)heads + 2ll * kv) * hs, context = (int64_t)heads * hs;

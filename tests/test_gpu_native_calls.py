@@ -121,3 +121,21 @@ def test_layer_takes_numbers_as_the_steps_do(isp):
         assert call() is not None
         with torch.autocast("cuda", torch.float16):
             assert call() is None
+
+
+@pytest.mark.parametrize("rows,dtype", [(100, torch.float16), (3, torch.float32)])
+def test_a_dispatch_mode_sees_the_products(isp, rows, dtype):
+    """torch's own counter of operations counts a layer's four products, whose library calls it sees in the steps."""
+    from torch.utils.flop_counter import FlopCounterMode
+
+    from inferspore_amd import context_layer as cl
+    hidden, inter = 128, 320
+    w = cl.LayerWeights(hidden, inter, dtype)
+    st = cl.BatchState([rows], rows, 2, 2, 64, inter, rows, 1, dtype)
+    x = torch.randn(rows, hidden, device="cuda").to(dtype)
+    with FlopCounterMode(display=False) as counter:
+        got = cl.context_decoder_layer(x, x.clone(), w, st, 0, w.attn_norm, rotary_dim=64)
+    assert counter.get_total_flops() == 2 * rows * (hidden * 3 * hidden + hidden * hidden + 3 * hidden * inter)
+    want = cl.context_decoder_layer(x, x.clone(), w, st, 0, w.attn_norm, rotary_dim=64)
+    # the library's sums and these: in float16 the four products are rounded to 2^-11 on either side
+    assert (got.float() - want.float()).abs().max() <= 2.0 ** -8 * want.float().abs().max()

@@ -306,13 +306,13 @@ int isp_context_attention_split_f16(const void* q, const void* k_cache, const vo
  */
 size_t isp_linear_f16_workspace(int m, int n, int k);
 int isp_linear_f16(const void* a, const void* w, void* out, void* workspace, int m, int n, int k, isp_stream_t stream);
-/* The same for any number of rows (above 64: n and k up to 2^22), prompts included. */
+/* The same for up to 2^30 - 1 rows (above 64: n and k up to 2^22; m n below 2^34 - 256), prompts included. */
 size_t isp_linear_rows_f16_workspace(int m, int n, int k);
 int isp_linear_rows_f16(const void* a, const void* w, void* out, void* workspace, int m, int n, int k, isp_stream_t stream);
 /* The tile of a workgroup (0 x 0: the kernel for few rows, whose workgroups take all of them and 128 columns) and the number of workgroups that
  * share its k. */
 int isp_linear_rows_f16_plan(int m, int n, int k, int* tile_rows, int* tile_cols, int* splits);
-/* The same in fp32 throughout: n and k multiples of 4 up to 2^22. */
+/* The same in fp32 throughout: n and k multiples of 4 up to 2^22, up to 2^29 - 1 rows. */
 size_t isp_linear_rows_f32_workspace(int m, int n, int k);
 int isp_linear_rows_f32(const void* a, const void* w, void* out, void* workspace, int m, int n, int k, isp_stream_t stream);
 int isp_linear_rows_f32_plan(int m, int n, int k, int* tile_rows, int* tile_cols, int* splits);

@@ -45,7 +45,7 @@ void launch_add_splits(const float* partial, int splits, __half* out, int m, int
 // Extents that the kernels can count: a few rows, or any number of them (the addition below indexes four values in 32 bits).
 static bool linear_shape(int m, int n, int k) {
     const int most = m <= kSkinnyMaxRows ? kSkinnyMaxExtent : kTiledMaxExtent;
-    return k > 0 && n % 8 == 0 && k % 8 == 0 && n <= most && k <= most && (long long)m * n < kTiledMaxValues;
+    return k > 0 && n % 8 == 0 && k % 8 == 0 && n <= most && k <= most && m <= kTiledMaxRows && (long long)m * n < kTiledMaxValues;
 }
 
 static int linear(const __half* a, const __half* w, __half* out, float* workspace, int m, int n, int k, hipStream_t stream) {

@@ -189,6 +189,8 @@ TiledPlan tiled_plan(int m, int n, int k, int max_splits, bool swiglu, double* u
 void tiled_extents(const TiledPlan& plan, int* rows, int* cols);
 constexpr int kTiledMaxSplits = 16;
 constexpr int kTiledMaxExtent = 1 << 22;  // of n and k: a tile's rows of A and of W are addressed in 32 bits
+// of m: the tiles of the fewest rows, 64 in fp16 and 32 in fp32, times 256 threads make a grid that can be launched
+constexpr int kTiledMaxRows = (1 << 30) - 1, kTiledMaxRowsF32 = (1 << 29) - 1;
 constexpr long long kTiledMaxValues = 0x3ffffff00ll;  // m n: the addition of splits counts four values in 32 bits
 // With plan.splits > 1 partial sums to `partial`, else the fp16 product to `out`.  Operands checked by the caller.
 void launch_tiled(const TiledPlan& plan, const __half* a, const __half* w, __half* out, float* partial, int m, int n, int k,

@@ -72,7 +72,8 @@ __global__ __launch_bounds__(kBlock) void linear_add_splits_f32(const float* __r
 
 // Extents that the kernels can count (the addition indexes four values in 32 bits).
 static bool linear_shape_f32(int m, int n, int k) {
-    return k > 0 && n % 4 == 0 && k % 4 == 0 && n <= kTiledMaxExtent && k <= kTiledMaxExtent && (long long)m * n < kTiledMaxValues;
+    return k > 0 && n % 4 == 0 && k % 4 == 0 && n <= kTiledMaxExtent && k <= kTiledMaxExtent && m <= kTiledMaxRowsF32 &&
+           (long long)m * n < kTiledMaxValues;
 }
 
 template <bool SWIGLU>

@@ -208,3 +208,16 @@ def test_a_float32_layer_is_taken_only_if_all_its_products_are(lib):
         a, b, s = ctypes.c_int(), ctypes.c_int(), ctypes.c_int()
         taken = all(lib.isp_linear_rows_f32_plan(*p, ctypes.byref(a), ctypes.byref(b), ctypes.byref(s)) == 0 for p in products)
         assert (layer(tokens, hidden, inter) != 0) == taken, (tokens, hidden, inter)
+
+
+@pytest.mark.parametrize("kind,most", [("f16", 2 ** 30 - 1), ("f32", 2 ** 29 - 1)])
+def test_products_refuse_more_rows_than_a_grid_holds(lib, kind, most):
+    from inferspore_amd import capi
+    plan, space, call = (getattr(lib, "isp_linear_rows_%s%s" % (kind, end)) for end in ("_plan", "_workspace", ""))
+    a, b, s = ctypes.c_int(), ctypes.c_int(), ctypes.c_int()
+    p = ctypes.c_void_p(16)   # never dereferenced: refused first
+    assert plan(most, 8, 8, ctypes.byref(a), ctypes.byref(b), ctypes.byref(s)) == 0
+    assert -(-most // a.value) * 256 < 2 ** 32
+    for m in (most + 1, 2 ** 31 - 40):
+        assert plan(m, 8, 8, ctypes.byref(a), ctypes.byref(b), ctypes.byref(s)) != 0
+        assert space(m, 8, 8) == 0 and call(p, p, p, p, m, 8, 8, None) == capi.ERR_UNSUPPORTED

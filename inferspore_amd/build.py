@@ -75,13 +75,33 @@ def _compile(src):
     return obj, out
 
 
+def _torch_version(torch_dir):
+    """torch.__version__ without importing it."""
+    names = {}
+    with open(os.path.join(torch_dir, "version.py")) as f:
+        exec(f.read(), names)
+    return names["__version__"]
+
+
 def _compile_calls():
-    """Host code only: torch's headers and libraries, the C ABI."""
-    torch_dir = os.path.dirname(importlib.util.find_spec("torch").origin)
+    """Host code only: torch's headers and libraries, the C ABI.  Where torch for ROCm, its headers or Python's are not installed there is
+    nothing to build it for: the libraries and the C++ programs do without, and so does ops.py, more slowly (capi.calls)."""
+    if os.path.exists(CALLS):
+        os.remove(CALLS)   # of another torch, perhaps
+    spec = importlib.util.find_spec("torch")
+    torch_dir = os.path.dirname(spec.origin) if spec is not None and spec.origin else None
+    python_include = sysconfig.get_paths()["include"]
+    needed = [os.path.join(python_include, "Python.h")]
+    if torch_dir:
+        needed += [os.path.join(torch_dir, "include", "ATen", "ATen.h"), os.path.join(torch_dir, "lib", "libc10_hip.so")]
+    if torch_dir is None or not all(os.path.exists(f) for f in needed):
+        print("torch for ROCm, its headers or Python's are not installed: %s is not built" % os.path.basename(CALLS))
+        return ""
     include, libs = os.path.join(torch_dir, "include"), os.path.join(torch_dir, "lib")
-    return _run(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", "-I" + INCLUDE,
+    return _run(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+                 '-DISP_TORCH_VERSION="%s"' % _torch_version(torch_dir), "-I" + INCLUDE,
                  "-isystem", include, "-isystem", os.path.join(include, "torch", "csrc", "api", "include"),
-                 "-isystem", sysconfig.get_paths()["include"], "-isystem", "/opt/rocm/include",
+                 "-isystem", python_include, "-isystem", "/opt/rocm/include",
                  os.path.join(CSRC, "torch_calls.cc"), "-o", CALLS, "-L" + LIBDIR, "-linferspore_amd", "-L" + libs, "-lc10", "-lc10_hip",
                  "-ltorch_cpu", "-ltorch_python", "-Wl,-rpath,$ORIGIN"])
 

@@ -3,6 +3,8 @@ import ctypes as C
 import importlib.machinery
 import importlib.util
 import os
+import sys
+import warnings
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "lib", "libinferspore_amd.so")
@@ -105,25 +107,42 @@ def lib():
 
 
 class _NoCalls:
-    """Stands for the module below where nothing has been built: every call is left to its general path, which raises."""
+    """Stands for the module below where there is none: every call is left to its general path, the same kernels through ctypes (which
+    raises where the library itself has not been built)."""
 
     def __getattr__(self, name):
         return lambda *args: None
+
+
+def _load_calls():
+    """The module, or why there is none for this interpreter."""
+    if not os.path.exists(CALLS_PATH):
+        return None, "it is not built"
+    lib()
+    import torch   # the module links to its libraries
+    loader = importlib.machinery.ExtensionFileLoader("_torch_calls", CALLS_PATH)
+    try:
+        module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_torch_calls", loader))
+        loader.exec_module(module)
+    except ImportError as e:
+        return None, str(e)
+    here = (str(torch.__version__),) + tuple(sys.version_info[:2])
+    if module.built_for != here:
+        return None, "it was built for torch %s, Python %d.%d" % module.built_for
+    return module, None
 
 
 def calls():
     """The native module that takes the calls on plain tensors (csrc/torch_calls.cc)."""
     global _calls
     if _calls is None:
-        if not os.path.exists(CALLS_PATH):
-            if os.path.exists(LIB_PATH):
-                raise RuntimeError("inferspore_amd: %s is missing -- build it with `python -m inferspore_amd.build`" % CALLS_PATH)
+        if not os.path.exists(LIB_PATH):
             return _NoCalls()
-        lib()
-        import torch  # noqa: F401  the module links to its libraries
-        loader = importlib.machinery.ExtensionFileLoader("_torch_calls", CALLS_PATH)
-        module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_torch_calls", loader))
-        loader.exec_module(module)
+        module, why = _load_calls()
+        if module is None:
+            warnings.warn("inferspore_amd: calls go through ctypes, several microseconds slower each, as %s cannot be used: %s -- "
+                          "`python -m inferspore_amd.build` builds it" % (CALLS_PATH, why), RuntimeWarning, stacklevel=3)
+            module = _NoCalls()
         _calls = module
     return _calls
 

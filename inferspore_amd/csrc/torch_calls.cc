@@ -361,4 +361,12 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_torch_calls", nullptr, -1, method
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__torch_calls() { return PyModule_Create(&module); }
+// `built_for`: the torch and the Python whose headers this was compiled with; the loader takes no other.
+PyMODINIT_FUNC PyInit__torch_calls() {
+    PyObject* m = PyModule_Create(&module);
+    if (m && PyModule_AddObject(m, "built_for", Py_BuildValue("(sii)", ISP_TORCH_VERSION, PY_MAJOR_VERSION, PY_MINOR_VERSION)) != 0) {
+        Py_DECREF(m);
+        return nullptr;
+    }
+    return m;
+}

@@ -12,6 +12,7 @@
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPStream.h>
 
+#include <algorithm>
 #include <initializer_list>
 
 #include "inferspore_amd.h"
@@ -20,14 +21,24 @@ namespace {
 
 using at::Tensor;
 
-// An operand as a call sees it: `t` is null for None.
+// An operand as a call sees it: `t` is null for None.  Extents and memory are what the checks have seen: once the interpreter's lock is
+// given up, another thread may change the tensor.
 struct Operand {
     const Tensor* t = nullptr;
-    int64_t size(int d) const { return t->size(d); }
-    int64_t dim() const { return t->dim(); }
-    int64_t numel() const { return t->numel(); }
-    void* data() const { return t ? t->mutable_data_ptr() : nullptr; }
-    bool is(std::initializer_list<int64_t> shape) const { return t->sizes() == at::IntArrayRef(shape.begin(), shape.size()); }
+    void* memory = nullptr;
+    int64_t dims = 0, count = 0, extent[5] = {};
+    Operand() = default;
+    explicit Operand(const Tensor& of) : t(&of), memory(of.mutable_data_ptr()), dims(of.dim()), count(of.numel()) {
+        for (int d = 0; d < 5 && d < dims; d++) extent[d] = of.size(d);
+    }
+    int64_t size(int d) const { return extent[d]; }
+    int64_t dim() const { return dims; }
+    int64_t numel() const { return count; }
+    void* data() const { return memory; }
+    bool is(std::initializer_list<int64_t> shape) const {
+        return dims == (int64_t)shape.size() && std::equal(shape.begin(), shape.end(), extent);
+    }
+    bool same_shape(const Operand& o) const { return dims <= 5 && dims == o.dims && std::equal(extent, extent + dims, o.extent); }
 };
 
 // A call that meets something else than plain operands notes it here and ends with None.
@@ -56,8 +67,7 @@ struct Call {
         const Tensor& t = THPVariable_Unpack(args[i]);
         plain = t.is_cuda() && t.scalar_type() == type && (t.key_set().raw_repr() & ~ordinary.raw_repr()) == 0 && t.has_storage() && t.is_contiguous();
         for (int64_t d = 0; plain && d < t.dim(); d++) plain = t.size(d) <= INT32_MAX;
-        o.t = &t;
-        return o;
+        return plain ? Operand(t) : o;
     }
     at::ScalarType float_type(Py_ssize_t i) {  // float16 or float32
         if (!plain) return at::kHalf;
@@ -156,7 +166,7 @@ ISP_METHOD(fused_add_bias_residual_rmsnorm) {  // residual, decoder_out, bias, g
     const Operand residual = c.tensor(0, type, true), x = c.tensor(1, type), bias = c.tensor(2, type, true), gamma = c.tensor(3, type);
     const float eps = c.number(4);
     const int flags = c.integer(5);
-    c.need(c.plain && x.dim() == 2 && (!residual.t || (residual.t->sizes() == x.t->sizes() && residual.data() != x.data())) &&
+    c.need(c.plain && x.dim() == 2 && (!residual.t || (residual.same_shape(x) && residual.data() != x.data())) &&
            gamma.numel() == x.size(1) && (!bias.t || bias.numel() == x.size(1)));
     return launched(c, [&] {
         return ISP_BY_TYPE(type, isp_fused_add_bias_residual_rmsnorm)(residual.data(), x.data(), bias.data(), gamma.data(), eps,
@@ -174,7 +184,7 @@ ISP_METHOD(act) {  // input, out
 
 // caches [layers, batch, kv_heads, max_seq_len, head_size] and a layer among theirs
 bool caches_fit(const Operand& k, const Operand& v, int layer, int64_t batch, int64_t kv_heads, int64_t head_size) {
-    return k.dim() == 5 && k.t->sizes() == v.t->sizes() && k.size(1) == batch && k.size(2) == kv_heads && k.size(4) == head_size &&
+    return k.dim() == 5 && k.same_shape(v) && k.size(1) == batch && k.size(2) == kv_heads && k.size(4) == head_size &&
            layer >= 0 && layer < k.size(0);
 }
 
@@ -262,7 +272,7 @@ ISP_METHOD(concat_kv_cache) {  // k_src, v_src, layer, query_length, history, k_
     const Operand k = c.tensor(0, type), v = c.tensor(1, type), lengths = c.tensor(3, at::kInt), history = c.tensor(4, at::kInt),
                   k_cache = c.tensor(5, type), v_cache = c.tensor(6, type);
     const int layer = c.integer(2);
-    c.need(c.plain && k.dim() == 4 && k.t->sizes() == v.t->sizes() &&
+    c.need(c.plain && k.dim() == 4 && k.same_shape(v) &&
            caches_fit(k_cache, v_cache, layer, k.size(0), k.size(1), k.size(3)) && lengths.numel() >= k.size(0) &&
            history.numel() >= k.size(0));
     return launched(c, [&] {
@@ -279,7 +289,7 @@ ISP_METHOD(repeat_kv_cache) {  // k_cache, v_cache, context_length, layer, k_dst
     const Operand k_cache = c.tensor(0, type), v_cache = c.tensor(1, type), context = c.tensor(2, at::kInt), k = c.tensor(4, type),
                   v = c.tensor(5, type);
     const int layer = c.integer(3);
-    c.need(c.plain && k_cache.dim() == 5 && k.dim() == 4 && k.t->sizes() == v.t->sizes() && context.dim() >= 1 &&
+    c.need(c.plain && k_cache.dim() == 5 && k.dim() == 4 && k.same_shape(v) && context.dim() >= 1 &&
            caches_fit(k_cache, v_cache, layer, context.size(0), k_cache.size(2), k.size(3)) && k.size(0) == context.size(0) &&
            k_cache.size(2) > 0 && k.size(1) % k_cache.size(2) == 0);
     return launched(c, [&] {
@@ -325,8 +335,8 @@ ISP_METHOD(context_layer) {
            !at::autocast::is_autocast_enabled(at::kCUDA));
     const bool grad = at::GradMode::is_enabled();
     for (int i = 0; c.plain && i < 18; i++) {
-        const Tensor* t = i < 14 ? f[i].t : lens[i - 14].t;
-        if (t) c.need(t->device() == f[0].t->device() && (i >= 14 || ((uintptr_t)t->mutable_data_ptr() % 16 == 0 && !(grad && t->requires_grad()))));
+        const Operand& o = i < 14 ? f[i] : lens[i - 14];
+        if (o.t) c.need(o.t->device() == f[0].t->device() && (i >= 14 || ((uintptr_t)o.data() % 16 == 0 && !(grad && o.t->requires_grad()))));
     }
     if (!c.plain || f[0].data() == f[1].data() || (type == at::kHalf && steps_are_faster(tokens, hidden, width, inter))) Py_RETURN_NONE;
     const char *q = static_cast<const char*>(f[9].data()), *packed = static_cast<const char*>(f[12].data());

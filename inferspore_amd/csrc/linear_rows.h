@@ -242,12 +242,14 @@ inline ProductPlan product_plan(int m, int n, int k, int max_splits = kTiledMaxS
     // The skinny kernel reads the weights straight to registers, 5.8 to 6.5 TB/s where its strips fill whole rounds of compute units; the tiled
     // one needs no whole rounds and feeds more rows.  us, skinny and tiled, additions included: 17 x 4096 x 28672 39.5, 43.1; 32 x 8192 x
     // 8192 27.6, 30.7; 17 x 8192 x 32768 87.0, 91.2; 48 x 4096 x 12288 26.4, 24.1; 32 x 4096 x 22016 43.3, 36.0; 64 x 4096 x 28672 49.5,
-    // 43.3.  The tiles' prices are 1.11 to 1.18 times what they take here.  SwiGLU inside saves a launch (3 us), but reads two narrower streams, slowest where
-    // rows are whole multiples of 2 KiB: 17 x 4096 x 28672 49.7 against 39.8 and 5.0; a whole layer of 48 rows x 4096, inter 11008, 125 against 131.  With these
-    // factors 102 layers of 512 to 8192 columns are within 1 % of the better of the two in the mean.
-    double tiled = 0.9 * us, skinny = skinny_us(p.skinny, m, n, k);
+    // 43.3.  The tiles' prices are 1.11 to 1.18 times what they take here, and what the skinny kernel
+    // saves with the third and fourth tile of rows is less sure, hence the factors.  SwiGLU inside a tiled product saves a launch (3 us), but
+    // reads two narrower streams, slowest where rows are whole multiples of 2 KiB: 17 x 4096 x 28672 49.7 against 39.8 and 5.0; a whole
+    // layer of 48 rows x 4096, inter 11008, 125 against 131.  261 layers of 512 to 8192 columns take 0.2 % more than with the better of both
+    // for each; at worst 2.3 % more than all skinny (which are up to 24 % slower) and 1.7 % more than all tiled (up to 14 %).
+    double tiled = (m <= 32 ? 0.9 : m <= 48 ? 0.86 : 0.76) * us, skinny = skinny_us(p.skinny, m, n, k);
     if (swiglu && p.tile.splits == 1) {
-        tiled *= 2ll * n % 2048 == 0 ? 1.33 : 1.11;
+        tiled *= 2ll * n % 2048 == 0 ? 1.28 : 1.05;
         skinny += 3.0;
     }
     p.tiled = tiled < skinny;

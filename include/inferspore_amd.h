@@ -312,6 +312,8 @@ int isp_linear_rows_f16(const void* a, const void* w, void* out, void* workspace
 /* The tile of a workgroup (0 x 0: the kernel for few rows, whose workgroups take all of them and 128 columns) and the number of workgroups that
  * share its k. */
 int isp_linear_rows_f16_plan(int m, int n, int k, int* tile_rows, int* tile_cols, int* splits);
+/* The same for the gate / up product [m, k] x [k, 2 inter] of a layer in one call: a tile without splits computes SwiGLU as well. */
+int isp_gate_up_rows_f16_plan(int m, int inter, int k, int* tile_rows, int* tile_cols, int* splits);
 /* The same in fp32 throughout: n and k multiples of 4 up to 2^22, up to 2^29 - 1 rows. */
 size_t isp_linear_rows_f32_workspace(int m, int n, int k);
 int isp_linear_rows_f32(const void* a, const void* w, void* out, void* workspace, int m, int n, int k, isp_stream_t stream);

@@ -61,6 +61,7 @@ SIGNATURES = {
     "isp_linear_rows_f16_workspace": (C.c_size_t, [_i, _i, _i]),
     "isp_linear_rows_f16": (_i, [_vp] * 4 + [_i] * 3 + [_vp]),
     "isp_linear_rows_f16_plan": (_i, [_i] * 3 + [C.POINTER(C.c_int)] * 3),
+    "isp_gate_up_rows_f16_plan": (_i, [_i] * 3 + [C.POINTER(C.c_int)] * 3),
     "isp_linear_rows_f32_workspace": (C.c_size_t, [_i, _i, _i]),
     "isp_linear_rows_f32": (_i, [_vp] * 4 + [_i] * 3 + [_vp]),
     "isp_linear_rows_f32_plan": (_i, [_i] * 3 + [C.POINTER(C.c_int)] * 3),

@@ -68,6 +68,16 @@ static int linear(const __half* a, const __half* w, __half* out, float* workspac
     return note_launch(hipGetLastError());
 }
 
+static int tell_plan(const ProductPlan& plan, int* tile_rows, int* tile_cols, int* splits) {
+    ISP_REQUIRE_PTR(tile_rows);
+    ISP_REQUIRE_PTR(tile_cols);
+    ISP_REQUIRE_PTR(splits);
+    *tile_rows = *tile_cols = 0;
+    if (plan.tiled) tiled_extents(plan.tile, tile_rows, tile_cols);
+    *splits = plan.splits();
+    return ISP_OK;
+}
+
 }  // namespace isp
 
 extern "C" {
@@ -85,11 +95,13 @@ int isp_linear_rows_f16(const void* a, const void* w, void* out, void* workspace
 
 int isp_linear_rows_f16_plan(int m, int n, int k, int* tile_rows, int* tile_cols, int* splits) {
     if (m <= 0 || n <= 0 || k <= 0 || !isp::linear_shape(m, n, k)) return ISP_ERR_BAD_SHAPE;
-    const isp::ProductPlan plan = isp::product_plan(m, n, k);
-    *tile_rows = *tile_cols = 0;
-    if (plan.tiled) isp::tiled_extents(plan.tile, tile_rows, tile_cols);
-    *splits = plan.splits();
-    return ISP_OK;
+    return isp::tell_plan(isp::product_plan(m, n, k), tile_rows, tile_cols, splits);
+}
+
+int isp_gate_up_rows_f16_plan(int m, int inter, int k, int* tile_rows, int* tile_cols, int* splits) {
+    if (m <= 0 || inter <= 0 || k <= 0 || inter > isp::kTiledMaxExtent / 2 || inter % 8 != 0 || !isp::linear_shape(m, 2 * inter, k))
+        return ISP_ERR_BAD_SHAPE;
+    return isp::tell_plan(isp::product_plan(m, 2 * inter, k, isp::kTiledMaxSplits, true), tile_rows, tile_cols, splits);
 }
 
 size_t isp_linear_f16_workspace(int m, int n, int k) {

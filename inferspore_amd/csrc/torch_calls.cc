@@ -300,13 +300,16 @@ ISP_METHOD(repeat_kv_cache) {  // k_cache, v_cache, context_length, layer, k_dst
 }
 
 // float16 layers that are faster step by step, with the library's product for what is wide: 17 to 64 rows where a product has more than 32768
-// columns, 65 to 192 rows where gate and up projections have more than 400 million weights.  us a layer, steps and one call: 48 rows x
-// 6144, inter 24576 278, 295; 40 x 10240, 27648, 8 key heads 411, 464; 96 x 8192, 28672 495, 554; 144 x 12288, 43008 1142, 1421.  Next to the
-// lines: 17 x 6144, 24576 262, 236; 40 x 5120, 13824 162, 159; 80 x 8192, 28672 544, 537; 128 x 8192, 22016 531, 491; 200 x 12288, 43008
-// 1480, 1308; 640 x 8192, 28672, the slowest above 192 rows, 1349, 1437.
+// columns; 65 to 128 rows of more than 8192 columns where gate and up projections have 400 to 650 million weights, 129 to 192 rows of more
+// than 9216 where they have more than 400 million.  us a layer, steps and one call: 48 rows x 6144, inter 24576 278, 295; 40 x 10240, 27648,
+// 8 key heads 411, 464; 96 x 9216, 24704 541, 625; 144 x 12288, 43008 1142, 1421.  Next to the lines: 17 x 6144, 24576 262, 236; 40 x 5120,
+// 13824 162, 159; 112 x 8192, 28672 580, 576; 80 x 10240, 35840 925, 807; 144 x 9216, 32256 729, 685; 200 x 12288, 43008 1480, 1308.  The library's times jump from one number of rows
+// to the next: 96 x 8192, 28672 takes 495 there and 554 here, 640 rows 1349 and 1437, the worst found on this side of the lines.
 bool steps_are_faster(int rows, int64_t hidden, int64_t width, int64_t inter) {
     if (rows <= 64) return rows > 16 && (2 * inter > 32768 || width > 32768);
-    return rows <= 192 && 2 * inter * hidden > 400000000;
+    const int64_t weights = 2 * inter * hidden;
+    if (rows <= 128) return hidden > 8192 && weights > 400000000 && weights <= 650000000;
+    return rows <= 192 && hidden > 9216 && weights > 400000000;
 }
 
 // A whole layer: its output, a status that is not 0, or None.  normed, residual, qkv, qkv_bias, o, gate_up, down, ffn_norm, next_norm, q,

@@ -84,8 +84,9 @@ def test_a_few_tokens_among_thousands_of_empty_sequences(isp):
 
 @pytest.mark.parametrize("rows,hidden,inter,kv,one", [(16, 64, 16392, 1, True), (17, 64, 16392, 1, False), (64, 64, 16384, 1, True),
                                                       (33, 64, 64, 171, False), (64, 64, 64, 170, True), (65, 64, 16392, 1, True),
-                                                      (65, 8192, 24416, 1, False), (192, 8192, 24416, 1, False),
-                                                      (193, 8192, 24416, 1, True), (192, 8192, 24408, 1, True)])
+                                                      (128, 8200, 24416, 1, False), (129, 8200, 24416, 1, True),
+                                                      (65, 8192, 24416, 1, True), (65, 8200, 24376, 1, True), (128, 8200, 39640, 1, True),
+                                                      (192, 9224, 21688, 1, False), (193, 9224, 21688, 1, True)])
 def test_layers_that_are_faster_step_by_step(isp, rows, hidden, inter, kv, one):
     """Few rows with wide products keep the library's product for them."""
     from inferspore_amd import context_layer as cl

@@ -4,7 +4,8 @@
 // TB/s.  us before and after, addition of splits included: 308 rows x 2048 -> 6144 79, 63; x 2048 -> 2048 33, 28; x 2048 -> 11264 174,
 // 119; x 5632 -> 2048 74, 60; 16 x 4096 -> 12288 46, 37; 64 x 11008 -> 4096 105, 53.  Over 250 products of models of 512 ... 5120
 // columns, 1 ... 3000 rows: 1.43 times as fast in the geometric mean, 0.89 times at worst (668 x 9792 -> 2560, whose tiles fill the chip
-// badly).  The matrix cores' fp32 rate bounds all but few rows: 116 to 147 of 157 TFLOP/s.
+// badly).  Whole layers of 3000 to 16000 rows x 4096 to 6144 take 0.90 to 1.025 times what they do with the library's products, longest where
+// rows are a multiple of 2048 (8192 x 4096, inter 11008: 24.1 ms, 23.5 with the library's; 8000 rows 23.7, 23.7).  The matrix cores' fp32 rate bounds all but few rows: 116 to 147 of 157 TFLOP/s.
 #include "linear_tiled_f32.h"
 
 #include <math.h>
@@ -145,6 +146,9 @@ int isp_linear_rows_f32(const void* a, const void* w, void* out, void* workspace
 
 int isp_linear_rows_f32_plan(int m, int n, int k, int* tile_rows, int* tile_cols, int* splits) {
     if (m <= 0 || n <= 0 || k <= 0 || !isp::linear_shape_f32(m, n, k)) return ISP_ERR_BAD_SHAPE;
+    ISP_REQUIRE_PTR(tile_rows);
+    ISP_REQUIRE_PTR(tile_cols);
+    ISP_REQUIRE_PTR(splits);
     const isp::TiledPlan plan = isp::tiled_plan_f32(m, n, k, isp::kTiledMaxSplits, nullptr);
     *tile_rows = isp::kTilesF32[plan.tile].rows;
     *tile_cols = isp::kTilesF32[plan.tile].cols;

@@ -221,3 +221,11 @@ def test_products_refuse_more_rows_than_a_grid_holds(lib, kind, most):
     for m in (most + 1, 2 ** 31 - 40):
         assert plan(m, 8, 8, ctypes.byref(a), ctypes.byref(b), ctypes.byref(s)) != 0
         assert space(m, 8, 8) == 0 and call(p, p, p, p, m, 8, 8, None) == capi.ERR_UNSUPPORTED
+
+
+@pytest.mark.parametrize("name", ["isp_linear_rows_f16_plan", "isp_linear_rows_f32_plan", "isp_gate_up_rows_f16_plan"])
+def test_plans_refuse_null_results(lib, name):
+    from inferspore_amd import capi
+    a = ctypes.byref(ctypes.c_int())
+    for results in ((None, a, a), (a, None, a), (a, a, None)):
+        assert getattr(lib, name)(100, 64, 64, *results) == capi.ERR_NULL_POINTER

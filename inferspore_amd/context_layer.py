@@ -19,8 +19,9 @@ order a model runs them:
     residual, normed_next = fused_add_bias_residual_rmsnorm(residual, ffn_out, next attn_norm)   * this library
 
 A layer of float16 or float32 rows is one call of the C ABI (isp_context_layer_rows_f16, _f32), products included.  Where a layer runs
-step by step (a mask of its own, unaligned buffers, gradients), products of up to 64 float16 rows go to ops.linear and the others to
-torch's library calls (hipBLASLt GEMMs); everything marked * goes through the C ABI.  All work is issued on torch's current stream.
+step by step (a mask of its own, unaligned buffers, gradients, a dispatch mode, few rows with the widest products), products of up to 64
+float16 rows go to ops.linear and the others to torch's library calls (hipBLASLt GEMMs); everything marked * goes through the C ABI.  All
+work is issued on torch's current stream.
 """
 import math
 
@@ -48,14 +49,17 @@ class LayerWeights:
 
 
 def _padded_is_faster(dtype, batch, max_q_len, max_k_len, head_num, kv_head_num, head_size):
-    """Thousands of contexts of a few keys.  A workgroup of the fused kernels costs 5 to 10 ns of the chip even then, one per key
-    head (up to 16 queries per group) or per query head; torch's kernel works in tiles of 16 keys and takes 2.5 to 9 ns per head.
+    """Thousands of contexts of a few keys.  The attention alone: a workgroup of the fused kernels costs 5 to 10 ns of the chip even then,
+    one per key head (up to 16 queries per group) or per query head; torch's kernel works in tiles of 16 keys and takes 2.5 to 9 ns per head.
     float16, 128 elements, us fused and padded: 1000 prompts of 7 / 12 / 16 tokens, 32 heads over 8 313 and 172 / 331 and 240 / 340
     and 296, of 24 363 and 673; 4000 decode rows of 8 keys, 8 heads 193 and 123, 8 over 2 below it.  Beyond ten thousand
     sequences the lengths that every workgroup adds up count as well: 16000 decode rows of 8 keys, 8 heads 959 and 470; in float32
     60000 of 1 / 8 / 12 keys 5359 and 3141 / 5585 and 4017 / level.  Heads of 96 in float16 lie in between (4000 rows of 2 keys
     132 and 117, 16000 of 12 876 and 808).  Fewer workgroups are over before torch's launches are: 1000 rows of 4 keys, 8 heads of
-    64, 30 and 41."""
+    64, 30 and 41.
+    Whole layers, which in the padded form have the library's products as well: decode rows keep that gain (4000 rows of 8 keys, 1024
+    wide, 342 in one call and 284 padded; 16000 x 4096 9470 and 7680; 30000 in float32 7810 and 7650); prompts do not (1000 of 7 / 12 / 16
+    tokens, 4096 wide, 2342 and 2644 / 3703 and 4426 / 4835 and 5197): for them the line is still the attention's."""
     if max_k_len > 16 or batch * head_num * head_size < 1000000:
         return False
     tiled = head_num // max(kv_head_num, 1) * max_q_len > 16

@@ -1,11 +1,11 @@
 // isp_context_layer_rows_f16: a whole context-decoder layer of packed fp16 rows in one call (isp_context_layer_f16: up to 64 of them);
 // isp_context_layer_rows_f32: of fp32 rows.
-// Seven to ten launches.  A product whose k is split over workgroups leaves fp32 partial sums, and the step that follows adds them where it
+// Seven to ten launches (two more where rows are wider than 8192 columns).  A product whose k is split over workgroups leaves fp32 partial sums, and the step that follows adds them where it
 // would have read the product -- QKV bias + RoPE + KV append, residual + RMSNorm (twice), SwiGLU; a gate / up product that is not
 // split computes SwiGLU itself.  As separate calls a layer
-// takes 14 launches (four products, their four additions, six steps) and, from Python, about 13 us of host time each, more than a
-// small layer's kernels take: 16 sequences at 256-1023 keys 271 against 262 us for two layers, one prompt of 37 tokens 256
-// against 246.
+// takes up to 14 launches (four products, their four additions, six steps) and host time in Python for each.  us per two layers, step by
+// step and in one call: 16 sequences at 256-1023 keys, 4096 wide, 268, 260; one prompt of 37 tokens 240, 230; 664 tokens, 1024 wide (the
+// steps' products by the library), 223, 130.
 // The steps and their order are those of the reference's kernel comments (see inferspore_amd/context_layer.py).
 #include <math.h>
 

@@ -8,13 +8,17 @@ namespace isp {
 
 // A tile and what it measured: a workgroup takes start_us + step_us per 64 k with a compute unit to itself, pair_us per 64 k where two
 // share one (tiles of up to 80 KiB of LDS); the weights arrive at stream_tb TB/s at most.  Fitted (mean error 7 to 9 %) to 1970
-// products of 17 ... 8192 rows over the layers of models of 512 ... 5120 columns, each with every tile and up to sixteen splits.  The plan
-// that these figures choose is 2 % behind the best of all (geometric mean; 10 % in one of twenty).
+// products of 17 ... 8192 rows over the layers of models of 512 ... 5120 columns, each with every tile and up to sixteen splits; then two
+// prices were corrected by measurement.
 // swiglu: steps of a product with SwiGLU inside take so much longer.  The wavefronts of 128 x 192 own 96 columns, in which gates and up
 // projections alternate 32 bytes at a time, not 64: 1.34 to 1.69 us per step and pair, not 1.22.  Without the factor 660 x 4096 x 22016 took
 // 173 us there (128 x 256: 152), 463 rows 104 (256 x 256: 100), 300 rows 93 (192 x 256: 86).  The 192 x 256 tile's step is not the
 // fit's 1.166: at 200 to 256 workgroups, for which it is mostly taken, it measures 1.21 to 1.26 (2611 x 4096 x 4096 87.1 us, 128 x 192 82.8;
 // x 11008 x 4096 219.6 and 213.1).
+// With these figures the plan is 3 % behind the best tile and splits for each of 398 other products of 65 to 8192 rows (geometric mean; 17 %
+// in one of twenty).  Worst are 90 to 140 rows and more than 22000 columns: 112 x 5120 x 26176 takes 64 x 128, 74 us, where 128 x 128
+// takes 55.  Against the library, of 166 products that take it more than 30 us: 1.29 times as fast in the geometric mean, 0.79 times at
+// worst (the same product), slower for 16 of them.
 struct TiledTile {
     int rows, cols, threads, per_unit;
     float start_us, step_us, pair_us, stream_tb, partial_tb, swiglu;
